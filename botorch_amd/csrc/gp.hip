@@ -1,10 +1,7 @@
-// SingleTaskGP prediction caches, posterior, and the qLogNEI baseline cache.
+// SingleTaskGP prediction caches and the qLogNEI baseline cache.
 //
 // Cache build (once per model, fast_pred_var form):
 //   K = k(X,X) + noise I  ->  L = chol(K)  ->  L^-1  ->  alpha = L^-T L^-1 (y - c)
-// Posterior over batch x mq points (original outcome scale):
-//   V = k(X*, X) L^-T;  mean = y_mean + y_std (c + k(X*,X) alpha)
-//   covar = y_std^2 (k(X*,X*) - V V^T)
 // qLogNEI baseline cache (acquisition/logei.py:393-459):
 //   A^T = V_b L^-1 (= (K^-1 k(X, X_b))^T), Lb = chol(Sigma_bb), best_f from the
 //   baseline samples, and the extended operator [L^-1; alpha^T; A^T] used by
@@ -17,38 +14,6 @@
 #include <cmath>
 
 namespace bta {
-
-// rows [i*mq_pad + r] of Xs = scaled X[i*mq + r] (zero rows in the padding)
-__global__ void scale_batched_kernel(const double* X, int64_t batch, int mq, int mq_pad, int d,
-                                     const double* center, const double* ls, double* Xs) {
-  const int64_t idx = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  const int64_t tot = batch * mq_pad * d;
-  if (idx >= tot) return;
-  const int j = (int)(idx % d);
-  const int64_t row = idx / d;
-  const int64_t bi = row / mq_pad;
-  const int r = (int)(row % mq_pad);
-  Xs[idx] = r < mq ? (X[(bi * mq + r) * d + j] - center[j]) / ls[j] : 0.0;
-}
-
-// mean[i*mq+r] = y_mean + y_std (c + KA[(i*mq_pad + r)*lda]);
-// covar/var from the padded batch blocks of Sg (already in the outcome scale)
-__global__ void posterior_out_kernel(const double* KA, int64_t lda, const double* Sg,
-                                     int64_t batch, int mq, int mq_pad, double y_mean,
-                                     double y_std, double c, double* mean, double* covar,
-                                     double* var) {
-  const int64_t bi = blockIdx.y;
-  const double* Sb = Sg + bi * mq_pad * mq_pad;
-  for (int e = blockIdx.x * blockDim.x + threadIdx.x; e < mq * mq; e += gridDim.x * blockDim.x) {
-    const int i = e / mq, j = e % mq;
-    const double v = Sb[i * mq_pad + j];
-    if (covar) covar[(bi * mq + i) * mq + j] = v;
-    if (i == j) {
-      if (var) var[bi * mq + i] = v;
-      if (mean) mean[bi * mq + i] = y_mean + y_std * (c + KA[(bi * mq_pad + i) * lda]);
-    }
-  }
-}
 
 // out[blockIdx.x] = max |x[i]| over the block's grid-stride share
 constexpr int MAXABS_BLOCKS = 256;
@@ -252,233 +217,6 @@ int gp_cache_build(const bta_gp_model* m, const double* y, double* L, double* Li
   return BTA_OK;
 }
 
-struct PostWs {
-  int mq_pad;
-  int64_t R_pad;
-  size_t xs, kx, vt, ka, kbb, sg, arow, total;
-  PostWs(const bta_gp_model* m, int64_t batch, int mq) {
-    mq_pad = (int)round_up(mq, 64);
-    R_pad = batch * mq_pad;
-    WsPlan p;
-    xs = p.take((size_t)R_pad * m->d * 8);
-    kx = p.take((size_t)R_pad * m->n_pad * 8);
-    vt = p.take((size_t)R_pad * m->n_pad * 8);
-    ka = p.take((size_t)R_pad * 64 * 8);
-    kbb = p.take((size_t)batch * mq_pad * mq_pad * 8);
-    sg = p.take((size_t)batch * mq_pad * mq_pad * 8);
-    arow = p.take((size_t)64 * m->n_pad * 8);
-    total = p.off;
-  }
-};
-
-int gp_posterior(const bta_gp_model* m, const double* X, int64_t batch, int mq, double* mean,
-                 double* covar_out, double* var, void* ws, size_t ws_bytes, hipStream_t s) {
-  if (!m || !X || batch < 1 || mq < 1 || !m->linv || !m->alpha || batch > 65535) {
-    set_error("gp_posterior: invalid arguments");
-    return BTA_ERR_INVALID;
-  }
-  const PostWs w(m, batch, mq);
-  if (!ws || ws_bytes < w.total) {
-    set_error("gp_posterior: workspace too small");
-    return BTA_ERR_WORKSPACE;
-  }
-  char* base = (char*)ws;
-  double* xs = (double*)(base + w.xs);
-  double* kx = (double*)(base + w.kx);
-  double* vt = (double*)(base + w.vt);
-  double* ka = (double*)(base + w.ka);
-  double* kbb = (double*)(base + w.kbb);
-  double* sg = (double*)(base + w.sg);
-  double* arow = (double*)(base + w.arow);
-  const int64_t np = m->n_pad;
-  const int64_t tot = w.R_pad * m->d;
-  hipLaunchKernelGGL(scale_batched_kernel, dim3((unsigned)((tot + 255) / 256)), dim3(256), 0, s,
-                     X, batch, mq, w.mq_pad, m->d, m->center, m->lengthscale, xs);
-  BTA_LAUNCH_CHECK("scale_batched_kernel");
-  int rc = covar(m->kind, xs, w.R_pad, m->train_xs, m->n, m->d, m->outputscale, 0.0, false, kx,
-                 np, w.R_pad, np, s);
-  if (rc) return rc;
-  rc = gemm(BTA_GEMM_B_LOWER, w.R_pad, np, np, 1.0, kx, np, m->linv, np, 0.0, nullptr, 0, vt, np,
-            s);
-  if (rc) return rc;
-  rc = cast_pad<double>(m->alpha, np, 1, np, arow, np, 64, np, s);
-  if (rc) return rc;
-  rc = gemm(0, w.R_pad, 64, np, 1.0, kx, np, arow, np, 0.0, nullptr, 0, ka, 64, s);
-  if (rc) return rc;
-  const int64_t mp = w.mq_pad;
-  rc = covar(m->kind, xs, mp, xs, mp, m->d, m->outputscale, 0.0, false, kbb, mp, mp, mp, s, 0,
-             (int)batch, mp * m->d, mp * m->d, mp * mp);
-  if (rc) return rc;
-  const double v2 = m->y_std * m->y_std;
-  rc = gemm(0, mp, mp, np, -v2, vt, np, vt, np, v2, kbb, mp, sg, mp, s, (int)batch, mp * np,
-            mp * np, mp * mp, mp * mp);
-  if (rc) return rc;
-  dim3 g((unsigned)std::min<int64_t>(64, ((int64_t)mq * mq + 255) / 256), (unsigned)batch);
-  hipLaunchKernelGGL(posterior_out_kernel, g, dim3(256), 0, s, ka, (int64_t)64, sg, batch, mq,
-                     w.mq_pad, m->y_mean, m->y_std, m->mean_constant, mean, covar_out, var);
-  BTA_LAUNCH_CHECK("posterior_out_kernel");
-  return BTA_OK;
-}
-
-// ---------------------------------------------------------------------------
-// Adjoint of the posterior: dX from d mean and d covar.
-//   dK_x   = y_std dmean alpha^T - y_std^2 (dC + dC^T) U,   U = V L^-1 = K_x K^-1
-//   dK_xx  = y_std^2 dC  (the prior covariance among the batch's own points)
-//   dX     = through dk/dX of both, divided by the lengthscale
-// ---------------------------------------------------------------------------
-// S_b = y_std^2 (dC_b + dC_b^T), zero-padded to mq_pad x mq_pad; dm_pad = y_std
-// dmean in the padded row layout (0 where dmean is NULL).
-__global__ void post_bwd_prep_kernel(const double* dmean, const double* dcov, int64_t batch, int mq,
-                                     int mq_pad, double y_std, double* S, double* dm_pad) {
-  const int64_t bi = blockIdx.y;
-  for (int e = blockIdx.x * blockDim.x + threadIdx.x; e < mq_pad * mq_pad;
-       e += gridDim.x * blockDim.x) {
-    const int i = e / mq_pad, j = e % mq_pad;
-    double v = 0.0;
-    if (dcov && i < mq && j < mq)
-      v = y_std * y_std *
-          (dcov[(bi * mq + i) * mq + j] + dcov[(bi * mq + j) * mq + i]);
-    S[bi * mq_pad * mq_pad + e] = v;
-    if (j == 0) dm_pad[bi * mq_pad + i] = (dmean && i < mq) ? y_std * dmean[bi * mq + i] : 0.0;
-  }
-}
-
-// G[r][k] += dm_pad[r] alpha[k]  (the mean's part of dK_x)
-__global__ void add_outer_kernel(double* G, int64_t ldg, const double* dm_pad,
-                                 const double* alpha, int64_t n) {
-  const int64_t r = blockIdx.y;
-  const double a = dm_pad[r];
-  if (a == 0.0) return;
-  for (int64_t k = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; k < n;
-       k += (int64_t)gridDim.x * blockDim.x)
-    G[r * ldg + k] += a * alpha[k];
-}
-
-// extra[r][j] = sum_i2 S_b[i][i2] dk(xs_i, xs_i2)/dxs_i[j] = -sum_i2 S_b[i][i2] h (xs_i - xs_i2)_j
-// (scaled coordinates; the row's own term has no gradient)
-__global__ void post_direct_grad_kernel(int kind, const double* xs, int64_t batch, int mq,
-                                        int mq_pad, int d, double s, const double* S,
-                                        double* extra) {
-  const int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (e >= batch * mq_pad * d) return;
-  const int j = (int)(e % d);
-  const int64_t row = e / d;
-  const int64_t bi = row / mq_pad;
-  const int i = (int)(row % mq_pad);
-  double acc = 0.0;
-  if (i < mq) {
-    const double* xi = xs + row * d;
-    for (int i2 = 0; i2 < mq; ++i2) {
-      if (i2 == i) continue;
-      const double sv = S[(bi * mq_pad + i) * mq_pad + i2];
-      if (sv == 0.0) continue;
-      const double* x2 = xs + (bi * mq_pad + i2) * d;
-      double r2 = 0.0;
-      for (int t = 0; t < d; ++t) {
-        const double df = xi[t] - x2[t];
-        r2 = fma(df, df, r2);
-      }
-      acc -= sv * kern_grad_factor(kind, r2, s, nullptr) * (xi[j] - x2[j]);
-    }
-  }
-  extra[e] = acc;
-}
-
-// dX[(bi mq + r) d + j] = dXp[(bi mq_pad + r) d + j]
-__global__ void unpad_rows_kernel(const double* dXp, int64_t batch, int mq, int mq_pad, int d,
-                                  double* dX) {
-  const int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (e >= batch * mq * d) return;
-  const int j = (int)(e % d);
-  const int64_t row = e / d;
-  const int64_t bi = row / mq;
-  const int r = (int)(row % mq);
-  dX[e] = dXp[(bi * mq_pad + r) * d + j];
-}
-
-struct PostBwdWs {
-  int mq_pad;
-  int64_t R_pad;
-  size_t xs, kx, vt, S, dm, extra, dxp, total;
-  PostBwdWs(const bta_gp_model* m, int64_t batch, int mq) {
-    mq_pad = (int)round_up(mq, 64);
-    R_pad = batch * mq_pad;
-    WsPlan p;
-    xs = p.take((size_t)R_pad * m->d * 8);
-    kx = p.take((size_t)R_pad * m->n_pad * 8);
-    vt = p.take((size_t)R_pad * m->n_pad * 8);
-    S = p.take((size_t)batch * mq_pad * mq_pad * 8);
-    dm = p.take((size_t)R_pad * 8);
-    extra = p.take((size_t)R_pad * m->d * 8);
-    dxp = p.take((size_t)R_pad * m->d * 8);
-    total = p.off;
-  }
-};
-
-int gp_posterior_backward(const bta_gp_model* m, const double* X, int64_t batch, int mq,
-                          const double* dmean, const double* dcov, double* dX, void* ws,
-                          size_t ws_bytes, hipStream_t s) {
-  if (!m || !X || !dX || batch < 1 || mq < 1 || !m->linv || !m->alpha || batch > 65535 ||
-      (!dmean && !dcov)) {
-    set_error("gp_posterior_backward: invalid arguments");
-    return BTA_ERR_INVALID;
-  }
-  const PostBwdWs w(m, batch, mq);
-  if (!ws || ws_bytes < w.total) {
-    set_error("gp_posterior_backward: workspace too small");
-    return BTA_ERR_WORKSPACE;
-  }
-  char* base = (char*)ws;
-  double* xs = (double*)(base + w.xs);
-  double* kx = (double*)(base + w.kx);
-  double* vt = (double*)(base + w.vt);
-  double* S = (double*)(base + w.S);
-  double* dm = (double*)(base + w.dm);
-  double* extra = (double*)(base + w.extra);
-  double* dxp = (double*)(base + w.dxp);
-  const int64_t np = m->n_pad, mp = w.mq_pad;
-  const int64_t tot = w.R_pad * m->d;
-  hipLaunchKernelGGL(scale_batched_kernel, dim3((unsigned)((tot + 255) / 256)), dim3(256), 0, s,
-                     X, batch, mq, w.mq_pad, m->d, m->center, m->lengthscale, xs);
-  BTA_LAUNCH_CHECK("scale_batched_kernel");
-  int rc = covar(m->kind, xs, w.R_pad, m->train_xs, m->n, m->d, m->outputscale, 0.0, false, kx,
-                 np, w.R_pad, np, s);
-  if (rc) return rc;
-  // V = K_x L^-T into vt, then U = V L^-1 into kx
-  rc = gemm(BTA_GEMM_B_LOWER, w.R_pad, np, np, 1.0, kx, np, m->linv, np, 0.0, nullptr, 0, vt, np,
-            s);
-  if (rc) return rc;
-  rc = gemm(BTA_GEMM_B_KN | BTA_GEMM_B_UPPER, w.R_pad, np, np, 1.0, vt, np, m->linv, np, 0.0,
-            nullptr, 0, kx, np, s);
-  if (rc) return rc;
-  {
-    const dim3 g((unsigned)std::min<int64_t>(64, (mp * mp + 255) / 256), (unsigned)batch);
-    hipLaunchKernelGGL(post_bwd_prep_kernel, g, dim3(256), 0, s, dmean, dcov, batch, mq,
-                       w.mq_pad, m->y_std, S, dm);
-    BTA_LAUNCH_CHECK("post_bwd_prep_kernel");
-  }
-  // G = -S U per batch block (into vt), then + y_std dmean alpha^T
-  rc = gemm(BTA_GEMM_B_KN, mp, np, mp, -1.0, S, mp, kx, np, 0.0, nullptr, 0, vt, np, s,
-            (int)batch, mp * mp, mp * np, 0, mp * np);
-  if (rc) return rc;
-  if (dmean) {
-    const dim3 g((unsigned)std::min<int64_t>(64, (np + 255) / 256), (unsigned)w.R_pad);
-    hipLaunchKernelGGL(add_outer_kernel, g, dim3(256), 0, s, vt, np, dm, m->alpha, m->n);
-    BTA_LAUNCH_CHECK("add_outer_kernel");
-  }
-  hipLaunchKernelGGL(post_direct_grad_kernel, dim3((unsigned)((tot + 255) / 256)), dim3(256), 0,
-                     s, m->kind, xs, batch, mq, w.mq_pad, m->d, m->outputscale, S, extra);
-  BTA_LAUNCH_CHECK("post_direct_grad_kernel");
-  rc = covar_grad(m->kind, xs, w.R_pad, m->train_xs, m->n, m->d, m->outputscale, vt, false, np,
-                  extra, m->lengthscale, dxp, s);
-  if (rc) return rc;
-  const int64_t to = batch * mq * m->d;
-  hipLaunchKernelGGL(unpad_rows_kernel, dim3((unsigned)((to + 255) / 256)), dim3(256), 0, s, dxp,
-                     batch, mq, w.mq_pad, m->d, dX);
-  BTA_LAUNCH_CHECK("unpad_rows_kernel");
-  return BTA_OK;
-}
-
 struct PrepWs {
   int64_t nbp;
   size_t kb, vb, at, kbb, sg, lbp, arow, ka, mu, fact, mx, total;
@@ -626,33 +364,6 @@ extern "C" int bta_gp_cache_build(const bta_gp_model* m, const double* y, double
                                   bta_stream_t stream) {
   return bta::gp_cache_build(m, y, L, Linv, alpha, max_tries, jitter_used, ws, ws_bytes,
                              (hipStream_t)stream);
-}
-
-extern "C" size_t bta_gp_posterior_workspace_size(const bta_gp_model* m, int64_t batch,
-                                                  int32_t mq) {
-  if (!m || batch < 1 || mq < 1) return 0;
-  return bta::PostWs(m, batch, mq).total;
-}
-
-extern "C" int bta_gp_posterior(const bta_gp_model* m, const double* X, int64_t batch,
-                                int32_t mq, double* mean, double* covar, double* var, void* ws,
-                                size_t ws_bytes, bta_stream_t stream) {
-  return bta::gp_posterior(m, X, batch, mq, mean, covar, var, ws, ws_bytes,
-                           (hipStream_t)stream);
-}
-
-extern "C" size_t bta_gp_posterior_backward_workspace_size(const bta_gp_model* m,
-                                                          int64_t batch, int32_t mq) {
-  if (!m || batch < 1 || mq < 1) return 0;
-  return bta::PostBwdWs(m, batch, mq).total;
-}
-
-extern "C" int bta_gp_posterior_backward(const bta_gp_model* m, const double* X, int64_t batch,
-                                         int32_t mq, const double* dmean, const double* dcov,
-                                         double* dX, void* ws, size_t ws_bytes,
-                                         bta_stream_t stream) {
-  return bta::gp_posterior_backward(m, X, batch, mq, dmean, dcov, dX, ws, ws_bytes,
-                                    (hipStream_t)stream);
 }
 
 extern "C" size_t bta_qlognei_prepare_workspace_size(const bta_gp_model* m, int32_t n_b,
