@@ -18,6 +18,12 @@ struct GemmArgs {
 
 int launch_gemm(const GemmArgs& g, int batch, hipStream_t s);
 
+// C = A op(B) for the R_pad x np matrices A and C and the triangular np x np B
+// (flags), of whose rows only the first R are used: rows of C past R rounded up to
+// 32 may stay unwritten.
+int gemm_rows(int flags, int64_t R, int64_t R_pad, int64_t np, const void* A, const void* B,
+              void* C, hipStream_t s);
+
 // Convenience: C = alpha A op(B) + beta C0 (single batch).
 inline int gemm(int flags, int64_t M, int64_t N, int64_t K, double alpha, const void* A,
                 int64_t lda, const void* B, int64_t ldb, double beta, const void* C0,

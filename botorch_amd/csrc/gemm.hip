@@ -19,6 +19,7 @@
 #include "gemm.h"
 #include "gemm_d.h"
 #include "gemm_tile.h"
+#include "gemm_w.h"
 #include "kernels.h"
 
 #include <algorithm>
@@ -220,6 +221,25 @@ static int launch_cfg(const GemmArgs& g, int batch, int W, hipStream_t s) {
   return launch_cfg2<T, BM, BN, BK, false>(g, batch, W, s);
 }
 
+// One triangular FP64 product with R rows in use of R_pad (a multiple of 64): the
+// small tiles need R rounded up to 32 only.
+int gemm_rows(int flags, int64_t R, int64_t R_pad, int64_t np, const void* A, const void* B,
+              void* C, hipStream_t s) {
+  GemmArgs g{};
+  g.A = A;
+  g.B = B;
+  g.C = C;
+  g.lda = g.ldb = g.ldc = np;
+  g.M = (int)round_up(R, 32);
+  g.N = g.K = (int)np;
+  g.flags = flags;
+  g.alpha = 1.0;
+  if (!(flags & BTA_GEMM_F32) && gemm_w_supported(g) && gemm_w_preferred(g.M, np, 1))
+    return gemm_w(g, 1, s);
+  g.M = (int)R_pad;
+  return launch_gemm(g, 1, s);
+}
+
 int launch_gemm(const GemmArgs& g, int batch, hipStream_t s) {
   if (g.M % 64 || g.N % 64 || g.K % 64 || g.M <= 0 || g.N <= 0 || g.K < 0) {
     set_error("bta_gemm: M, N, K must be positive multiples of 64 (got %d %d %d)", g.M, g.N,
@@ -282,5 +302,11 @@ extern "C" int bta_gemm(int32_t flags, int64_t M, int64_t N, int64_t K, double a
     bta::set_error("bta_gemm: unknown flag bits 0x%x", flags & ~known);
     return BTA_ERR_INVALID;
   }
+  // The small tiles are taken here and by gemm_rows, not inside launch_gemm: the
+  // baseline preparation's products keep the order of their sums, since a changed
+  // last bit there moves every later iterate of an optimisation that starts from it.
+  if (batch > 0 && !(flags & BTA_GEMM_F32) && M % 64 == 0 && N % 64 == 0 && K % 64 == 0 &&
+      bta::gemm_w_supported(g) && bta::gemm_w_preferred(M, N, (int)batch))
+    return bta::gemm_w(g, (int)batch, (hipStream_t)stream);
   return bta::launch_gemm(g, (int)batch, (hipStream_t)stream);
 }

@@ -312,6 +312,8 @@ struct PostLayout {
       R_pad = batch * mq_pad;
     }
   }
+  // rows the products have to form
+  int64_t used(int64_t batch, int mq) const { return mq_pad == mq ? batch * mq : R_pad; }
 };
 
 struct PostWs {
@@ -380,8 +382,7 @@ int gp_posterior(const bta_gp_model* m, const double* X, int64_t batch, int mq, 
   const int64_t np = m->n_pad;
   rc = post_rows(m, X, batch, mq, w.lay, xs, kx, part, s);
   if (rc) return rc;
-  rc = gemm(BTA_GEMM_B_LOWER, w.lay.R_pad, np, np, 1.0, kx, np, m->linv, np, 0.0, nullptr, 0, vt,
-            np, s);
+  rc = gemm_rows(BTA_GEMM_B_LOWER, w.lay.used(batch, mq), w.lay.R_pad, np, kx, m->linv, vt, s);
   if (rc) return rc;
   PostOutArgs o;
   o.V = vt;
@@ -666,11 +667,10 @@ int gp_posterior_backward(const bta_gp_model* m, const double* X, int64_t batch,
   a.U = nullptr;
   if (dcov) {
     // V = K_x L^-T into vt, then U = V L^-1 into kx
-    rc = gemm(BTA_GEMM_B_LOWER, R_pad, np, np, 1.0, kx, np, m->linv, np, 0.0, nullptr, 0, vt, np,
-              s);
+    const int64_t R = w.lay.used(batch, mq);
+    rc = gemm_rows(BTA_GEMM_B_LOWER, R, R_pad, np, kx, m->linv, vt, s);
     if (rc) return rc;
-    rc = gemm(BTA_GEMM_B_KN | BTA_GEMM_B_UPPER, R_pad, np, np, 1.0, vt, np, m->linv, np, 0.0,
-              nullptr, 0, kx, np, s);
+    rc = gemm_rows(BTA_GEMM_B_KN | BTA_GEMM_B_UPPER, R, R_pad, np, vt, m->linv, kx, s);
     if (rc) return rc;
     a.U = kx;
     if (!mix) {

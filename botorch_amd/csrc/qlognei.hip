@@ -367,13 +367,12 @@ int qlognei_value_grad(const bta_gp_model* m, const bta_qlognei_state* st, const
   if (A.split) {
     rc = gemm_h2(A.fwd, s);
   } else {
-    rc = gemm(A.gemm_flags | BTA_GEMM_B_LOWER, A.R_pad, A.np, A.np, 1.0, A.kx, A.np, A.linv,
-              A.np, 0.0, nullptr, 0, A.vt, A.np, s);
+    rc = gemm_rows(A.gemm_flags | BTA_GEMM_B_LOWER, A.R, A.R_pad, A.np, A.kx, A.linv, A.vt, s);
   }
   if (rc) return rc;
   if (A.grad && !A.split) {
-    rc = gemm(A.gemm_flags | BTA_GEMM_B_KN | BTA_GEMM_B_UPPER, A.R_pad, A.np, A.np, 1.0, A.vt,
-              A.np, A.linv, A.np, 0.0, nullptr, 0, A.kx, A.np, s);
+    rc = gemm_rows(A.gemm_flags | BTA_GEMM_B_KN | BTA_GEMM_B_UPPER, A.R, A.R_pad, A.np, A.vt,
+                   A.linv, A.kx, s);
     if (rc) return rc;
   }
   // split mode with the gradient: U and the MC stage in one launch where it
