@@ -14,15 +14,34 @@
 // segment sums do, so the default path keeps no FP64 accumulators and runs
 // two workgroups (two waves per SIMD) on each CU.
 //
-// Tile 128 x BN (BN = 128 or 64), 256 threads = 4 waves of 64 x BN/2, K chunks
-// of 32.  Operands move global -> LDS with direct LDS loads
-// (global_load_lds_dwordx4: no registers, no ds_write) through a ring of LDS
-// stages with STAGES - 1 chunks in flight; one barrier per chunk.  Each plane
-// row (64 bytes) holds its four 16-byte chunks in XOR-swizzled slots
-// (h2_swizzle), which keeps the fragment reads free of bank conflicts; the
-// 1 KiB wave loads write contiguous LDS.  The epilogue writes C in FP32 and,
-// optionally, C's own hi/lo planes (scaled by c_scale) for a following split
-// GEMM.  Triangular K ranges follow gemm_kernel; a cost model picks BN and the
+// Operands move global -> LDS with direct LDS loads (global_load_lds_dwordx4: no
+// registers, no ds_write) through a ring of three LDS stages with two chunks of 32
+// K in flight; one barrier per chunk.  A stage row is 128 bytes, a row's chunk of
+// both planes, with the eight 16-byte pieces in slots XOR-ed by the row: every
+// ds_read_b128 is free of bank conflicts (SQ_LDS_BANK_CONFLICT 0; 64-byte rows
+// per plane had two-way conflicts, about 4 cycles a read).  The first third of a
+// chunk's products starts once the lo plane of A and the hi plane of B are in
+// registers.  The epilogue writes C in FP32 and, optionally, C's own hi/lo planes
+// (scaled by c_scale) for a following split GEMM.
+//
+// Four tiles, which give bit-identical results (us per triangular product M x N x
+// N; the 128 x 64 and 128 x 128 tiles with 64-byte rows that they replace in the
+// last column; shapes of one line were measured in one run):
+//                      64 x 64   128 x 64   128 x 128   128 x 256   before
+//     512 x  2048         24         34          42          74         42
+//     512 x  4096         48         62          79         136         79
+//    2048 x  2048         54         37          44          74         44
+//    4096 x  2048                    70          59          80         71
+//    2048 x  4096                   128         107         144        125
+//    4096 x  4096        315        248         203         184        200
+//    8192 x 16384      11600       9500                    6300       9500
+// 64 x 64 (three workgroups per CU) has the shortest chunk, 0.3 us against 0.5,
+// which is what counts while each CU has one tile or less; 128 x 256 with eight
+// waves of 64 x 64 moves half the bytes per product and runs large products at the
+// rate of a plain FP16 matrix product (1030 TFLOP/s), 128 x 128 with sixteen waves
+// of 32 x 32 fills the gap where 128 x 256 gives a CU one tile only.  128 x 64 lies
+// between, and is the tile of the launches that share CUs with other work.
+// Triangular K ranges follow gemm_kernel; for 128 x 64 a cost model picks the
 // worker count, and workers pair heavy with light tiles on each CU.
 #include "bta_common.h"
 #include "gemm.h"
@@ -40,21 +59,41 @@
 
 namespace bta {
 
-template <int BN, bool ACC64>
-__global__ __launch_bounds__(256, (H2Cfg<BN, ACC64>::WG_PER_CU)) void gemm_h2_kernel(H2Args g) {
+template <bool ACC64>
+__global__ __launch_bounds__(256, (ACC64 ? 1 : 2)) void gemm_h2_kernel(H2Args g) {
   __shared__ __attribute__((aligned(1024)))
-  unsigned char lds[H2Cfg<BN, ACC64>::STAGES * H2Cfg<BN, ACC64>::STAGE];
-  gemm_h2_body<BN, ACC64>(g, blockIdx.x, gridDim.x, lds);
+  unsigned char lds[H2Mid::STAGES * H2Mid::STAGE];
+  gemm_h2_body<ACC64>(g, blockIdx.x, gridDim.x, lds);
+}
+
+// One workgroup per tile, longest first.  64 x 64 tiles: odd rounds of one
+// workgroup per CU run backwards, so the workgroups sharing a CU hold long and
+// short tiles (the larger tiles have a CU each and keep the order: 128 x 256, 196
+// against 230 us at 4096 x 4096 with reversed rounds).
+template <typename CFG, bool REV>
+__global__ __launch_bounds__(64 * CFG::NW, (CFG::NW == 4 ? 3 : CFG::NW / 4)) void gemm_h2_tiles_kernel(
+    H2Args g, int ncu) {
+  __shared__ __attribute__((aligned(1024))) unsigned char lds[CFG::STAGES * CFG::STAGE];
+  const int MT = g.M / CFG::TM, NT = (g.N + CFG::TN - 1) / CFG::TN, total = MT * NT;
+  int t = blockIdx.x;
+  if (REV) {
+    const int rd = t / ncu;
+    if (rd & 1) t = rd * ncu + min(ncu, total - rd * ncu) - 1 - (t - rd * ncu);
+  }
+  int tm, tn;
+  decode_tile(t, g.flags, MT, NT, tm, tn);
+  gemm_h2_tile(CFG(), g, tm, tn, lds);
 }
 
 // Cost model of the worker schedule: chunk counts per worker (plus a per-tile
 // fixed cost); a CU's time is the sum over the workers it hosts, worker w on
 // CU w % ncu.
-static double h2_cost(const H2Args& g, int BN, int W) {
+static double h2_cost(const H2Args& g, int W) {
+  constexpr int BN = H2Mid::TN;
   const int MT = g.M / H2_BM, NT = g.N / BN, total = MT * NT;
   const int ncu = num_cus();
   std::vector<double> cu(ncu, 0.0);
-  const double per_chunk = BN == 128 ? 1.0 : 0.55;  // MFMA + LDS time of one K chunk
+  const double per_chunk = 0.55;  // MFMA + LDS time of one K chunk
   for (int w = 0; w < W; ++w) {
     double load = 0.0;
     for (int j = 0; j * W < total; ++j) {
@@ -72,8 +111,11 @@ static double h2_cost(const H2Args& g, int BN, int W) {
   return *std::max_element(cu.begin(), cu.end());
 }
 
+// bn: tile width.  64 with xcd >= 1: 128 x 64 tiles dealt to `workers` workgroups;
+// with xcd 0 one workgroup per tile, 64 x 64 tiles for 64, 128 x bn above.
 struct H2Plan {
   int bn, workers, xcd;
+  bool tuned;
 };
 
 // Worker groups for gemm_h2_body's strip dealing: one per XCD (workgroups go
@@ -83,20 +125,24 @@ struct H2Plan {
 // BTA_H2_XCD=1 is set: it lets one L2 serve each L^-1 strip, but on the
 // 2048 x 2048 x 2048 step products it measured no faster (50.7-52.6 us against
 // 50.2-52.9 us per forward product, step 0.189-0.193 ms against 0.185-0.187 ms).
-static int h2_xcd_allowed(const H2Args& g, int BN, int W) {
+static int h2_xcd_allowed(const H2Args& g, int W) {
   const int G = num_cus() / 32;
   if (G < 2 || !(g.flags & (BTA_GEMM_B_LOWER | BTA_GEMM_B_UPPER)) || W % G ||
-      (g.N / BN) % (2 * G))
+      (g.N / H2Mid::TN) % (2 * G))
     return 1;
   return G;
 }
 
-static int h2_xcd_groups(const H2Args& g, int BN, int W) {
+static int h2_xcd_groups(const H2Args& g, int W) {
   static const int on = [] {
     const char* e = getenv("BTA_H2_XCD");
     return e && e[0] == '1';
   }();
-  return on ? h2_xcd_allowed(g, BN, W) : 1;
+  return on ? h2_xcd_allowed(g, W) : 1;
+}
+
+static int h2_tiles(const H2Args& g, int tm, int tn) {
+  return (int)((int64_t)(g.M / tm) * ((g.N + tn - 1) / tn));
 }
 
 // The plans per problem signature: filled by the cost model below on a shape's
@@ -112,37 +158,59 @@ static std::map<H2Key, H2Plan>& h2_cache() {
   return cache;
 }
 
-static H2Plan h2_plan(const H2Args& g, bool acc64) {
+// 128 x 64 tiles with the cost model's worker count
+static H2Plan h2_mid_plan(const H2Args& g, bool acc64) {
+  const int ncu = num_cus();
+  const int slots = acc64 ? ncu : 2 * ncu;  // resident workgroups
+  H2Plan best{64, 1, 1, false};
+  double bt = 1e300;
+  const int total = h2_tiles(g, H2Mid::TM, H2Mid::TN);
+  for (int c : {slots, slots / 2, 3 * slots / 8, slots / 4}) {
+    const int W = std::max(1, std::min(c, total));
+    const double t = h2_cost(g, W);
+    if (t < bt) {
+      bt = t;
+      best = {64, W, h2_xcd_groups(g, W), false};
+    }
+  }
+  return best;
+}
+
+// The tile by the number of tiles the chip would get (table at the top): 64 x 64
+// while the 128 x 64 tiles leave every CU at most one, 128 x 256 from 1.5 of its
+// own per CU (3072 x 4096: 158 us, 128 x 128 165, 128 x 64 162), 128 x 128 from 1.75
+// of its own, 128 x 64 between.  `shared`: the launch also carries the MC stage,
+// which needs 128 x 64 workers; then 128 x 256 (and a launch of its own for the MC
+// stage) pays only where the product is long against the stage beside it, whose
+// work grows with M alone: from N = 6144 (at 8192 x 4096 the product gains 110 us
+// and the separate MC launch costs about as much).
+static H2Plan h2_plan(const H2Args& g, bool acc64, bool shared = false) {
   std::mutex& mu = h2_mu();
   auto& cache = h2_cache();
-  const auto key = std::make_tuple(g.M, g.N, g.K, g.flags, (int)acc64);
+  const auto key = std::make_tuple(g.M, g.N, g.K, g.flags, (int)acc64 + 2 * (int)shared);
   {
     std::lock_guard<std::mutex> lk(mu);
     auto it = cache.find(key);
     if (it != cache.end()) return it->second;
   }
   const int ncu = num_cus();
-  const int slots = acc64 ? ncu : 2 * ncu;  // resident workgroups
-  H2Plan best{64, 1, 1};
-  double bt = 1e300;
-  for (int bn : {64, 128}) {
-    if (g.N % bn) continue;
-    const int total = (g.M / H2_BM) * (g.N / bn);
-    for (int c : {slots, slots / 2, 3 * slots / 8, slots / 4}) {
-      const int W = std::max(1, std::min(c, total));
-      const double t = h2_cost(g, bn, W);
-      if (t < bt) {
-        bt = t;
-        best = {bn, W, h2_xcd_groups(g, bn, W)};
-      }
-    }
-  }
+  H2Plan p;
+  const int small = h2_tiles(g, H2Mid::TM, H2Mid::TN), wide = h2_tiles(g, H2Wide::TM, H2Wide::TN),
+            large = h2_tiles(g, H2Large::TM, H2Large::TN);
+  if (!acc64 && 2 * large >= 3 * ncu && (!shared || g.N >= 6144))
+    p = {H2Large::TN, large, 0, false};
+  else if (!acc64 && !shared && 4 * wide >= 7 * ncu)
+    p = {H2Wide::TN, wide, 0, false};
+  else if (!acc64 && !shared && small <= ncu)
+    p = {64, h2_tiles(g, H2Small::TM, H2Small::TN), 0, false};
+  else
+    p = h2_mid_plan(g, acc64);
   std::lock_guard<std::mutex> lk(mu);
-  cache[key] = best;
-  return best;
+  cache[key] = p;
+  return p;
 }
 
-static int h2_check(const H2Args& a) {
+int gemm_h2_check(const H2Args& a) {
   const uintptr_t al16 = (uintptr_t)a.Ah | (uintptr_t)a.Al | (uintptr_t)a.Bh | (uintptr_t)a.Bl;
   if (a.M % H2_BM || a.N % 64 || a.K % H2_BK || a.M <= 0 || a.N <= 0 || a.K <= 0 ||
       a.lda % 8 || a.ldb % 8 || a.lda < a.K || a.ldb < a.K || a.ldc < a.N || !a.Ah || !a.Al ||
@@ -155,65 +223,87 @@ static int h2_check(const H2Args& a) {
   return BTA_OK;
 }
 
-int gemm_h2_candidates(const H2Args& g, int* out, int max) {
-  if (h2_check(g)) return 0;
+int gemm_h2_candidates(const H2Args& g, bool shared, int* out, int max) {
+  if (gemm_h2_check(g)) return 0;
   const int ncu = num_cus();
   const bool acc64 = g.seg_chunks > 0;
   const int slots = acc64 ? ncu : 2 * ncu;
   int k = 0;
-  for (int bn : {64, 128}) {
-    if (g.N % bn) continue;
-    const int total = (g.M / H2_BM) * (g.N / bn);
-    int last = -1;
-    for (int c : {slots, 3 * slots / 4, slots / 2, 3 * slots / 8, slots / 4}) {
-      const int W = std::max(1, std::min(c, total));
-      if (W == last) continue;
-      last = W;
-      for (int G : {1, h2_xcd_allowed(g, bn, W)}) {
-        if (G == 1 && k > 0 && out[3 * (k - 1)] == bn && out[3 * (k - 1) + 1] == W &&
-            out[3 * (k - 1) + 2] == 1)
-          continue;
-        if (k >= max) return k;
-        out[3 * k] = bn;
-        out[3 * k + 1] = W;
-        out[3 * k + 2] = G;
-        ++k;
-      }
-    }
+  auto add = [&](int bn, int W, int G) {
+    if (k >= max) return;
+    out[3 * k] = bn;
+    out[3 * k + 1] = W;
+    out[3 * k + 2] = G;
+    ++k;
+  };
+  const int total = h2_tiles(g, H2Mid::TM, H2Mid::TN);
+  int last = -1;
+  for (int c : {slots, 3 * slots / 4, slots / 2, 3 * slots / 8, slots / 4}) {
+    const int W = std::max(1, std::min(c, total));
+    if (W == last) continue;
+    last = W;
+    add(64, W, 1);
+    const int G = h2_xcd_allowed(g, W);
+    if (G > 1) add(64, W, G);
+  }
+  if (!acc64) {
+    if (!shared) add(64, h2_tiles(g, H2Small::TM, H2Small::TN), 0);
+    if (!shared && h2_tiles(g, H2Wide::TM, H2Wide::TN) >= ncu)
+      add(H2Wide::TN, h2_tiles(g, H2Wide::TM, H2Wide::TN), 0);
+    if (h2_tiles(g, H2Large::TM, H2Large::TN) >= ncu)
+      add(H2Large::TN, h2_tiles(g, H2Large::TM, H2Large::TN), 0);
   }
   return k;
 }
 
-void gemm_h2_set_plan(const H2Args& g, int bn, int workers, int xcd_groups) {
-  const auto key = std::make_tuple(g.M, g.N, g.K, g.flags, (int)(g.seg_chunks > 0));
+void gemm_h2_set_plan(const H2Args& g, bool shared, int bn, int workers, int xcd_groups) {
+  const auto key =
+      std::make_tuple(g.M, g.N, g.K, g.flags, (int)(g.seg_chunks > 0) + 2 * (int)shared);
   std::lock_guard<std::mutex> lk(h2_mu());
-  h2_cache()[key] = H2Plan{bn, workers, xcd_groups};
+  h2_cache()[key] = H2Plan{bn, workers, xcd_groups, true};
 }
 
-int gemm_h2_plan(const H2Args& a, int* bn, int* workers, int* xcd_groups) {
-  const int rc = h2_check(a);
+int gemm_h2_shared_plan(const H2Args& a, int others, int* workers, int* xcd_groups) {
+  const int rc = gemm_h2_check(a);
   if (rc) return rc;
-  const H2Plan p = h2_plan(a, a.seg_chunks > 0);
-  *bn = p.bn;
+  const H2Plan p = h2_plan(a, a.seg_chunks > 0, true);
+  if (p.xcd == 0) return -1;
   *workers = p.workers;
-  if (xcd_groups) *xcd_groups = p.xcd;
+  *xcd_groups = p.xcd;
+  // One worker per CU when the other workgroups fit in one round in the CUs' second
+  // slots: they then start at once instead of after the first workers (2048 x 2048
+  // with 256 paired MC workgroups: 68 us with 512 workers, 50 with 256).
+  const int ncu = num_cus();
+  if (!p.tuned && others <= ncu && p.workers > ncu) {
+    *workers = ncu;
+    *xcd_groups = 1;
+  }
   return BTA_OK;
 }
 
-int gemm_h2(const H2Args& args, hipStream_t s) {
-  const int rc = h2_check(args);
+int gemm_h2(const H2Args& args, hipStream_t s, bool shared) {
+  const int rc = gemm_h2_check(args);
   if (rc) return rc;
   const bool acc64 = args.seg_chunks > 0;
-  const H2Plan p = h2_plan(args, acc64);
+  const H2Plan p = h2_plan(args, acc64, shared);
   H2Args a = args;
   a.xcd_groups = p.xcd;
-  if (p.bn == 128) {
-    if (acc64) hipLaunchKernelGGL((gemm_h2_kernel<128, true>), dim3(p.workers), dim3(256), 0, s, a);
-    else hipLaunchKernelGGL((gemm_h2_kernel<128, false>), dim3(p.workers), dim3(256), 0, s, a);
-  } else {
-    if (acc64) hipLaunchKernelGGL((gemm_h2_kernel<64, true>), dim3(p.workers), dim3(256), 0, s, a);
-    else hipLaunchKernelGGL((gemm_h2_kernel<64, false>), dim3(p.workers), dim3(256), 0, s, a);
-  }
+  if (p.bn == H2Large::TN)
+    hipLaunchKernelGGL((gemm_h2_tiles_kernel<H2Large, false>),
+                       dim3(h2_tiles(a, H2Large::TM, H2Large::TN)), dim3(64 * H2Large::NW), 0, s,
+                       a, num_cus());
+  else if (p.bn == H2Wide::TN)
+    hipLaunchKernelGGL((gemm_h2_tiles_kernel<H2Wide, false>),
+                       dim3(h2_tiles(a, H2Wide::TM, H2Wide::TN)), dim3(64 * H2Wide::NW), 0, s, a,
+                       num_cus());
+  else if (p.xcd == 0)
+    hipLaunchKernelGGL((gemm_h2_tiles_kernel<H2Small, true>),
+                       dim3(h2_tiles(a, H2Small::TM, H2Small::TN)), dim3(64 * H2Small::NW), 0, s,
+                       a, num_cus());
+  else if (acc64)
+    hipLaunchKernelGGL((gemm_h2_kernel<true>), dim3(p.workers), dim3(256), 0, s, a);
+  else
+    hipLaunchKernelGGL((gemm_h2_kernel<false>), dim3(p.workers), dim3(256), 0, s, a);
   BTA_LAUNCH_CHECK("gemm_h2_kernel");
   return BTA_OK;
 }

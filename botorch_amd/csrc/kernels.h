@@ -73,17 +73,21 @@ struct H2Args {
   int seg_chunks;           // 0: FP32 sums over all of K; > 0: FP64 sums of FP32
                             // segments of seg_chunks x 32 K
   int xcd_groups;           // set by the plan: > 1 deals column strips to G worker
-                            // groups (one per XCD), see gemm_h2_body
+                            // groups (one per XCD), see gemm_h2_body; 0: one
+                            // workgroup per tile
 };
-int gemm_h2(const H2Args& a, hipStream_t s);
-// The tile width, worker count and worker groups gemm_h2 would launch with
-// (after its checks).
-int gemm_h2_plan(const H2Args& a, int* bn, int* workers, int* xcd_groups = nullptr);
+// shared: the plan of the launch shared with the MC stage (the adjoint product).
+int gemm_h2(const H2Args& a, hipStream_t s, bool shared = false);
+int gemm_h2_check(const H2Args& a);
+// The worker count and worker groups of a launch that runs the product's 128 x 64
+// workers beside `others` workgroups of another kind (after gemm_h2's checks); -1
+// when the product is better launched alone.
+int gemm_h2_shared_plan(const H2Args& a, int others, int* workers, int* xcd_groups);
 // The plans the measured tuner tries for a problem: up to max (bn, workers,
 // xcd_groups) triples into out; returns their number.
-int gemm_h2_candidates(const H2Args& a, int* out, int max);
+int gemm_h2_candidates(const H2Args& a, bool shared, int* out, int max);
 // Makes (bn, workers, xcd_groups) the plan of the problem's signature.
-void gemm_h2_set_plan(const H2Args& a, int bn, int workers, int xcd_groups);
+void gemm_h2_set_plan(const H2Args& a, bool shared, int bn, int workers, int xcd_groups);
 int split_f16(bool f64, const void* X, int64_t ldx, int64_t rows, int64_t cols,
               int64_t rows_pad, int64_t cols_pad, float scale, bool transpose, _Float16* hi,
               _Float16* lo, int64_t ldo, hipStream_t s);

@@ -78,7 +78,7 @@ __global__ __launch_bounds__(256, 2) void gemm_h2_list_kernel(const H2Args* __re
                                                               const int4* __restrict__ tiles,
                                                               int total) {
   __shared__ __attribute__((aligned(1024))) unsigned char lds[FUSED_LDS];
-  gemm_h2_list_body<64>(tab, tiles, total, blockIdx.x, gridDim.x, lds);
+  gemm_h2_list_body(tab, tiles, total, blockIdx.x, gridDim.x, lds);
 }
 
 // Workgroups [0, W): adjoint GEMM workers; [W, W + mc blocks): the MC stage,
@@ -90,7 +90,7 @@ __global__ __launch_bounds__(256, 2) void adjoint_mc_list_kernel(
     const McArgs* __restrict__ mc, const int* __restrict__ mc_start, int nm) {
   __shared__ __attribute__((aligned(1024))) unsigned char lds[FUSED_LDS];
   if ((int)blockIdx.x < W) {
-    gemm_h2_list_body<64>(adj, tiles, total, blockIdx.x, W, lds);
+    gemm_h2_list_body(adj, tiles, total, blockIdx.x, W, lds);
   } else {
     const int blk = (int)blockIdx.x - W;
     const int m = find_item(mc_start, nm, blk);
@@ -242,8 +242,8 @@ int qlognei_batch_prepare(const bta_qlognei_batch_item* items, int nm, void* ws,
       return BTA_ERR_UNSUPPORTED;
     }
     int bn = 0, wk = 0;  // the split GEMMs' shape and alignment checks
-    rc = gemm_h2_plan(A[i].fwd, &bn, &wk);
-    if (!rc && grad) rc = gemm_h2_plan(A[i].adj, &bn, &wk);
+    rc = gemm_h2_check(A[i].fwd);
+    if (!rc && grad) rc = gemm_h2_check(A[i].adj);
     if (rc) return rc;
     const McLayout lay(q, it.state->n_b, it.state->S);
     if ((size_t)lay.total * sizeof(double) > MC_LDS_MAX) {

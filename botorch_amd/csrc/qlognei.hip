@@ -56,7 +56,7 @@ template <int Q, typename TV, int NR>
 __global__ __launch_bounds__(256, 2) void adjoint_mc_kernel(H2Args g, int W, McArgs a) {
   __shared__ __attribute__((aligned(1024))) unsigned char lds[FUSED_LDS];
   if ((int)blockIdx.x < W)
-    gemm_h2_body<64, false>(g, blockIdx.x, W, lds);
+    gemm_h2_body(g, blockIdx.x, W, lds);
   else
     mc_body<Q, TV, NR>(a, (int)blockIdx.x - W, (double*)lds);
 }
@@ -71,20 +71,21 @@ static bool fused_disabled() {
 }
 
 
-// Launches the fused kernel when it applies (q <= 5, mixed sample arithmetic,
-// the GEMM planned with 64-column tiles, the MC layout within MC_LDS_MAX);
-// returns -1 (nothing launched) otherwise.
+// Launches the fused kernel when it applies (q <= 5, mixed sample arithmetic, a
+// plan with 128 x 64 workers, the MC layout within MC_LDS_MAX); returns -1
+// (nothing launched) otherwise.
 static int launch_adjoint_mc(const H2Args& args, const McArgs& a, int q, int64_t b, bool f32,
                              hipStream_t s) {
-  int bn = 0, W = 0, G = 1;
-  const int rc = gemm_h2_plan(args, &bn, &W, &G);
+  const McLayout lay(q, a.n_b, a.S);
+  if (!f32 || q > 5 || args.seg_chunks > 0 || fused_disabled() ||
+      (size_t)lay.total * sizeof(double) > MC_LDS_MAX || b < 1 || b > (1 << 24))
+    return -1;
+  int W = 0, G = 1;
+  const int64_t others = a.nr == 2 ? (b + 1) / 2 : b;
+  const int rc = gemm_h2_shared_plan(args, (int)others, &W, &G);
   if (rc) return rc;
   H2Args g = args;
   g.xcd_groups = G;
-  const McLayout lay(q, a.n_b, a.S);
-  if (!f32 || q > 5 || bn != 64 || g.seg_chunks > 0 || fused_disabled() ||
-      (size_t)lay.total * sizeof(double) > MC_LDS_MAX || b < 1 || b > (1 << 24))
-    return -1;
   if (a.nr == 2) {
     const dim3 grid((unsigned)(W + (b + 1) / 2));
     switch (q) {
@@ -107,6 +108,9 @@ static int launch_adjoint_mc(const H2Args& args, const McArgs& a, int q, int64_t
   BTA_LAUNCH_CHECK("adjoint_mc_kernel");
   return BTA_OK;
 }
+
+// Whether the adjoint product's plan is that of the launch shared with the MC stage.
+static bool mc_fusable(const StepArgs& A) { return A.f32 && A.q <= 5; }
 
 template <int Q>
 static int launch_mc_q(const McArgs& a, int64_t b, bool f32, bool split, hipStream_t s) {
@@ -380,7 +384,7 @@ int qlognei_value_grad(const bta_gp_model* m, const bta_qlognei_state* st, const
   rc = A.grad && A.split ? launch_adjoint_mc(A.adj, A.mc, A.q, A.b, A.f32, s) : -1;
   if (rc == -1) {
     if (A.grad && A.split) {
-      rc = gemm_h2(A.adj, s);
+      rc = gemm_h2(A.adj, s, mc_fusable(A));
       if (rc) return rc;
     }
     rc = launch_mc(A.mc, A.q, A.b, A.f32, A.split, s);
@@ -483,11 +487,12 @@ int qlognei_autotune(const bta_gp_model* m, const bta_qlognei_state* st, const d
   const H2Args* prob[2] = {&A.fwd, &A.adj};
   for (int p = 0; p < (A.grad ? 2 : 1) && !rc; ++p) {
     int cand[3 * 32];
-    const int nc = gemm_h2_candidates(*prob[p], cand, 32);
+    const bool shared = p == 1 && mc_fusable(A);
+    const int nc = gemm_h2_candidates(*prob[p], shared, cand, 32);
     float best = 1e30f;
     int bi = -1;
     for (int c = 0; c < nc && !rc; ++c) {
-      gemm_h2_set_plan(*prob[p], cand[3 * c], cand[3 * c + 1], cand[3 * c + 2]);
+      gemm_h2_set_plan(*prob[p], shared, cand[3 * c], cand[3 * c + 1], cand[3 * c + 2]);
       float ms = 0.0f;
       rc = time_step(&ms);
       if (!rc && ms < best) {
@@ -496,7 +501,7 @@ int qlognei_autotune(const bta_gp_model* m, const bta_qlognei_state* st, const d
       }
     }
     if (!rc && bi >= 0) {
-      gemm_h2_set_plan(*prob[p], cand[3 * bi], cand[3 * bi + 1], cand[3 * bi + 2]);
+      gemm_h2_set_plan(*prob[p], shared, cand[3 * bi], cand[3 * bi + 1], cand[3 * bi + 2]);
       for (int i = 0; i < 3; ++i) chosen[3 * p + i] = cand[3 * bi + i];
     }
   }

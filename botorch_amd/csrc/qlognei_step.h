@@ -737,7 +737,7 @@ __device__ __forceinline__ void mc_body(const McArgs& a, const int bw, double* s
 // One launch for the adjoint GEMM U = V L^-1 and the MC stage uses the first
 // NR McLayout areas of the GEMM's LDS ring (64-column tiles; NR areas stay
 // within MC_LDS_MAX).
-constexpr int FUSED_LDS = H2Cfg<64, false>::STAGES * H2Cfg<64, false>::STAGE;
+constexpr int FUSED_LDS = H2Mid::STAGES * H2Mid::STAGE;
 static_assert(MC_LDS_MAX <= (size_t)FUSED_LDS, "MC layout must fit the fused ring");
 
 // dX = (sum of the column-tile partials + direct term) / lengthscale.
