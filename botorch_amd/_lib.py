@@ -11,6 +11,7 @@ import ctypes
 import os
 import threading
 
+import numpy as np
 import torch
 
 from .exceptions import NanError, NotPSDError, UnsupportedError
@@ -220,6 +221,11 @@ def ptr(t: torch.Tensor | None) -> ctypes.c_void_p | None:
     if not t.is_contiguous():
         raise ValueError("botorch_amd kernels need contiguous tensors")
     return ctypes.c_void_p(t.data_ptr())
+
+
+def status_bits(status: torch.Tensor) -> int:
+    """The OR of the status words, read in one copy (waits for the stream)."""
+    return int(np.bitwise_or.reduce(status.detach().cpu().numpy(), axis=None, initial=0))
 
 
 def workspace(nbytes: int, device) -> torch.Tensor:

@@ -17,6 +17,7 @@ import ctypes
 import math
 import warnings
 
+import numpy as np
 import torch
 from torch import Tensor
 
@@ -63,6 +64,19 @@ def prune_inferior_points(model: SingleTaskGP, X: Tensor, objective=None,
         counts, order_idcs = torch.sort(counts, stable=True, descending=True)
         idcs = order_idcs[:max_points]
     return X[idcs]
+
+
+# status bits after which the reference samples from the joint posterior instead
+_CACHED_ROOT_FAILED = _lib.STATUS_NAN | _lib.STATUS_NOT_PSD
+
+
+def _raise_on_status(bits: int) -> None:
+    if bits & _lib.STATUS_NAN:
+        raise NanError("Samples contain nans or infs.")
+    if bits & _lib.STATUS_NOT_PSD:
+        raise NotPSDError("Matrix not positive definite after repeatedly adding jitter.")
+    if bits & _lib.STATUS_JITTER:
+        warnings.warn("A not p.d., added jitter to the diagonal", RuntimeWarning)
 
 
 class _QLogNEIFn(torch.autograd.Function):
@@ -298,16 +312,7 @@ class qLogNoisyExpectedImprovement(torch.nn.Module):
     def check_status(status: Tensor) -> None:
         """Raise like the reference would on failed samples (utils/low_rank.py:162-171,
         psd_safe_cholesky NotPSDError); warn when jitter was added."""
-        s = torch.zeros(3, dtype=torch.bool, device=status.device)
-        for i, f in enumerate((_lib.STATUS_NAN, _lib.STATUS_NOT_PSD, _lib.STATUS_JITTER)):
-            s[i] = ((status & f) != 0).any()
-        nan, notpsd, jit = s.tolist()
-        if nan:
-            raise NanError("Samples contain nans or infs.")
-        if notpsd:
-            raise NotPSDError("Matrix not positive definite after repeatedly adding jitter.")
-        if jit:
-            warnings.warn("A not p.d., added jitter to the diagonal", RuntimeWarning)
+        _raise_on_status(_lib.status_bits(status))
 
     def autotune(self, X: Tensor) -> dict:
         """Times the plan candidates of the step's two split-FP16 products on X
@@ -333,13 +338,10 @@ class qLogNoisyExpectedImprovement(torch.nn.Module):
         return {"forward": {"bn": c[0], "workers": c[1], "xcd_groups": c[2]},
                 "adjoint": {"bn": c[3], "workers": c[4], "xcd_groups": c[5]}}
 
-    @staticmethod
-    def _cached_root_failed(status: Tensor) -> bool:
-        return bool(((status & (_lib.STATUS_NAN | _lib.STATUS_NOT_PSD)) != 0).any())
-
     def _run(self, X: Tensor, need_grad: bool):
         value, grad, status = self._launch(X, need_grad)
-        if self._cached_root_failed(status):
+        bits = _lib.status_bits(status)
+        if bits & _CACHED_ROOT_FAILED:
             # acquisition/cached_cholesky.py:143-158: the low-rank update raised
             # NanError / NotPSDError, so the whole batch is sampled again from the
             # joint posterior's Cholesky
@@ -347,7 +349,8 @@ class qLogNoisyExpectedImprovement(torch.nn.Module):
                           "ill-conditioned covariance matrix. Falling back to standard "
                           "sampling.", BotorchWarning, stacklevel=3)
             value, grad, status = self._launch(X, need_grad, joint=True)
-        self.check_status(status)
+            bits = _lib.status_bits(status)
+        _raise_on_status(bits)
         return value, grad
 
     def value_and_grad(self, X: Tensor):
@@ -398,18 +401,24 @@ class BatchedQLogNEI:
         self.q = q
         self.need_grad = need_grad
         dev = self.acqfs[0].X_baseline.device
-        self.X, self.value, self.grad, self.status = [], [], [], []
+        # every model's buffers are slices of one tensor per kind, so that a step
+        # fills, reads back and hands out each kind in one operation
+        sizes = [(b, q, acq.X_baseline.shape[-1]) for acq, b in zip(self.acqfs, restarts)]
+        n_x, n_b = sum(b * q * d for b, q, d in sizes), sum(restarts)
+        self._flat_X = torch.zeros(n_x, dtype=torch.float64, device=dev)
+        self._flat_value = torch.empty(n_b, dtype=torch.float64, device=dev)
+        self._flat_grad = (torch.empty(n_x, dtype=torch.float64, device=dev) if need_grad
+                           else None)
+        self._flat_status = torch.empty(n_b, dtype=torch.int32, device=dev)
+        self._sizes = sizes
+        self.X, self.value = self._split_x(self._flat_X), self._split_b(self._flat_value)
+        self.grad = self._split_x(self._flat_grad) if need_grad else [None] * len(acqfs)
+        self.status = self._split_b(self._flat_status)
         self._states = []
         items = (_lib.QLogNEIBatchItem * len(acqfs))()
         for i, (acq, b) in enumerate(zip(self.acqfs, restarts)):
             if acq.precision != "mixed":
                 raise UnsupportedError("the batched step runs the mixed precision only")
-            d = acq.X_baseline.shape[-1]
-            self.X.append(torch.zeros(b, q, d, dtype=torch.float64, device=dev))
-            self.value.append(torch.empty(b, dtype=torch.float64, device=dev))
-            self.grad.append(torch.empty(b, q, d, dtype=torch.float64, device=dev)
-                             if need_grad else None)
-            self.status.append(torch.empty(b, dtype=torch.int32, device=dev))
             st = _lib.QLogNEIState()  # a copy: this batch's q and base samples
             ctypes.memmove(ctypes.byref(st), ctypes.byref(acq._state), ctypes.sizeof(st))
             st.q = q
@@ -433,6 +442,14 @@ class BatchedQLogNEI:
                                                self.ws.numel(), ctypes.byref(self.plan),
                                                _lib.stream()), "qlognei_batch_prepare")
 
+    def _split_x(self, flat: Tensor):
+        """The models' b x q x d parts of a flat tensor."""
+        parts = flat.split([b * q * d for b, q, d in self._sizes])
+        return [p.view(size) for p, size in zip(parts, self._sizes)]
+
+    def _split_b(self, flat: Tensor):
+        return list(flat.split([b for b, _, _ in self._sizes]))
+
     def launch(self) -> None:
         """Enqueue one step over every model (reads ``X``, writes ``value``,
         ``grad``, ``status``); no host synchronisation."""
@@ -444,11 +461,22 @@ class BatchedQLogNEI:
         """Copies Xs[i] (restarts[i] x q x d) into the buffers, runs the step and
         returns ([value_i], [grad_i]), raising like the one-model step on failed
         samples."""
-        for buf, X in zip(self.X, Xs):
-            buf.copy_(X)
+        Xs = list(Xs)
+        buf = self._flat_X
+        if len(Xs) == len(self._sizes) and all(
+                X.shape == size and X.device == buf.device and X.dtype == buf.dtype
+                for X, size in zip(Xs, self._sizes)):
+            torch.cat([X.detach().reshape(-1) for X in Xs], out=buf)
+        else:
+            for dst, X in zip(self.X, Xs):
+                dst.copy_(X)
         self.launch()
+        bits = self._flat_status.cpu().numpy()
+        row = 0
         for i, acq in enumerate(self.acqfs):
-            if qLogNoisyExpectedImprovement._cached_root_failed(self.status[i]):
+            mine = bits[row:row + self._sizes[i][0]]
+            row += self._sizes[i][0]
+            if (mine & _CACHED_ROOT_FAILED).any():
                 # this model's cached-root update failed: its acquisition function
                 # samples it again from the joint posterior (and warns)
                 v, g = acq._run(self.X[i], self.need_grad)
@@ -456,6 +484,7 @@ class BatchedQLogNEI:
                 if self.need_grad:
                     self.grad[i].copy_(g)
                 self.status[i].zero_()
-        qLogNoisyExpectedImprovement.check_status(torch.cat(self.status))
-        return ([v.clone() for v in self.value],
-                [g.clone() for g in self.grad] if self.need_grad else None)
+                mine[:] = 0
+        _raise_on_status(int(np.bitwise_or.reduce(bits, initial=0)))
+        return (self._split_b(self._flat_value.clone()),
+                self._split_x(self._flat_grad.clone()) if self.need_grad else None)

@@ -53,20 +53,22 @@ class ExactMarginalLogLikelihood(torch.nn.Module):
     def loglik_and_grad(self):
         """Un-normalised log N(y; c, K) and its gradient w.r.t. the natural
         parameters (lengthscale d, outputscale, noise, constant)."""
+        return self._loglik_and_grad(self.model._host_values())
+
+    def _loglik_and_grad(self, values):
         L = _lib.lib()
         m = self.model
         X = m.train_inputs[0].contiguous()
         y = m.train_targets.contiguous()
         n, d = X.shape
-        hp = m.hyperparameters()
-        ls = hp["lengthscale"].cpu().tolist()
+        ls, outputscale, noise, constant = values[:4]
         need = L.bta_mll_workspace_size(n, d)
         if self._ws is None or self._ws.numel() < need:
             self._ws = _lib.workspace(need, X.device)
         out = (ctypes.c_double * (4 + d))()
         lsh = (ctypes.c_double * d)(*ls)
         _lib.check(L.bta_mll_value_grad(m.kernel_kind, _lib.ptr(X), _lib.ptr(y), n, d, lsh,
-                                        hp["outputscale"], hp["noise"], hp["constant"], 6, out,
+                                        outputscale, noise, constant, 6, out,
                                         _lib.ptr(self._ws), self._ws.numel(), _lib.stream()),
                    "mll_value_grad")
         o = list(out)
@@ -75,16 +77,20 @@ class ExactMarginalLogLikelihood(torch.nn.Module):
 
     def loss_and_grads(self):
         """loss = -(loglik + sum log priors) / n and d loss / d raw parameter."""
-        ll, g = self.loglik_and_grad()
+        params = [(name, mod, attr, getattr(mod, f"raw_{attr}"))
+                  for name, mod, attr in self._params()]
+        # parameters, their constrained values and the statistics in one read
+        values = self.model._host_values([raw for _, _, _, raw in params])
+        ll, g = self._loglik_and_grad(values)
         n = self.model.train_inputs[0].shape[0]
         total = ll
         grads = []
-        for name, mod, attr in self._params():
-            raw = getattr(mod, f"raw_{attr}").detach().cpu()
+        for (name, mod, attr, raw_p), flat in zip(params, values[5]):
             if name == "constant":
                 dv = torch.tensor(g["constant"], dtype=torch.float64)
                 grads.append(-dv / n)
                 continue
+            raw = torch.tensor(flat, dtype=torch.float64).reshape(raw_p.shape)
             c = getattr(mod, f"raw_{attr}_constraint")
             val = c.transform_value(raw)
             dv = torch.as_tensor(g[name], dtype=torch.float64).reshape(raw.shape)

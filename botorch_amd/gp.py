@@ -366,14 +366,36 @@ class SingleTaskGP(torch.nn.Module):
     def kernel_kind(self) -> int:
         return self.covar_module.kind
 
+    def _host_values(self, extra=()):
+        """The hyperparameters, the outcome statistics and the tensors ``extra`` as
+        host numbers, read in one copy (each read of its own waits for the GPU):
+        (lengthscale list, outputscale, noise, constant, (y_mean, y_std), the values
+        of each extra tensor as a flat list)."""
+        with torch.no_grad():
+            k = self.covar_module
+            t = getattr(self, "outcome_transform", None)
+            parts = [k.lengthscale, k.outputscale, self.likelihood.noise,
+                     self.mean_module.constant]
+            if t is not None:
+                parts += [t.means, t.stdvs]
+            parts += extra
+            flat = [p.detach().reshape(-1) for p in parts]
+            dev, dt = flat[0].device, torch.float64
+            if any(p.device != dev or p.dtype != dt for p in flat):
+                flat = [p.to(device=dev, dtype=dt) for p in flat]
+            vals = torch.cat(flat).tolist()
+        out, i = [], 0
+        for p in flat:
+            out.append(vals[i:i + p.numel()])
+            i += p.numel()
+        stats = (out[4][0], out[5][0]) if t is not None else (0.0, 1.0)
+        return (out[0], out[1][0], out[2][0], out[3][0], stats,
+                out[len(out) - len(extra):] if extra else [])
+
     def hyperparameters(self) -> dict:
-        k = self.covar_module
-        return {
-            "lengthscale": k.lengthscale.detach(),
-            "outputscale": float(k.outputscale.detach()),
-            "noise": float(self.likelihood.noise.detach()),
-            "constant": float(self.mean_module.constant.detach()),
-        }
+        _, outputscale, noise, constant, _, _ = self._host_values()
+        return {"lengthscale": self.covar_module.lengthscale.detach(),
+                "outputscale": outputscale, "noise": noise, "constant": constant}
 
     @property
     def y_stats(self) -> tuple[float, float]:
@@ -394,10 +416,9 @@ class SingleTaskGP(torch.nn.Module):
     def prediction_cache(self) -> dict:
         """L, L^-1, alpha and the C struct describing the model; rebuilt when a
         hyperparameter changed (like gpytorch's prediction strategy reset)."""
-        hp = self.hyperparameters()
-        key = (tuple(hp["lengthscale"].tolist()), hp["outputscale"], hp["noise"],
-               hp["constant"], self.y_stats, float(self.cholesky_jitter),
-               int(self.refine_solves))
+        lengthscale, outputscale, noise, constant, y_stats, _ = self._host_values()
+        key = (tuple(lengthscale), outputscale, noise, constant, y_stats,
+               float(self.cholesky_jitter), int(self.refine_solves))
         if self._cache is not None and self._cache_key == key:
             return self._cache
         X = self.train_inputs[0]
@@ -405,14 +426,15 @@ class SingleTaskGP(torch.nn.Module):
         L = _lib.lib()
         n, d = X.shape
         n_pad = _lib.round_up(n, 128)
-        ls = hp["lengthscale"].to(device=dev, dtype=torch.float64).contiguous()
+        ls = self.covar_module.lengthscale.detach().to(device=dev,
+                                                       dtype=torch.float64).contiguous()
         center = torch.empty(d, dtype=torch.float64, device=dev)
         xs = torch.empty(n_pad, d, dtype=torch.float64, device=dev)
         st = _lib.stream()
         _lib.check(L.bta_scale_inputs(_lib.ptr(X.contiguous()), n, d, None, _lib.ptr(ls),
                                       _lib.ptr(center), _lib.ptr(xs), n_pad, st),
                    "scale_inputs")
-        y_mean, y_std = self.y_stats
+        y_mean, y_std = y_stats
         m = _lib.GpModel()
         m.kind = self.kernel_kind
         m.d = d
@@ -421,9 +443,9 @@ class SingleTaskGP(torch.nn.Module):
         m.train_xs = _lib.ptr(xs)
         m.center = _lib.ptr(center)
         m.lengthscale = _lib.ptr(ls)
-        m.outputscale = hp["outputscale"]
-        m.noise = hp["noise"]
-        m.mean_constant = hp["constant"]
+        m.outputscale = outputscale
+        m.noise = noise
+        m.mean_constant = constant
         m.y_mean = y_mean
         m.y_std = y_std
         m.chol_jitter = float(self.cholesky_jitter)
@@ -551,10 +573,10 @@ def psd_safe_cholesky(A: Tensor, max_tries: int = 6, jitter: float = 1e-8) -> Te
         status = torch.zeros(nb, dtype=torch.int32, device=A.device)
         _lib.check(L.bta_chol_small_batched(_lib.ptr(Af), k, k, k * k, nb, max_tries, jitter,
                                             _lib.ptr(status), st), "chol_small_batched")
-        flags = [bool(((status & f) != 0).any()) for f in (_lib.STATUS_NAN, _lib.STATUS_NOT_PSD)]
-        if flags[0]:
+        bits = _lib.status_bits(status)
+        if bits & _lib.STATUS_NAN:
             raise NanError("cholesky input contains NaNs")
-        if flags[1]:
+        if bits & _lib.STATUS_NOT_PSD:
             raise NotPSDError("Matrix not positive definite after repeatedly adding jitter")
         return Af.reshape(*batch, k, k)
     kp = _lib.round_up(k, 128)
