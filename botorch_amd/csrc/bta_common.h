@@ -86,6 +86,56 @@ __host__ __device__ __forceinline__ double exp_nonpos(double x) {
   return under ? 0.0 : ldexp(p, (int)kf);
 }
 
+// n / d for a normal d whose reciprocal is normal too: reciprocal seed, two Newton
+// steps, and one residual correction of the quotient.
+__host__ __device__ __forceinline__ double div_normal(double n, double d) {
+#ifdef __HIP_DEVICE_COMPILE__
+  double r = __builtin_amdgcn_rcp(d);
+#else
+  double r = (1.0 / d) * (1.0 + 0x1p-25);  // a seed as inexact as v_rcp_f64's
+#endif
+  r = fma(fma(-d, r, 1.0), r, r);
+  r = fma(fma(-d, r, 1.0), r, r);
+  const double q = n * r;
+  return fma(fma(-d, q, n), r, q);
+}
+
+// log x for 0 < x < infinity (NaN gives NaN, infinity infinity): x = 2^k (1 + f) with
+// 1 + f in [sqrt 1/2, sqrt 2), s = f / (2 + f), log(1 + f) = 2 atanh s summed as
+// f - (f^2 / 2 - s (f^2 / 2 + R)) as in fdlibm, R = sum_{i >= 1} 2 s^2i / (2 i + 1) by
+// its Taylor series to s^22 (remainder < 1e-18 relative), and k ln 2 in two parts.
+__host__ __device__ __forceinline__ double log_pos(double x) {
+  int k;
+#ifdef __HIP_DEVICE_COMPILE__
+  double m = __builtin_amdgcn_frexp_mant(x);
+  k = __builtin_amdgcn_frexp_exp(x);
+#else
+  double m = frexp(x, &k);
+#endif
+  const bool low = m < 0.70710678118654752440;
+  m = low ? m + m : m;
+  const double kf = (double)(low ? k - 1 : k);
+  const double f = m - 1.0;
+  const double s = div_normal(f, 2.0 + f);
+  const double z = s * s;
+  double r = 2.0 / 23.0;
+  r = fma(r, z, 2.0 / 21.0);
+  r = fma(r, z, 2.0 / 19.0);
+  r = fma(r, z, 2.0 / 17.0);
+  r = fma(r, z, 2.0 / 15.0);
+  r = fma(r, z, 2.0 / 13.0);
+  r = fma(r, z, 2.0 / 11.0);
+  r = fma(r, z, 2.0 / 9.0);
+  r = fma(r, z, 2.0 / 7.0);
+  r = fma(r, z, 2.0 / 5.0);
+  r = fma(r, z, 2.0 / 3.0);
+  r *= z;
+  const double h = 0.5 * f * f;
+  const double lo = fma(s, h + r, kf * 1.90821492927058770002e-10);
+  const double v = fma(kf, 6.93147180369123816490e-01, f - (h - lo));
+  return x < 1.7976931348623157e308 ? v : x + x;
+}
+
 // sqrt(r2) for r2 >= 1e-30: v_rsq_f64 seed, one Goldschmidt step for the
 // root and half-reciprocal pair, two Newton corrections of the root.
 __device__ __forceinline__ double sqrt_pos(double r2) {
