@@ -116,6 +116,8 @@ SIGNATURES = {
                                          ctypes.POINTER(_f64), _p, _sz, _p]),
     "bta_trtri_lower": (ctypes.c_int, [_p, _i64, _p, _i64, _i64, _p, _sz, _p]),
     "bta_chol_small_batched": (ctypes.c_int, [_p, _i32, _i64, _i64, _i64, _i32, _f64, _p, _p]),
+    "bta_sobol_scramble": (ctypes.c_int, [ctypes.c_uint32, _i32, _p, _p]),
+    "bta_sobol_normal": (ctypes.c_int, [_p, _p, _p, _i32, _i64, _p, _p]),
     "bta_gp_cache_workspace_size": (_sz, [_i64]),
     "bta_gp_cache_build": (ctypes.c_int, [ctypes.POINTER(GpModel), _p, _p, _p, _p, _i32,
                                           ctypes.POINTER(_f64), _p, _sz, _p]),

@@ -200,6 +200,22 @@ int bta_chol_small_batched(double* A, int32_t n, int64_t lda, int64_t stride,
                            int32_t* status, bta_stream_t stream);
 
 /* ------------------------------------------------------------------------ */
+/* Sobol-QMC normal base samples (sampling/qmc.py:59-97,                     */
+/* utils/sampling.py:114-143: torch.quasirandom.SobolEngine + erfinv).       */
+/* ------------------------------------------------------------------------ */
+
+/* Host only: the random bits of SobolEngine(d, scramble=True, seed): rows (d x 30
+ * words, host) are the lower-triangular scrambling matrices with unit diagonal, bit
+ * 29 - k the entry of column k; shift (d words, host) the digital shifts. */
+int bta_sobol_scramble(uint32_t seed, int32_t d, uint32_t* rows, uint32_t* shift);
+
+/* out[i][j] (n x d) = sqrt2 erfinv(2 v - 1), v = 1/2 + (1 - eps)(u - 1/2), for the
+ * points u_i of the engine with the unscrambled direction numbers cols (d x 30),
+ * rows and shift of bta_sobol_scramble.  n <= 4194240. */
+int bta_sobol_normal(const uint32_t* cols, const uint32_t* rows, const uint32_t* shift,
+                     int32_t d, int64_t n, double* out, bta_stream_t stream);
+
+/* ------------------------------------------------------------------------ */
 /* GP model: SingleTaskGP exact prediction (fast_pred_var).                  */
 /* Replaces models/gpytorch.py:544-610 (BatchedMultiOutputGPyTorchModel.     */
 /* posterior) -> gpytorch ExactGP.__call__ / DefaultPredictionStrategy, with  */
