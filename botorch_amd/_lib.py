@@ -116,6 +116,9 @@ SIGNATURES = {
                                          ctypes.POINTER(_f64), _p, _sz, _p]),
     "bta_trtri_lower": (ctypes.c_int, [_p, _i64, _p, _i64, _i64, _p, _sz, _p]),
     "bta_chol_small_batched": (ctypes.c_int, [_p, _i32, _i64, _i64, _i64, _i32, _f64, _p, _p]),
+    "bta_mvn_sample": (ctypes.c_int, [_p, _p, _p, _i64, _i64, _i64, _i64, _i32, _p, _p]),
+    "bta_mvn_sample_backward": (ctypes.c_int, [_p, _p, _i64, _i64, _i64, _i64, _i32, _p, _p,
+                                               _p]),
     "bta_sobol_scramble": (ctypes.c_int, [ctypes.c_uint32, _i32, _p, _p]),
     "bta_sobol_normal": (ctypes.c_int, [_p, _p, _p, _i32, _i64, _p, _p]),
     "bta_gp_cache_workspace_size": (_sz, [_i64]),
@@ -127,6 +130,11 @@ SIGNATURES = {
     "bta_gp_posterior_backward_workspace_size": (_sz, [ctypes.POINTER(GpModel), _i64, _i32]),
     "bta_gp_posterior_backward": (ctypes.c_int, [ctypes.POINTER(GpModel), _p, _i64, _i32, _p,
                                                  _p, _p, _p, _sz, _p]),
+    "bta_gp_posterior_keep_size": (_sz, [ctypes.POINTER(GpModel), _i64, _i32]),
+    "bta_gp_posterior_keep": (ctypes.c_int, [ctypes.POINTER(GpModel), _p, _i64, _i32, _p, _p,
+                                             _p, _p, _p, _sz, _p]),
+    "bta_gp_posterior_backward_kept": (ctypes.c_int, [ctypes.POINTER(GpModel), _i64, _i32, _p,
+                                                      _p, _p, _p, _p, _sz, _p]),
     "bta_chol_small_backward": (ctypes.c_int, [_p, _p, _i32, _i64, _i64, _p, _p]),
     "bta_qlognei_prepare_workspace_size": (_sz, [ctypes.POINTER(GpModel), _i32, _i32]),
     "bta_qlognei_prepare": (ctypes.c_int, [ctypes.POINTER(GpModel),

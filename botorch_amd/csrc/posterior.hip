@@ -16,7 +16,8 @@
 //                          rows, k(xs, xs), and all the outputs
 //   post_cov_joint_kernel  above: lower 128 x 64 tiles of V V^T, the same
 //                          epilogue, the upper triangle mirrored
-// Adjoint: K_x, V and U = V L^-1 = K_x K^-1 again, then
+// Adjoint: U = V L^-1 = K_x K^-1 (with xs and V kept from the moments' call, or K_x
+// and V formed again: 120 of 520 us at 256 x 4 points and n = 2048), then
 //   post_grad_kernel       g_rc = y_std dmean_r alpha_c - sum_j S_rj U_jc with
 //                          S = y_std^2 (dC + dC^T), times dk/dxs, over a share
 //                          of the columns
@@ -329,6 +330,17 @@ struct PostWs {
   }
 };
 
+// What the adjoint takes over from the moments of the same call: xs and V.
+struct PostKeep {
+  size_t xs, vt, total;
+  PostKeep(const bta_gp_model* m, const PostLayout& lay) {
+    WsPlan p;
+    xs = p.take((size_t)lay.R_pad * m->d * 8);
+    vt = p.take((size_t)lay.R_pad * m->n_pad * 8);
+    total = p.off;
+  }
+};
+
 static int post_check(const char* what, const bta_gp_model* m, int64_t batch, int mq) {
   if (m->d < 1 || m->d > PC_MAXD || m->n < 1 || m->n_pad < m->n || m->n_pad % 128) {
     set_error("%s: bad sizes (d=%d n=%ld n_pad=%ld)", what, m->d, (long)m->n, (long)m->n_pad);
@@ -362,7 +374,8 @@ static int post_rows(const bta_gp_model* m, const double* X, int64_t batch, int 
 }
 
 int gp_posterior(const bta_gp_model* m, const double* X, int64_t batch, int mq, double* mean,
-                 double* covar_out, double* var, void* ws, size_t ws_bytes, hipStream_t s) {
+                 double* covar_out, double* var, void* keep, void* ws, size_t ws_bytes,
+                 hipStream_t s) {
   if (!m || !X || batch < 1 || mq < 1 || !m->linv || !m->alpha || batch > 65535) {
     set_error("gp_posterior: invalid arguments");
     return BTA_ERR_INVALID;
@@ -379,6 +392,11 @@ int gp_posterior(const bta_gp_model* m, const double* X, int64_t batch, int mq, 
   double* kx = (double*)(base + w.kx);
   double* vt = (double*)(base + w.vt);
   double* part = (double*)(base + w.part);
+  if (keep) {
+    const PostKeep k(m, w.lay);
+    xs = (double*)((char*)keep + k.xs);
+    vt = (double*)((char*)keep + k.vt);
+  }
   const int64_t np = m->n_pad;
   rc = post_rows(m, X, batch, mq, w.lay, xs, kx, part, s);
   if (rc) return rc;
@@ -639,10 +657,11 @@ static void post_grad_kind(PostGradArgs& a, int kind, bool mix, hipStream_t s) {
     post_grad_mode<RB, MD, BTA_KERNEL_RBF>(a, mix, g, s);
 }
 
+// keep: null, or the xs and V of the moments' call (X is then not read)
 int gp_posterior_backward(const bta_gp_model* m, const double* X, int64_t batch, int mq,
-                          const double* dmean, const double* dcov, double* dX, void* ws,
-                          size_t ws_bytes, hipStream_t s) {
-  if (!m || !X || !dX || batch < 1 || mq < 1 || !m->linv || !m->alpha || batch > 65535 ||
+                          const double* dmean, const double* dcov, double* dX, const void* keep,
+                          void* ws, size_t ws_bytes, hipStream_t s) {
+  if (!m || (!X && !keep) || !dX || batch < 1 || mq < 1 || !m->linv || !m->alpha || batch > 65535 ||
       (!dmean && !dcov)) {
     set_error("gp_posterior_backward: invalid arguments");
     return BTA_ERR_INVALID;
@@ -661,16 +680,25 @@ int gp_posterior_backward(const bta_gp_model* m, const double* X, int64_t batch,
   double* S = (double*)(base + w.S);
   const int64_t np = m->n_pad, mp = w.lay.mq_pad, R_pad = w.lay.R_pad;
   const bool mix = mq <= POST_SMALL_MQ;
-  rc = post_rows(m, X, batch, mq, w.lay, xs, kx, nullptr, s);
-  if (rc) return rc;
+  const double* V = vt;
+  if (keep) {
+    const PostKeep k(m, w.lay);
+    xs = (double*)((char*)keep + k.xs);
+    V = (const double*)((const char*)keep + k.vt);
+  } else {
+    rc = post_rows(m, X, batch, mq, w.lay, xs, kx, nullptr, s);
+    if (rc) return rc;
+  }
   PostGradArgs a;
   a.U = nullptr;
   if (dcov) {
-    // V = K_x L^-T into vt, then U = V L^-1 into kx
+    // V = K_x L^-T into vt (unless it was kept), then U = V L^-1 into kx
     const int64_t R = w.lay.used(batch, mq);
-    rc = gemm_rows(BTA_GEMM_B_LOWER, R, R_pad, np, kx, m->linv, vt, s);
-    if (rc) return rc;
-    rc = gemm_rows(BTA_GEMM_B_KN | BTA_GEMM_B_UPPER, R, R_pad, np, vt, m->linv, kx, s);
+    if (!keep) {
+      rc = gemm_rows(BTA_GEMM_B_LOWER, R, R_pad, np, kx, m->linv, vt, s);
+      if (rc) return rc;
+    }
+    rc = gemm_rows(BTA_GEMM_B_KN | BTA_GEMM_B_UPPER, R, R_pad, np, V, m->linv, kx, s);
     if (rc) return rc;
     a.U = kx;
     if (!mix) {
@@ -731,8 +759,37 @@ extern "C" size_t bta_gp_posterior_workspace_size(const bta_gp_model* m, int64_t
 extern "C" int bta_gp_posterior(const bta_gp_model* m, const double* X, int64_t batch,
                                 int32_t mq, double* mean, double* covar, double* var, void* ws,
                                 size_t ws_bytes, bta_stream_t stream) {
-  return bta::gp_posterior(m, X, batch, mq, mean, covar, var, ws, ws_bytes,
+  return bta::gp_posterior(m, X, batch, mq, mean, covar, var, nullptr, ws, ws_bytes,
                            (hipStream_t)stream);
+}
+
+extern "C" size_t bta_gp_posterior_keep_size(const bta_gp_model* m, int64_t batch, int32_t mq) {
+  if (!m || batch < 1 || mq < 1) return 0;
+  return bta::PostKeep(m, bta::PostLayout(batch, mq)).total;
+}
+
+extern "C" int bta_gp_posterior_keep(const bta_gp_model* m, const double* X, int64_t batch,
+                                     int32_t mq, double* mean, double* covar, double* var,
+                                     void* keep, void* ws, size_t ws_bytes,
+                                     bta_stream_t stream) {
+  if (!keep) {
+    bta::set_error("gp_posterior_keep: null pointer");
+    return BTA_ERR_INVALID;
+  }
+  return bta::gp_posterior(m, X, batch, mq, mean, covar, var, keep, ws, ws_bytes,
+                           (hipStream_t)stream);
+}
+
+extern "C" int bta_gp_posterior_backward_kept(const bta_gp_model* m, int64_t batch, int32_t mq,
+                                              const double* dmean, const double* dcov,
+                                              double* dX, const void* keep, void* ws,
+                                              size_t ws_bytes, bta_stream_t stream) {
+  if (!keep) {
+    bta::set_error("gp_posterior_backward_kept: null pointer");
+    return BTA_ERR_INVALID;
+  }
+  return bta::gp_posterior_backward(m, nullptr, batch, mq, dmean, dcov, dX, keep, ws, ws_bytes,
+                                    (hipStream_t)stream);
 }
 
 extern "C" size_t bta_gp_posterior_backward_workspace_size(const bta_gp_model* m,
@@ -745,6 +802,10 @@ extern "C" int bta_gp_posterior_backward(const bta_gp_model* m, const double* X,
                                          int32_t mq, const double* dmean, const double* dcov,
                                          double* dX, void* ws, size_t ws_bytes,
                                          bta_stream_t stream) {
-  return bta::gp_posterior_backward(m, X, batch, mq, dmean, dcov, dX, ws, ws_bytes,
+  if (!X) {
+    bta::set_error("gp_posterior_backward: invalid arguments");
+    return BTA_ERR_INVALID;
+  }
+  return bta::gp_posterior_backward(m, X, batch, mq, dmean, dcov, dX, nullptr, ws, ws_bytes,
                                     (hipStream_t)stream);
 }

@@ -502,59 +502,82 @@ class SingleTaskGP(torch.nn.Module):
 
     def _posterior_moments(self, Xf: Tensor):
         """Mean (nb x mq) and covariance (nb x mq x mq), original outcome scale."""
+        mean, cov, _, _ = self._posterior_call(Xf, False)
+        return mean, cov
+
+    def _posterior_call(self, Xf: Tensor, for_grad: bool):
+        """The moments, the prediction cache they came from and, for_grad, the buffer
+        the adjoint takes over (None above KEEP_BYTES: it then recomputes)."""
         c = self.prediction_cache()
         L = _lib.lib()
+        m = ctypes.byref(c["model"])
         nb, mq, _ = Xf.shape
         dev = Xf.device
         mean = torch.empty(nb, mq, dtype=torch.float64, device=dev)
         cov = torch.empty(nb, mq, mq, dtype=torch.float64, device=dev)
-        ws = _lib.workspace(L.bta_gp_posterior_workspace_size(ctypes.byref(c["model"]), nb, mq),
-                            dev)
-        _lib.check(L.bta_gp_posterior(ctypes.byref(c["model"]), _lib.ptr(Xf), nb, mq,
-                                      _lib.ptr(mean), _lib.ptr(cov), None, _lib.ptr(ws),
-                                      ws.numel(), _lib.stream()), "gp_posterior")
-        return mean, cov
+        ws = _lib.workspace(L.bta_gp_posterior_workspace_size(m, nb, mq), dev)
+        size = L.bta_gp_posterior_keep_size(m, nb, mq) if for_grad else 0
+        keep = _lib.workspace(size, dev) if 0 < size <= KEEP_BYTES else None
+        if keep is not None:
+            _lib.check(L.bta_gp_posterior_keep(m, _lib.ptr(Xf), nb, mq, _lib.ptr(mean),
+                                               _lib.ptr(cov), None, _lib.ptr(keep), _lib.ptr(ws),
+                                               ws.numel(), _lib.stream()), "gp_posterior")
+        else:
+            _lib.check(L.bta_gp_posterior(m, _lib.ptr(Xf), nb, mq, _lib.ptr(mean),
+                                          _lib.ptr(cov), None, _lib.ptr(ws), ws.numel(),
+                                          _lib.stream()), "gp_posterior")
+        return mean, cov, c, keep
 
-    def _posterior_backward(self, Xf: Tensor, dmean: Tensor | None, dcov: Tensor | None):
-        """d X (nb x mq x d) of <dmean, mean> + <dcov, covariance>."""
-        c = self.prediction_cache()
+    @staticmethod
+    def _posterior_backward(c: dict, Xf: Tensor, dmean: Tensor | None, dcov: Tensor | None,
+                            keep: Tensor | None = None):
+        """d X (nb x mq x d) of <dmean, mean> + <dcov, covariance> for the moments
+        formed with the prediction cache c."""
         L = _lib.lib()
+        m = ctypes.byref(c["model"])
         nb, mq, d = Xf.shape
         dev = Xf.device
         dX = torch.empty(nb, mq, d, dtype=torch.float64, device=dev)
         if dmean is None and dcov is None:
             return dX.zero_()
-        ws = _lib.workspace(L.bta_gp_posterior_backward_workspace_size(
-            ctypes.byref(c["model"]), nb, mq), dev)
+        ws = _lib.workspace(L.bta_gp_posterior_backward_workspace_size(m, nb, mq), dev)
         dm = None if dmean is None else dmean.to(torch.float64).contiguous()
         dc = None if dcov is None else dcov.to(torch.float64).contiguous()
-        _lib.check(L.bta_gp_posterior_backward(ctypes.byref(c["model"]), _lib.ptr(Xf), nb, mq,
-                                               _lib.ptr(dm), _lib.ptr(dc), _lib.ptr(dX),
-                                               _lib.ptr(ws), ws.numel(), _lib.stream()),
-                   "gp_posterior_backward")
+        if keep is not None:
+            _lib.check(L.bta_gp_posterior_backward_kept(
+                m, nb, mq, _lib.ptr(dm), _lib.ptr(dc), _lib.ptr(dX), _lib.ptr(keep),
+                _lib.ptr(ws), ws.numel(), _lib.stream()), "gp_posterior_backward")
+        else:
+            _lib.check(L.bta_gp_posterior_backward(
+                m, _lib.ptr(Xf), nb, mq, _lib.ptr(dm), _lib.ptr(dc), _lib.ptr(dX), _lib.ptr(ws),
+                ws.numel(), _lib.stream()), "gp_posterior_backward")
         return dX
 
     def forward(self, X: Tensor):
         raise UnsupportedError("use posterior(); the prior MVN is not materialised")
 
 
+# Largest buffer (scaled points and V = K_x L^-T) a posterior that requires grad holds
+# for its adjoint
+KEEP_BYTES = 256 << 20
+
+
 class _PosteriorFn(torch.autograd.Function):
     """Posterior moments with the adjoint of bta_gp_posterior_backward (the
     reference keeps SingleTaskGP.posterior differentiable in X,
-    models/gpytorch.py:544-610)."""
+    models/gpytorch.py:544-610), of the prediction cache the moments came from."""
 
     @staticmethod
     def forward(ctx, Xf: Tensor, model: "SingleTaskGP"):
         Xc = Xf.detach().contiguous()
-        mean, cov = model._posterior_moments(Xc)
-        ctx.model = model
-        ctx.save_for_backward(Xc)
+        mean, cov, ctx.cache, keep = model._posterior_call(Xc, True)
+        ctx.save_for_backward(Xc, keep)
         return mean, cov
 
     @staticmethod
     def backward(ctx, dmean: Tensor | None, dcov: Tensor | None):
-        (Xc,) = ctx.saved_tensors
-        return ctx.model._posterior_backward(Xc, dmean, dcov), None
+        Xc, keep = ctx.saved_tensors
+        return SingleTaskGP._posterior_backward(ctx.cache, Xc, dmean, dcov, keep), None
 
 
 # ----------------------------------------------------------------------------
@@ -659,6 +682,17 @@ class GPyTorchPosterior:
         z = base_samples.to(self._mean).expand(*sample_shape, *self._mean.shape)
         S = int(torch.Size(sample_shape).numel())
         nb = int(self._mean[..., 0].numel())
+        if m <= MVN_SAMPLE_MAX and S * nb > 0 and z.dtype == Lt.dtype == torch.float64:
+            # base samples shared by the batch stay an expanded view
+            zv = z.reshape(S, nb, m)
+            if zv.stride(-1) != 1 and m > 1:
+                zv = zv.contiguous()
+            mean, L = self._mean.reshape(nb, m), Lt.reshape(nb, m, m)
+            if torch.is_grad_enabled() and (Lt.requires_grad or mean.requires_grad):
+                out = _MvnSampleFn.apply(mean, L, zv)
+            else:
+                out = _mvn_sample(mean, L, zv)
+            return out.reshape(*sample_shape, *self._mean.shape, 1)
         zf = z.reshape(S, nb, m).permute(1, 0, 2).contiguous()  # nb x S x m
         if torch.is_grad_enabled() and Lt.requires_grad:
             out = _LowerMatmulFn.apply(Lt.reshape(nb, m, m), zf)
@@ -671,6 +705,45 @@ class GPyTorchPosterior:
         sample_shape = sample_shape or torch.Size([1])
         z = torch.randn(*sample_shape, *self._mean.shape, dtype=self.dtype, device=self.device)
         return self.rsample_from_base_samples(sample_shape, z)
+
+
+# points per element up to which samples are formed by bta_mvn_sample (one launch on
+# the unpadded elements); above, by the GEMM on elements padded to 64
+MVN_SAMPLE_MAX = 16
+
+
+def _mvn_sample(mean: Tensor, Lt: Tensor, z: Tensor) -> Tensor:
+    """mean + L z: S x nb x m for mean nb x m, L nb x m x m and z S x nb x m (any
+    strides but the last)."""
+    S, nb, m = z.shape
+    mean, Lt = mean.detach().contiguous(), Lt.detach().contiguous()
+    out = torch.empty(S, nb, m, dtype=torch.float64, device=z.device)
+    _lib.check(_lib.lib().bta_mvn_sample(_lib.ptr(mean), _lib.ptr(Lt), z.data_ptr(), z.stride(0),
+                                         z.stride(1), S, nb, m, _lib.ptr(out), _lib.stream()),
+               "mvn_sample")
+    return out
+
+
+class _MvnSampleFn(torch.autograd.Function):
+    """Samples mean + L z with dmean = sum g and dL = tril(sum g z^T); the base
+    samples are constants."""
+
+    @staticmethod
+    def forward(ctx, mean: Tensor, Lt: Tensor, z: Tensor):
+        ctx.save_for_backward(z)
+        return _mvn_sample(mean, Lt, z)
+
+    @staticmethod
+    def backward(ctx, g: Tensor):
+        (z,) = ctx.saved_tensors
+        S, nb, m = z.shape
+        g = g.to(torch.float64).contiguous()
+        dmean = torch.empty(nb, m, dtype=torch.float64, device=g.device)
+        dL = torch.empty(nb, m, m, dtype=torch.float64, device=g.device)
+        _lib.check(_lib.lib().bta_mvn_sample_backward(
+            _lib.ptr(g), z.data_ptr(), z.stride(0), z.stride(1), S, nb, m, _lib.ptr(dmean),
+            _lib.ptr(dL), _lib.stream()), "mvn_sample_backward")
+        return dmean, dL, None
 
 
 def _batched_lower_matmul(Lt: Tensor, Z: Tensor) -> Tensor:

@@ -193,6 +193,19 @@ int bta_trtri_lower(const double* L, int64_t ldl, double* Linv, int64_t ldinv,
 int bta_chol_small_backward(const double* L, const double* dL, int32_t n, int64_t stride,
                             int64_t batch, double* dA, bta_stream_t stream);
 
+/* Samples of batch small multivariate normals (posteriors/gpytorch.py:86-127,
+ * rsample_from_base_samples): out (S x batch x m) = mean + L z for mean batch x m,
+ * lower-triangular L batch x m x m and base samples z(s, b) = z + s z_s + b z_b (m
+ * consecutive doubles; z_b 0 for samples shared by the batch).  1 <= m <= 16. */
+int bta_mvn_sample(const double* mean, const double* L, const double* z, int64_t z_s, int64_t z_b,
+                   int64_t S, int64_t batch, int32_t m, double* out, bta_stream_t stream);
+
+/* Its adjoint for g (S x batch x m): dmean (batch x m) = sum_s g, dL (batch x m x m)
+ * = tril(sum_s g z^T). */
+int bta_mvn_sample_backward(const double* g, const double* z, int64_t z_s, int64_t z_b, int64_t S,
+                            int64_t batch, int32_t m, double* dmean, double* dL,
+                            bta_stream_t stream);
+
 /* Batched Cholesky of small n x n matrices (n <= 64) with per-matrix jitter
  * escalation; status[b] gets BTA_STATUS_* bits.  Strict upper triangle zeroed. */
 int bta_chol_small_batched(double* A, int32_t n, int64_t lda, int64_t stride,
@@ -275,6 +288,18 @@ size_t bta_gp_posterior_backward_workspace_size(const bta_gp_model* m, int64_t b
 int bta_gp_posterior_backward(const bta_gp_model* m, const double* X, int64_t batch, int32_t mq,
                               const double* dmean, const double* dcov, double* dX, void* ws,
                               size_t ws_bytes, bta_stream_t stream);
+
+/* The pair above with the adjoint's inputs handed over: bta_gp_posterior that also
+ * leaves what the adjoint needs (the scaled points and V) in keep, and the adjoint
+ * from it, with the model of that call. */
+size_t bta_gp_posterior_keep_size(const bta_gp_model* m, int64_t batch, int32_t mq);
+int bta_gp_posterior_keep(const bta_gp_model* m, const double* X, int64_t batch, int32_t mq,
+                          double* mean, double* covar, double* var, void* keep, void* ws,
+                          size_t ws_bytes, bta_stream_t stream);
+int bta_gp_posterior_backward_kept(const bta_gp_model* m, int64_t batch, int32_t mq,
+                                   const double* dmean, const double* dcov, double* dX,
+                                   const void* keep, void* ws, size_t ws_bytes,
+                                   bta_stream_t stream);
 
 /* ------------------------------------------------------------------------ */
 /* qLogNoisyExpectedImprovement (cache_root=True, fat=True, incremental,     */

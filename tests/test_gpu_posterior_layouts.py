@@ -81,3 +81,55 @@ def test_posterior_nan_stays_in_its_batch_element():
         assert torch.isnan(cov[2, 1]).all()
         keep = [0, 1, 3, 4]
         assert torch.equal(cov[keep], ref[keep])
+
+
+@pytest.mark.parametrize("nb,m,S,shared", [(1, 1, 1, True), (3, 4, 64, True), (5, 7, 33, False),
+                                           (2, 16, 300, True), (2, 17, 20, True)])
+def test_samples_and_their_gradient(nb, m, S, shared):
+    """Samples over the packed kernel (m <= 16) and the GEMM above, with base samples
+    shared by the batch (an expanded view) or one set each, against torch: sums of at
+    most max(m, S) products, 1e-12 of the largest entry."""
+    g = torch.Generator().manual_seed(m + S)
+    A = torch.randn(nb, m, m, generator=g, dtype=torch.float64)
+    cov = (A @ A.transpose(-1, -2) + m * torch.eye(m, dtype=torch.float64)).to(DEV)
+    mean = torch.randn(nb, m, generator=g, dtype=torch.float64).to(DEV)
+    z = torch.randn(S, 1 if shared else nb, m, generator=g, dtype=torch.float64).to(DEV)
+    w = torch.randn(S, nb, m, generator=g, dtype=torch.float64).to(DEV)
+    args = [mean.clone().requires_grad_(True), cov.clone().requires_grad_(True)]
+    post = B.GPyTorchPosterior(*args)
+    out = post.rsample_from_base_samples(torch.Size([S]), z.expand(S, nb, m))
+    got = torch.autograd.grad(out.squeeze(-1), args, w)
+    ref_args = [mean.cpu().requires_grad_(True), cov.cpu().requires_grad_(True)]
+    L = torch.linalg.cholesky(ref_args[1])
+    ref = ref_args[0] + torch.stack([(L * v.unsqueeze(-2)).sum(-1)
+                                     for v in z.cpu().expand(S, nb, m)])
+    want = torch.autograd.grad(ref, ref_args, w.cpu())
+    for x, y in zip([out.detach().squeeze(-1), *got], [ref.detach(), *want]):
+        assert x.shape == y.shape
+        assert (x.cpu() - y).abs().max() < 1e-12 * y.abs().max() * max(m, S)
+    with torch.no_grad():
+        plain = B.GPyTorchPosterior(mean, cov).rsample_from_base_samples(
+            torch.Size([S]), z.expand(S, nb, m))
+    assert torch.equal(plain, out.detach())
+
+
+def test_posterior_adjoint_kept_and_recomputed_agree(monkeypatch):
+    """The adjoint from the moments' own buffer equals the one that forms K_x and V
+    again (above KEEP_BYTES) bit for bit, and belongs to the hyperparameters of the
+    forward pass."""
+    from botorch_amd import gp as G
+    model, _ = _pair(150, 5, O.MATERN52)
+    for mq in (3, 40):
+        X = torch.rand(4, mq, 5, dtype=torch.float64, device=DEV, requires_grad=True)
+        grads = []
+        for limit in (G.KEEP_BYTES, 0):
+            monkeypatch.setattr(G, "KEEP_BYTES", limit)
+            post = model.posterior(X)
+            loss = post.mean.sum() + post.covariance_matrix.square().sum()
+            if not limit:
+                noise = model.likelihood.noise.detach().clone()
+                model.likelihood.noise = 0.5
+            grads.append(torch.autograd.grad(loss, X)[0])
+        model.likelihood.noise = noise
+        monkeypatch.undo()
+        assert torch.equal(*grads)
