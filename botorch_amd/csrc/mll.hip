@@ -4,7 +4,9 @@
 //   log p(y) = -1/2 (|t|^2 + 2 sum log L_ii + n log 2 pi)
 //   d log p / d theta = 1/2 sum_ij W_ij dK_ij/dtheta,   W = a a^T - K^-1
 //
-// K^-1 = X^T X with X = L^-1 is never stored: mll_trace_kernel forms each
+// K^-1 = X^T X with X = L^-1 is never stored.  Up to trs_max_n points
+// mll_trace_small_kernel forms 32 x 32 lower tiles of it, one workgroup each; above,
+// mll_trace_kernel forms each
 // lower 128 x 64 tile of it on the FP64 MFMA main loop (d_mainloop, both
 // operands read K-major straight from X), the K range of a tile,
 // [max(128 tm, 64 tn), n_pad), cut into chunks of KC so that no task grows
@@ -35,6 +37,13 @@ namespace bta {
 
 constexpr int TR_B = 128;   // trace tile
 constexpr int TR_KC = 4096;  // K chunk per task
+constexpr int TRS = 32;     // small trace tile
+// Padded points up to which the small tiles are used.  Whole calls, large / small
+// tiles, us: n = 150 196 / 120, 512 297 / 236, 1000 508 / 422, 2048 1020 / 926, 3000
+// 1600 / 1555; with more than 16 coordinates the epilogue of the small tiles weighs
+// more: n = 2048 1033 / 1027.  (Below the line n is also padded to 64 instead of 128
+// and the products around the trace take fewer launches.)
+inline int trs_max_n(int d) { return d <= 16 ? 3072 : 2048; }
 
 struct TraceArgs {
   const double* X;  // L^-1 (lower), n_pad x n_pad, row stride ld
@@ -393,14 +402,16 @@ static int trace_schedule(int MT, int CB, int n_pad, int W, const int** out) {
 struct MllWs {
   int64_t n_pad;
   int W, MD;
-  size_t ls, center, xs, L, Linv, fact, t, lgd, alpha, part, partial, out, total;
+  bool small;
+  size_t xs, L, Linv, fact, t, lgd, alpha, part, partial, out, total;
   MllWs(int64_t n, int d) {
-    n_pad = round_up(n, 128);
-    MD = d <= 16 ? 16 : 32;
-    W = 2 * num_cus();
+    // the large trace tiles need a multiple of 128
+    small = round_up(n, 64) <= trs_max_n(d);
+    n_pad = round_up(n, small ? 64 : 128);
+    MD = small && d <= 8 ? 8 : d <= 16 ? 16 : 32;
+    const int64_t T = n_pad / TRS;
+    W = small ? (int)(T * (T + 1) / 2) : 2 * num_cus();
     WsPlan p;
-    ls = p.take(d * 8);
-    center = p.take(d * 8);
     xs = p.take((size_t)n_pad * d * 8);
     L = p.take((size_t)n_pad * n_pad * 8);
     Linv = p.take((size_t)n_pad * n_pad * 8);
@@ -414,6 +425,190 @@ struct MllWs {
     total = p.off;
   }
 };
+
+// Trace terms for small n: the large tiles leave the chip nearly idle there (6 tasks
+// at n = 150, whose 32 kernel values per thread in turn took most of 41 us).  One
+// workgroup per lower 32 x 32 tile; the four waves split the tile's K range
+// [32 ti, n_pad) in chunks of 16 with the fragments loaded straight to registers (X is
+// read K-major, four rows of 256 bytes per load), their partial tiles are added
+// through LDS in wave order, and each thread then evaluates four point pairs.  A
+// lane's two neighbouring columns are the rows 2 l16, 2 l16 + 1 of the two blocks.
+template <int MD, int KIND>
+__global__ __launch_bounds__(256) void mll_trace_small_kernel(TraceArgs a) {
+  __shared__ double red[4][4][4][64];
+  __shared__ double xr[TRS][MD + 1], xc[TRS][MD + 1];
+  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+  const int l16 = lane & 15, gq = lane >> 4, d = a.d;
+  const int t = blockIdx.x;
+  int ti = (int)((__builtin_sqrt(8.0 * (double)t + 1.0) - 1.0) * 0.5);
+  while ((ti + 1) * (ti + 2) / 2 <= t) ++ti;
+  while (ti * (ti + 1) / 2 > t) --ti;
+  const int tj = t - ti * (ti + 1) / 2;
+  const int kb = ti * TRS, nk = (a.n_pad - kb) / 16;
+  const double* pa = a.X + (int64_t)(kb + 2 * gq) * a.ld + 2 * l16 + ti * TRS;
+  const double* pb = pa + (tj - ti) * TRS;
+  // a[s]: row k = 8 (s / 2) + 2 g + s % 2 of the chunk, the lane's two columns
+  auto load = [&](int c, v2d(&x)[4], v2d(&y)[4]) {
+#pragma unroll
+    for (int s = 0; s < 4; ++s) {
+      const int64_t o = ((int64_t)16 * c + 8 * (s >> 1) + (s & 1)) * a.ld;
+      x[s] = *(const v2d*)(pa + o);
+      y[s] = *(const v2d*)(pb + o);
+    }
+  };
+  v4d acc[2][2];
+#pragma unroll
+  for (int mi = 0; mi < 2; ++mi)
+#pragma unroll
+    for (int ni = 0; ni < 2; ++ni) acc[mi][ni] = (v4d)(0.0);
+  auto mul = [&](const v2d(&x)[4], const v2d(&y)[4]) {
+#pragma unroll
+    for (int s = 0; s < 4; ++s)
+#pragma unroll
+      for (int mi = 0; mi < 2; ++mi)
+#pragma unroll
+        for (int ni = 0; ni < 2; ++ni)
+          acc[mi][ni] = __builtin_amdgcn_mfma_f64_16x16x4f64(x[s][mi], y[s][ni], acc[mi][ni], 0, 0, 0);
+  };
+  v2d x0[4], y0[4], x1[4], y1[4];
+  int c = wv;
+  if (c < nk) load(c, x0, y0);
+  // the tile's scaled points, while the first chunks are on their way
+  for (int e = threadIdx.x; e < 2 * TRS * MD; e += 256) {
+    const int r = (e / MD) & (TRS - 1), j = e % MD;
+    const bool col = e >= TRS * MD;
+    const int p = (col ? tj : ti) * TRS + r;
+    const double v = (j < d && p < a.n) ? a.xs[(int64_t)p * d + j] : 0.0;
+    if (col) xc[r][j] = v;
+    else xr[r][j] = v;
+  }
+  for (; c < nk; c += 8) {
+    if (c + 4 < nk) load(c + 4, x1, y1);
+    mul(x0, y0);
+    if (c + 4 >= nk) break;
+    if (c + 8 < nk) load(c + 8, x0, y0);
+    mul(x1, y1);
+  }
+#pragma unroll
+  for (int f = 0; f < 4; ++f)
+#pragma unroll
+    for (int q = 0; q < 4; ++q) red[wv][f][q][lane] = acc[f >> 1][f & 1][q];
+  __syncthreads();
+  // wave wv: fragment (wv / 2, wv % 2)
+  const int jl = 2 * l16 + (wv & 1), gj = tj * TRS + jl;
+  const bool jok = gj < a.n;
+  const double aj = jok ? a.alpha[gj] : 0.0;
+  double v[MD + 2];
+#pragma unroll
+  for (int e = 0; e < MD + 2; ++e) v[e] = 0.0;
+#pragma unroll
+  for (int q = 0; q < 4; ++q) {
+    const int il = 2 * (gq + 4 * q) + (wv >> 1), gi = ti * TRS + il;
+    const bool ok = jok && gi < a.n && gi >= gj;
+    const double pij = (red[0][wv][q][lane] + red[1][wv][q][lane]) +
+                       (red[2][wv][q][lane] + red[3][wv][q][lane]);
+    const double wij = a.alpha[gi] * aj - pij;
+    const double f = ok ? (gi == gj ? 1.0 : 2.0) : 0.0;
+    double r2 = 0.0, dsq[MD];
+#pragma unroll
+    for (int j = 0; j < MD; ++j) {
+      const double df = xr[il][j] - xc[jl][j];
+      dsq[j] = df * df;
+      r2 += dsq[j];
+    }
+    double kv, h;
+    if (KIND == BTA_KERNEL_MATERN52) {
+      const double r = sqrt_pos(fmax(r2, 1e-30));
+      const double sr = 2.2360679774997896964 * r;
+      const double e = a.s * exp_nonpos(-sr);
+      kv = (1.0 + sr + (5.0 / 3.0) * r2) * e;
+      h = (5.0 / 3.0) * (1.0 + sr) * e;
+    } else {
+      kv = a.s * exp_nonpos(-0.5 * r2);
+      h = kv;
+    }
+    const double fw = ok ? f * wij : 0.0;
+    v[0] = fma(fw, kv, v[0]);
+    v[1] += (ok && gi == gj) ? wij : 0.0;
+    const double fwh = fw * h;
+#pragma unroll
+    for (int j = 0; j < MD; ++j) v[2 + j] = fma(fwh, dsq[j], v[2 + j]);
+  }
+  __syncthreads();  // red is read; it takes the waves' sums now
+  double* sums = &red[0][0][0][0];
+  if constexpr (MD + 2 <= 32) {
+    int e;
+    const double s = wave_sum_spread<MD + 2>(v, &e);
+    if (e >= 0) sums[wv * (MD + 2) + e] = s;
+  } else {
+    wave_sum_n<MD + 2>(v);
+    if (lane == 0)
+#pragma unroll
+      for (int e = 0; e < MD + 2; ++e) sums[wv * (MD + 2) + e] = v[e];
+  }
+  __syncthreads();
+  for (int e = threadIdx.x; e < MD + 2; e += 256)
+    a.partial[(int64_t)t * (MD + 2) + e] = sums[e] + sums[(MD + 2) + e] + sums[2 * (MD + 2) + e] +
+                                           sums[3 * (MD + 2) + e];
+}
+
+template <int MD>
+static void launch_trace_small(int kind, const TraceArgs& ta, int W, hipStream_t st) {
+  if (kind == BTA_KERNEL_MATERN52)
+    hipLaunchKernelGGL((mll_trace_small_kernel<MD, BTA_KERNEL_MATERN52>), dim3(W), dim3(256), 0,
+                       st, ta);
+  else
+    hipLaunchKernelGGL((mll_trace_small_kernel<MD, BTA_KERNEL_RBF>), dim3(W), dim3(256), 0, st,
+                       ta);
+}
+
+// a = X^T t in one launch for small n: 64 columns per workgroup, its four waves split
+// the rows i >= j; the two-launch form above needs enough row blocks to pay.
+__global__ __launch_bounds__(256) void trmv_lower_t_kernel(const double* __restrict__ X,
+                                                           int64_t ld,
+                                                           const double* __restrict__ t,
+                                                           int64_t n_pad,
+                                                           double* __restrict__ a) {
+  __shared__ double red[4][64];
+  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+  const int64_t j0 = (int64_t)blockIdx.x * 64, j = j0 + lane;
+  double s = 0.0;
+  for (int64_t i0 = j0 + 16 * wv; i0 < n_pad; i0 += 64) {
+    double x[16];
+#pragma unroll
+    for (int u = 0; u < 16; ++u) x[u] = X[(i0 + u) * ld + j];
+#pragma unroll
+    for (int u = 0; u < 16; ++u) s = fma(i0 + u >= j ? x[u] : 0.0, t[i0 + u], s);
+  }
+  red[wv][lane] = s;
+  __syncthreads();
+  if (wv == 0) a[j] = (red[0][lane] + red[1][lane]) + (red[2][lane] + red[3][lane]);
+}
+
+struct LsArg {
+  double v[32];
+};
+
+// Column means of X and xs = (X - mean) / l (zero rows up to n_pad), one workgroup per
+// column, the length scales as a kernel argument: one launch and no host copy where
+// scale_inputs takes two launches after a copy.  The sums are col_mean_kernel's.
+__global__ __launch_bounds__(256) void mean_scale_kernel(const double* __restrict__ X, int64_t n,
+                                                         int d, LsArg ls, double* __restrict__ xs,
+                                                         int64_t n_pad) {
+  const int j = blockIdx.x;
+  __shared__ double red[4];
+  double s = 0.0;
+  for (int64_t i = threadIdx.x; i < n; i += 256) s += X[i * d + j];
+  s = wave_sum(s);
+  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = s;
+  __syncthreads();
+  const double mean = (red[0] + red[1] + red[2] + red[3]) / (double)n;
+  double l = 1.0;
+#pragma unroll
+  for (int k = 0; k < 32; ++k) l = k == j ? ls.v[k] : l;
+  for (int64_t i = threadIdx.x; i < n_pad; i += 256)
+    xs[i * d + j] = i < n ? (X[i * d + j] - mean) / l : 0.0;
+}
 
 template <int MD>
 static void launch_trace(int kind, const TraceArgs& ta, int W, hipStream_t st) {
@@ -452,7 +647,11 @@ static int enqueue_mll(const MllWs& w, int kind, int64_t n, int d, double s, dou
   hipLaunchKernelGGL(trmv_lower_kernel, dim3((unsigned)((np + 3) / 4)), dim3(256), 0, st, Linv,
                      np, y, c, n, np, t, L, lgd);
   BTA_LAUNCH_CHECK("trmv_lower_kernel");
-  {
+  if (w.small) {
+    hipLaunchKernelGGL(trmv_lower_t_kernel, dim3((unsigned)(np / 64)), dim3(256), 0, st, Linv, np,
+                       t, np, alpha);
+    BTA_LAUNCH_CHECK("trmv_lower_t_kernel");
+  } else {
     const unsigned gx = (unsigned)std::min<int64_t>((np + 255) / 256, 16);
     hipLaunchKernelGGL(trmv_lower_t_part_kernel, dim3(gx, (unsigned)(np / 64)), dim3(256), 0, st,
                        Linv, np, t, np, part);
@@ -473,19 +672,32 @@ static int enqueue_mll(const MllWs& w, int kind, int64_t n, int d, double s, dou
   ta.MT = (int)(np / TR_B);
   ta.CB = TR_KC / TR_B;
   ta.s = s;
-  const int tasks = trace_tasks(ta.MT, ta.CB);
-  const int W = std::min(w.W, tasks);
-  rc = trace_schedule(ta.MT, ta.CB, (int)np, W, &ta.sched);
-  if (rc) return rc;
-  if (d <= 16)
-    launch_trace<16>(kind, ta, W, st);
-  else
-    launch_trace<32>(kind, ta, W, st);
+  int W = w.W;
+  if (w.small) {
+    ta.sched = nullptr;
+    if (w.MD == 8)
+      launch_trace_small<8>(kind, ta, W, st);
+    else if (w.MD == 16)
+      launch_trace_small<16>(kind, ta, W, st);
+    else
+      launch_trace_small<32>(kind, ta, W, st);
+  } else {
+    W = std::min(W, trace_tasks(ta.MT, ta.CB));
+    rc = trace_schedule(ta.MT, ta.CB, (int)np, W, &ta.sched);
+    if (rc) return rc;
+    if (d <= 16)
+      launch_trace<16>(kind, ta, W, st);
+    else
+      launch_trace<32>(kind, ta, W, st);
+  }
   BTA_LAUNCH_CHECK("mll_trace_kernel");
   // the factorisation's status pair goes next to the sums (read back with them)
   const int* stat = potrf_status(fact, np);
   int* stat_out = (int*)(out + 3 + w.MD + 2);
-  if (w.MD == 16)
+  if (w.MD == 8)
+    hipLaunchKernelGGL(mll_finish_kernel<10>, dim3(1), dim3(256), 0, st, t, lgd, alpha, n, partial,
+                       W, out, stat, stat_out);
+  else if (w.MD == 16)
     hipLaunchKernelGGL(mll_finish_kernel<18>, dim3(1), dim3(256), 0, st, t, lgd, alpha, n, partial,
                        W, out, stat, stat_out);
   else
@@ -509,25 +721,19 @@ int mll_value_grad(int kind, const double* X, const double* y, int64_t n, int d,
     return BTA_ERR_WORKSPACE;
   }
   char* base = (char*)ws;
-  double* ls = (double*)(base + w.ls);
-  double* center = (double*)(base + w.center);
   double* xs = (double*)(base + w.xs);
   void* fact = base + w.fact;
   const size_t fact_bytes = std::max(potrf_ws_bytes(w.n_pad), trtri_ws_bytes(w.n_pad));
   double* out = (double*)(base + w.out);
   const int64_t np = w.n_pad;
 
-  // small host copies go through this thread's pinned buffer when there is one:
-  // [0, 32) the length scales, [64, 64 + MD + 6) the sums read back
+  // the sums are read back through this thread's pinned buffer when there is one
   double* pin = pinned_host_buffer();
-  if (pin) {
-    std::memcpy(pin, ls_host, d * sizeof(double));
-    BTA_HIP(hipMemcpyAsync(ls, pin, d * sizeof(double), hipMemcpyHostToDevice, st));
-  } else {
-    BTA_HIP(hipMemcpyAsync(ls, ls_host, d * sizeof(double), hipMemcpyHostToDevice, st));
-  }
-  int rc = scale_inputs(X, n, d, nullptr, ls, center, xs, np, st);
-  if (rc) return rc;
+  LsArg ls;
+  for (int j = 0; j < 32; ++j) ls.v[j] = j < d ? ls_host[j] : 1.0;
+  hipLaunchKernelGGL(mean_scale_kernel, dim3((unsigned)d), dim3(256), 0, st, X, n, d, ls, xs, np);
+  BTA_LAUNCH_CHECK("mean_scale_kernel");
+  int rc;
   // psd_safe_cholesky's schedule: no jitter, then jitter0 * 10^(i-1); K is
   // rebuilt for each attempt instead of being saved.  The whole call is
   // enqueued before the factorisation's outcome is known (one host
@@ -540,7 +746,7 @@ int mll_value_grad(int kind, const double* X, const double* y, int64_t n, int d,
     const double jit = attempt == 0 ? 0.0 : jitter0 * std::pow(10.0, (double)(attempt - 1));
     rc = enqueue_mll(w, kind, n, d, s, noise + jit, y, c, st, base, fact, fact_bytes);
     if (rc) return rc;
-    double* hb = pin ? pin + 64 : h.data();
+    double* hb = pin ? pin : h.data();
     BTA_HIP(hipMemcpyAsync(hb, out, h.size() * sizeof(double), hipMemcpyDeviceToHost, st));
     BTA_HIP(hipStreamSynchronize(st));
     if (pin) std::memcpy(h.data(), hb, h.size() * sizeof(double));
