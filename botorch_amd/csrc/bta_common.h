@@ -172,34 +172,110 @@ __device__ __forceinline__ double kern_grad_factor_k(double r2, double s) {
   return s * exp_nonpos(-0.5 * r2);
 }
 
-__device__ __forceinline__ double wave_sum(double v) {
-#pragma unroll
-  for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
-  return v;
+// v of lane (this lane ^ OFF), OFF = 1, 2, 4 or 8, by DPP moves within rows of 16
+// lanes (every lane of the row active): no LDS traffic, where a shuffle is two
+// ds_bpermute and their wait.
+template <int CTRL>
+__device__ __forceinline__ double dpp_d(double v) {
+  const int2 p = __builtin_bit_cast(int2, v);
+  int2 r;
+  r.x = __builtin_amdgcn_update_dpp(0, p.x, CTRL, 0xF, 0xF, false);
+  r.y = __builtin_amdgcn_update_dpp(0, p.y, CTRL, 0xF, 0xF, false);
+  return __builtin_bit_cast(double, r);
+}
+template <int OFF>
+__device__ __forceinline__ double row_xor(double v) {
+  static_assert(OFF == 1 || OFF == 2 || OFF == 4 || OFF == 8, "within a row of 16");
+  if constexpr (OFF == 1) return dpp_d<0xB1>(v);                // quad_perm [1, 0, 3, 2]
+  else if constexpr (OFF == 2) return dpp_d<0x4E>(v);           // quad_perm [2, 3, 0, 1]
+  else if constexpr (OFF == 4) return dpp_d<0x1B>(dpp_d<0x141>(v));  // i -> 7 - i -> i ^ 4
+  else return dpp_d<0x128>(v);                                  // row_ror:8
 }
 
-// NV independent wave sums with the shuffles of each butterfly step issued
-// together: one cross-lane latency per step instead of one per value and step.
-// Each value is summed in the same order as wave_sum.
+// Exchanges the upper 32 lanes (OFF = 32) or the odd rows of 16 (OFF = 16) of a with
+// the lower ones (the even rows) of b; all 64 lanes active.
+template <int OFF>
+__device__ __forceinline__ void lane_swap(double& a, double& b) {
+  static_assert(OFF == 16 || OFF == 32, "half waves or rows");
+#ifdef __HIP_DEVICE_COMPILE__
+  uint2 x = __builtin_bit_cast(uint2, a), y = __builtin_bit_cast(uint2, b);
+  if constexpr (OFF == 32) {
+    const auto lo = __builtin_amdgcn_permlane32_swap(x.x, y.x, false, false);
+    const auto hi = __builtin_amdgcn_permlane32_swap(x.y, y.y, false, false);
+    x.x = lo[0], y.x = lo[1], x.y = hi[0], y.y = hi[1];
+  } else {
+    const auto lo = __builtin_amdgcn_permlane16_swap(x.x, y.x, false, false);
+    const auto hi = __builtin_amdgcn_permlane16_swap(x.y, y.y, false, false);
+    x.x = lo[0], y.x = lo[1], x.y = hi[0], y.y = hi[1];
+  }
+  a = __builtin_bit_cast(double, x);
+  b = __builtin_bit_cast(double, y);
+#endif
+}
+
+// op over the 64 lanes in the order of a butterfly of steps 32, 16, .., 1 (every lane
+// gets the result).  The two first steps are one swap and one operation each: a step's
+// two operands are the halves of the swapped copies.
+template <typename OP>
+__device__ __forceinline__ double wave_reduce(double v, OP op) {
+  double w = v;
+  lane_swap<32>(v, w);
+  v = w = op(v, w);
+  lane_swap<16>(v, w);
+  v = op(v, w);
+  v = op(v, row_xor<8>(v));
+  v = op(v, row_xor<4>(v));
+  v = op(v, row_xor<2>(v));
+  return op(v, row_xor<1>(v));
+}
+__device__ __forceinline__ double wave_sum(double v) {
+  return wave_reduce(v, [](double a, double b) { return a + b; });
+}
+__device__ __forceinline__ double wave_max(double v) {
+  return wave_reduce(v, [](double a, double b) { return fmax(a, b); });
+}
+__device__ __forceinline__ double wave_min(double v) {
+  return wave_reduce(v, [](double a, double b) { return fmin(a, b); });
+}
+
+// NV independent wave sums, each in the order of wave_sum.
 template <int NV>
 __device__ __forceinline__ void wave_sum_n(double (&v)[NV]) {
 #pragma unroll
-  for (int off = 32; off > 0; off >>= 1) {
-    double t[NV];
-#pragma unroll
-    for (int i = 0; i < NV; ++i) t[i] = __shfl_xor(v[i], off, 64);
-#pragma unroll
-    for (int i = 0; i < NV; ++i) v[i] += t[i];
-  }
+  for (int i = 0; i < NV; ++i) v[i] = wave_sum(v[i]);
 }
 
-// NV <= 32 wave sums with P - 1 + (6 - log2 P) shuffles instead of 6 NV
+// NV <= 32 wave sums with P - 1 + (6 - log2 P) exchanges instead of 6 NV
 // (P = NV rounded up to a power of two): the first log2 P butterfly steps
 // halve the values each lane carries (the lane with the step's bit set keeps
 // the upper half, its partner the lower), the remaining steps are ordinary
 // butterflies.  The total of value e ends in lanes e * 64/P .. (e + 1) * 64/P - 1;
 // the first of them gets *e_out = e, every other lane -1 (also lanes past NV).
 // Every value is summed over the same tree as wave_sum: bit-identical totals.
+template <int OFF, int H, int P>
+__device__ __forceinline__ void spread_step(double (&a)[P], int lane) {
+  if constexpr (OFF >= 16) {  // a swap leaves both operands of every lane's sum
+#pragma unroll
+    for (int i = 0; i < H; ++i) {
+      lane_swap<OFF>(a[i], a[H + i]);
+      a[i] += a[H + i];
+    }
+  } else {
+    const bool up = (lane & OFF) != 0;
+#pragma unroll
+    for (int i = 0; i < H; ++i) {
+      // The empty asm (no instruction) makes lo and hi opaque values: without
+      // it the compiler turns the lane-dependent choice below into a select of
+      // the element index and extracts a[index] through compare/select chains
+      // over the whole array (about 7x the instructions at NV = 10).
+      double lo = a[i], hi = a[H + i];
+      __asm__("" : "+v"(lo), "+v"(hi));
+      const double keep = up ? hi : lo;
+      const double send = up ? lo : hi;
+      a[i] = keep + row_xor<OFF>(send);
+    }
+  }
+}
 template <int NV>
 __device__ __forceinline__ double wave_sum_spread(const double (&v)[NV], int* e_out) {
   static_assert(NV >= 1 && NV <= 32, "wave_sum_spread: 1..32 values");
@@ -209,35 +285,29 @@ __device__ __forceinline__ double wave_sum_spread(const double (&v)[NV], int* e_
   double a[P];
 #pragma unroll
   for (int i = 0; i < P; ++i) a[i] = i < NV ? v[i] : 0.0;
-#pragma unroll
-  for (int s = 0; s < LG; ++s) {
-    const int h = P >> (s + 1), off = 32 >> s;
-    const bool up = (lane & off) != 0;
-#pragma unroll
-    for (int i = 0; i < h; ++i) {
-      // The empty asm (no instruction) makes lo and hi opaque values: without
-      // it the compiler turns the lane-dependent choice below into a select of
-      // the element index and extracts a[index] through compare/select chains
-      // over the whole array (about 7x the instructions at NV = 10).
-      double lo = a[i], hi = a[h + i];
-      __asm__("" : "+v"(lo), "+v"(hi));
-      const double keep = up ? hi : lo;
-      const double send = up ? lo : hi;
-      a[i] = keep + __shfl_xor(send, off, 64);
-    }
-  }
+  if constexpr (LG >= 1) spread_step<32, (P >> 1)>(a, lane);
+  if constexpr (LG >= 2) spread_step<16, (P >> 2)>(a, lane);
+  if constexpr (LG >= 3) spread_step<8, (P >> 3)>(a, lane);
+  if constexpr (LG >= 4) spread_step<4, (P >> 4)>(a, lane);
+  if constexpr (LG >= 5) spread_step<2, (P >> 5)>(a, lane);
   double t = a[0];
-#pragma unroll
-  for (int off = 32 >> LG; off > 0; off >>= 1) t += __shfl_xor(t, off, 64);
+  if constexpr (LG == 0) {
+    double w = t;
+    lane_swap<32>(t, w);
+    t += w;
+  }
+  if constexpr (LG <= 1) {
+    double w = t;
+    lane_swap<16>(t, w);
+    t += w;
+  }
+  if constexpr (LG <= 2) t += row_xor<8>(t);
+  if constexpr (LG <= 3) t += row_xor<4>(t);
+  if constexpr (LG <= 4) t += row_xor<2>(t);
+  t += row_xor<1>(t);
   const int e = lane >> (6 - LG);
   *e_out = ((lane & ((64 >> LG) - 1)) == 0 && e < NV) ? e : -1;
   return t;
-}
-
-__device__ __forceinline__ double wave_max(double v) {
-#pragma unroll
-  for (int off = 32; off > 0; off >>= 1) v = fmax(v, __shfl_xor(v, off, 64));
-  return v;
 }
 
 }  // namespace bta

@@ -33,18 +33,9 @@ constexpr int64_t LB_MAX_LDS = 64 * 1024;
 struct WaveLanes {
   static constexpr int W = LB_LANES;
   __device__ int lane() const { return (int)threadIdx.x; }
-  __device__ double sum(double v) const {
-    for (int o = W / 2; o > 0; o >>= 1) v += __shfl_xor(v, o, W);
-    return v;
-  }
-  __device__ double max(double v) const {
-    for (int o = W / 2; o > 0; o >>= 1) v = fmax(v, __shfl_xor(v, o, W));
-    return v;
-  }
-  __device__ double min(double v) const {
-    for (int o = W / 2; o > 0; o >>= 1) v = fmin(v, __shfl_xor(v, o, W));
-    return v;
-  }
+  __device__ double sum(double v) const { return wave_sum(v); }
+  __device__ double max(double v) const { return wave_max(v); }
+  __device__ double min(double v) const { return wave_min(v); }
   __device__ int sum_int(int v) const {
     for (int o = W / 2; o > 0; o >>= 1) v += __shfl_xor(v, o, W);
     return v;

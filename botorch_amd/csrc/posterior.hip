@@ -162,8 +162,10 @@ __device__ __forceinline__ double post_mean16(const PostOutArgs& a, int64_t p) {
   const double* q = a.part + p * nt;
   double v = 0.0;
   for (int t = threadIdx.x & 15; t < nt; t += 16) v += q[t];
-#pragma unroll
-  for (int off = 8; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
+  v += row_xor<8>(v);
+  v += row_xor<4>(v);
+  v += row_xor<2>(v);
+  v += row_xor<1>(v);
   return a.y_mean + a.y_std * (a.c + v);
 }
 
@@ -605,8 +607,10 @@ __global__ __launch_bounds__(256) void post_grad_finish_kernel(PostGradArgs a,
   for (int j = 0; j < PC_MAXD; ++j) {
     if (j >= d) break;
     double v = acc[j];
-#pragma unroll
-    for (int off = 8; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
+    v += row_xor<8>(v);
+    v += row_xor<4>(v);
+    v += row_xor<2>(v);
+    v += row_xor<1>(v);
     if (sub == (j & 15)) {
       for (int sp = 0; sp < a.splits; ++sp) v += a.part[((int64_t)sp * R + row) * d + j];
       dX[row * d + j] = v / ls[j];

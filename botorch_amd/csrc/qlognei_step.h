@@ -105,36 +105,202 @@ __device__ __forceinline__ TM div_tm(TM a, TM b) {
 
 // log(tau * (softplus(x/tau) + 0.1 / (1 + (x/tau)^2))) and its derivative
 // (utils/safe_math.py:298-325), evaluated in TM (FP64, or FP32 for the mixed
-// modes' sample arithmetic) from the FP64 difference x; rtau = 1 / tau.  In
-// FP32, log1p(e) follows Goldberg's rule log(u) e / (u - 1), u = 1 + e (a few
+// modes' sample arithmetic) from the FP64 difference x; rtau = 1 / tau.
+//
+// In FP32, log1p(e) follows Goldberg's rule log(u) e / (u - 1), u = 1 + e (a few
 // ulp; "What every computer scientist should know about floating-point
 // arithmetic", 1991, thm. 4), and the divisions use div_tm.
+//
+// In FP64 log1p(e) = log u + (e - (u - 1)) / u, whose correction is at most an ulp of
+// u, so the hardware reciprocal is enough for it; logs, exponentials and quotients
+// are those of bta_common.h, without the general forms' branches for operands that
+// cannot occur (z^2 and its products are held below 1e300 so that every divisor and
+// its reciprocal stay normal).  With the library's forms and exact divisions the
+// samples of one candidate took 9400 cycles of a 49900-cycle workgroup, now 7200 of 32000.
 template <typename TM>
 __device__ __forceinline__ void log_fatplus_grad(double x, double tau, double rtau, double* v,
                                                  double* dv) {
   constexpr bool f32 = sizeof(TM) == 4;
-  const TM z = f32 ? (TM)(x * rtau) : (TM)(x / tau);
+  const TM z = (TM)(x * rtau);
   TM sp, sig;
-  if (z > (TM)20) {  // torch softplus threshold
-    sp = z;
-    sig = (TM)1;
+  if constexpr (f32) {
+    if (z > (TM)20) {  // torch softplus threshold
+      sp = z;
+      sig = (TM)1;
+    } else {
+      const TM e = exp(z);
+      const TM u = (TM)1 + e;
+      sp = u == (TM)1 ? e : log(u) * div_tm(e, u - (TM)1);
+      sig = div_tm(e, u);
+    }
+    const TM z2 = (TM)1 + z * z;
+    const TM cz = div_tm((TM)1, z2);
+    const TM f = sp + (TM)0.1 * cz;
+    const TM tt = (TM)tau;
+    *v = (double)log(tt * f);
+    // dv = (sig - 0.2 z cz^2) / (f tau), with cz / f = 1 / (sp (1 + z^2) + 0.1) so
+    // that no intermediate underflows for large |z|
+    const TM cf = sp > (TM)0 ? div_tm((TM)1, sp * z2 + (TM)0.1) : (TM)10;
+    const TM g = div_tm(sig, f) - (TM)0.2 * z * cz * cf;
+    *dv = (double)(g * (TM)rtau);
   } else {
-    const TM e = exp(z);
-    const TM u = (TM)1 + e;
-    if constexpr (f32) sp = u == (TM)1 ? e : log(u) * div_tm(e, u - (TM)1);
-    else sp = log1p(e);
-    sig = div_tm(e, u);
+    const bool lin = z > 20.0;
+    const double e = exp_nonpos(lin ? 0.0 : z);  // (its reduction holds up to e^20)
+    const double u = 1.0 + e;
+    const double l1p = fma(e - (u - 1.0), __builtin_amdgcn_rcp(u), log_pos(u));
+    sp = lin ? z : l1p;
+    sig = lin ? 1.0 : div_normal(e, u);
+    double z2 = fma(z, z, 1.0);
+    z2 = z2 > 1e300 ? 1e300 : z2;
+    const double cz = div_normal(1.0, z2);
+    const double f = fma(0.1, cz, sp);
+    *v = log_pos(tau * f);
+    double t = fma(sp, z2, 0.1);
+    t = t > 1e300 ? 1e300 : t;
+    const double cf = div_normal(1.0, t);
+    const double g = div_normal(sig, f) - 0.2 * z * cz * cf;
+    *dv = g * rtau;
   }
-  const TM z2 = (TM)1 + z * z;
-  const TM cz = div_tm((TM)1, z2);
-  const TM f = sp + (TM)0.1 * cz;
-  const TM tt = (TM)tau;
-  *v = (double)log(tt * f);
-  // dv = (sig - 0.2 z cz^2) / (f tau), with cz / f = 1 / (sp (1 + z^2) + 0.1) so
-  // that no intermediate underflows for large |z|
-  const TM cf = sp > (TM)0 ? div_tm((TM)1, sp * z2 + (TM)0.1) : (TM)10;
-  const TM g = div_tm(sig, f) - (TM)0.2 * z * cz * cf;
-  *dv = (double)(f32 ? g * (TM)rtau : g / tt);
+}
+
+// x / l with r = 1 / l (correctly rounded), equal to the division: q is within two
+// ulps after the product, faithful after the first residual correction and correctly
+// rounded after the second (Markstein, "Computation of elementary functions on the IBM
+// RISC System/6000 processor", 1990).  An infinite x stays infinite.
+__device__ __forceinline__ double div_by(double x, double l, double r) {
+  const double q0 = x * r;
+  const double q1 = fma(fma(-q0, l, x), r, q0);
+  const double q2 = fma(fma(-q1, l, x), r, q1);
+  return fabs(q0) < INFINITY ? q2 : q0;
+}
+
+// v of lane l of the wave (l uniform)
+__device__ __forceinline__ double lane_bcast(double v, int l) {
+  const int2 p = __builtin_bit_cast(int2, v);
+  int2 r;
+  r.x = __builtin_amdgcn_readlane(p.x, l);
+  r.y = __builtin_amdgcn_readlane(p.y, l);
+  return __builtin_bit_cast(double, r);
+}
+
+// Triangular solves with the baseline factor L (n_b x n_b, row-major) for the Q rows of
+// x (pitch px): x <- x L^-T (forward) or out <- x L^-1 (back), the subtractions of an
+// element in column order.  Columns are eliminated one after the other, so the chain
+// per column counts: a quotient by the reciprocal of the diagonal (div_by), a broadcast
+// by DPP or readlane and one product.  Coefficients outside the triangle are zero, so a
+// finished element stays as it is, still to be divided at the end: no lane masks on the
+// chain.  (With an exact division, a shuffle and an LDS read per column a solve of 8
+// columns took 8100 cycles, now 2600.)  EXACT: quotients equal to the division's; else
+// (the FP64 mode) x times the reciprocal, six operations fewer on the chain.
+//
+// Up to 16 columns: four rows per wave, lane 16 r + j holding column j of row r and its
+// coefficients in registers.
+template <bool EXACT>
+__device__ __forceinline__ double solve_quot(double x, double ld, double rd) {
+  return EXACT ? div_by(x, ld, rd) : x * rd;
+}
+template <int U, bool EXACT>
+__device__ __forceinline__ void solve16_step(double& x, const double (&c)[16], double ld,
+                                             double rd) {
+  // (0x150 + U: row_newbcast, lane U of each row of 16)
+  x = fma(-c[U], dpp_d<0x150 | U>(solve_quot<EXACT>(x, ld, rd)), x);
+}
+template <int G, bool BACK, bool EXACT>
+__device__ __forceinline__ void solve16_four(double& x, const double (&c)[16], double ld,
+                                             double rd) {
+  solve16_step<4 * G + (BACK ? 3 : 0), EXACT>(x, c, ld, rd);
+  solve16_step<4 * G + (BACK ? 2 : 1), EXACT>(x, c, ld, rd);
+  solve16_step<4 * G + (BACK ? 1 : 2), EXACT>(x, c, ld, rd);
+  solve16_step<4 * G + (BACK ? 0 : 3), EXACT>(x, c, ld, rd);
+}
+template <int Q, bool BACK, bool EXACT>
+__device__ __forceinline__ void solve16(const double* L, int n_b, const double* x, int px,
+                                        double* out, int po, int wv, int wpr) {
+  const int lane = threadIdx.x & 63, j = min(lane & 15, n_b - 1);
+  const double ld = L[j * n_b + j], rd = 1.0 / ld;
+  double c[16];
+#pragma unroll
+  for (int u = 0; u < 16; ++u) {
+    const int k = min(u, n_b - 1);
+    const double l = BACK ? L[k * n_b + j] : L[j * n_b + k];
+    c[u] = (BACK ? j < u && u < n_b : j > u) ? l : 0.0;
+  }
+  for (int i0 = 4 * wv; i0 < Q; i0 += 4 * wpr) {  // (uniform over the wave)
+    const int i = min(i0 + (lane >> 4), Q - 1);
+    double v = x[i * px + j];
+    if constexpr (BACK) {
+      if (n_b > 12) solve16_four<3, true, EXACT>(v, c, ld, rd);
+      if (n_b > 8) solve16_four<2, true, EXACT>(v, c, ld, rd);
+      if (n_b > 4) solve16_four<1, true, EXACT>(v, c, ld, rd);
+      solve16_four<0, true, EXACT>(v, c, ld, rd);
+    } else {
+      solve16_four<0, false, EXACT>(v, c, ld, rd);
+      if (n_b > 4) solve16_four<1, false, EXACT>(v, c, ld, rd);
+      if (n_b > 8) solve16_four<2, false, EXACT>(v, c, ld, rd);
+      if (n_b > 12) solve16_four<3, false, EXACT>(v, c, ld, rd);
+    }
+    v = solve_quot<EXACT>(v, ld, rd);
+    if ((lane & 15) < n_b && i0 + (lane >> 4) < Q) out[i * po + j] = v;
+  }
+}
+// Any n_b (up to 256): one wave per row, lane l holding columns l + 64 t; 16 columns
+// are eliminated within their slot, then taken off the other slots.  (Lanes past n_b
+// repeat the last column and store nothing.)
+template <int Q, bool BACK, bool EXACT>
+__device__ __forceinline__ void solve_any(const double* L, int n_b, const double* x, int px,
+                                          double* out, int po, int wv, int wpr) {
+  constexpr int NS = MC_MAXNB_SLOTS;
+  const int lane = threadIdx.x & 63;
+  const int nc = (n_b + 15) / 16;
+  for (int i = wv; i < Q; i += wpr) {
+    double v[NS], ld[NS], rd[NS];
+#pragma unroll
+    for (int t = 0; t < NS; ++t) {
+      const int j = min(lane + 64 * t, n_b - 1);
+      v[t] = x[i * px + j];
+      ld[t] = L[j * n_b + j];
+    }
+#pragma unroll
+    for (int t = 0; t < NS; ++t) rd[t] = 1.0 / ld[t];
+    for (int ci = 0; ci < nc; ++ci) {
+      const int k0 = 16 * (BACK ? nc - 1 - ci : ci), ks = k0 >> 6;
+      double y[16];
+#pragma unroll
+      for (int t0 = 0; t0 < NS; ++t0) {
+        // the chunk's own slot first, then the others that still depend on it
+        const int t = BACK ? NS - 1 - t0 : t0;
+        if ((BACK ? t > ks : t < ks) || 64 * t >= n_b) continue;
+        const int j = lane + 64 * t, jc = min(j, n_b - 1);
+        double c[16];
+#pragma unroll
+        for (int u = 0; u < 16; ++u) {
+          const int k = k0 + u, kc = min(k, n_b - 1);
+          const double l = BACK ? L[kc * n_b + jc] : L[jc * n_b + kc];
+          c[u] = (BACK ? j < k && k < n_b : j > k) ? l : 0.0;
+        }
+        if (t == ks) {
+#pragma unroll
+          for (int u0 = 0; u0 < 16; ++u0) {
+            const int u = BACK ? 15 - u0 : u0;
+            y[u] = lane_bcast(solve_quot<EXACT>(v[t], ld[t], rd[t]), (k0 + u) & 63);
+            v[t] = fma(-c[u], y[u], v[t]);
+          }
+        } else {
+#pragma unroll
+          for (int u0 = 0; u0 < 16; ++u0) {
+            const int u = BACK ? 15 - u0 : u0;
+            v[t] = fma(-c[u], y[u], v[t]);
+          }
+        }
+      }
+    }
+#pragma unroll
+    for (int t = 0; t < NS; ++t) {
+      const int j = lane + 64 * t;
+      const double q = solve_quot<EXACT>(v[t], ld[t], rd[t]);
+      if (j < n_b) out[i * po + j] = q;
+    }
+  }
 }
 
 // Reductions over the WPR waves of one restart (wave w of the restart writes
@@ -180,30 +346,41 @@ __device__ __forceinline__ double group_max1(double v, double* red, int wv) {
   return r;
 }
 
+// |a - b|^2, eight coordinates loaded at a time
 __device__ __forceinline__ double sq_dist(const double* a, const double* b, int d) {
   double r2 = 0.0;
-  for (int j = 0; j < d; ++j) {
-    double df = a[j] - b[j];
-    r2 = fma(df, df, r2);
+  for (int j0 = 0; j0 < d; j0 += 8) {
+    double x[8], y[8];
+#pragma unroll
+    for (int u = 0; u < 8; ++u) {
+      const int j = min(j0 + u, d - 1);
+      x[u] = a[j];
+      y[u] = b[j];
+    }
+#pragma unroll
+    for (int u = 0; u < 8; ++u) {
+      const double df = x[u] - y[u];
+      if (j0 + u < d) r2 = fma(df, df, r2);
+    }
   }
   return r2;
 }
 
-// In-register Cholesky of a Q x Q SPD matrix (row-major, lower result).
+// Cholesky of a Q x Q matrix by one wave, lane i holding row i (lanes past Q repeat the
+// last): ar its row of the matrix, l its row of the factor (entries right of the
+// diagonal are not meaningful).  False at a pivot that is not positive.
 template <int Q>
-__device__ bool small_chol(const double* A, double jit, double* L) {
-  for (int i = 0; i < Q * Q; ++i) L[i] = 0.0;
+__device__ __forceinline__ bool small_chol(const double (&ar)[Q], double jit, int i,
+                                           double (&l)[Q]) {
+#pragma unroll
   for (int j = 0; j < Q; ++j) {
-    double s = A[j * Q + j] + jit;
-    for (int k = 0; k < j; ++k) s -= L[j * Q + k] * L[j * Q + k];
+    double t = i == j ? ar[j] + jit : ar[j];
+#pragma unroll
+    for (int k = 0; k < j; ++k) t = fma(-l[k], lane_bcast(l[k], j), t);
+    const double s = lane_bcast(t, j);
     if (!(s > 0.0)) return false;
     const double dj = sqrt(s), rdj = 1.0 / dj;
-    L[j * Q + j] = dj;
-    for (int i = j + 1; i < Q; ++i) {
-      double t = A[i * Q + j];
-      for (int k = 0; k < j; ++k) t -= L[i * Q + k] * L[j * Q + k];
-      L[i * Q + j] = t * rdj;
-    }
+    l[j] = i == j ? dj : t * rdj;
   }
   return true;
 }
@@ -296,21 +473,25 @@ __device__ __forceinline__ void mc_body(const McArgs& a, const int bw, double* s
   constexpr int NQ = Q * (Q + 1) / 2;
   double* pv = sm + lay.pv;  // Q x (n_b + 1): P[r0 + i][j]
   double* vv = sm + lay.vv;  // packed lower triangle of V_b V_b^T
+  constexpr bool ZPRE = Q <= 4;  // (the registers of more rows are taken)
+  double zpre[2][8], bpre[2];
   {
-    // 4 NR tasks per wave per pass (16 per restart), their loads issued
-    // together; each task's sum is the same whatever the batch
-    constexpr int TB = 4 * NR;
+    // 16 tasks per wave per pass, their loads issued together; each task's sum is
+    // the same whatever the batch
+    constexpr int TB = 16;
     const int ne = n_b + 1;
     for (int t0 = wv * TB; t0 < Q * ne; t0 += TB * WPR) {
       double s[TB];
 #pragma unroll
-      for (int u = 0; u < TB; ++u) {
-        const int t = t0 + u;
-        s[u] = 0.0;
-        if (t < Q * ne) {
-          const double* p = a.P + ((r0 + t / ne) * ne + t % ne) * a.p_parts;
-          for (int pt = lane; pt < a.p_parts; pt += 64) s[u] += p[pt];
-        }
+      for (int u = 0; u < TB; ++u) s[u] = 0.0;
+      const double* p = a.P + (r0 * ne + t0) * a.p_parts;
+      const int last = Q * ne - 1 - t0;
+      for (int pt = lane; pt < a.p_parts; pt += 64) {
+        double x[TB];
+#pragma unroll
+        for (int u = 0; u < TB; ++u) x[u] = p[(int64_t)min(u, last) * a.p_parts + pt];
+#pragma unroll
+        for (int u = 0; u < TB; ++u) s[u] += x[u];
       }
       int e;
       const double tot = wave_sum_spread<TB>(s, &e);
@@ -340,6 +521,19 @@ __device__ __forceinline__ void mc_body(const McArgs& a, const int bw, double* s
 #pragma unroll
       for (int i = 0; i < Q; ++i) v[i] = *(const vec_t*)(vt + (r0 + i) * a.ldv + k);
       vv_pass(v);
+    }
+    // the first eight base samples of this thread's first two samples, for the sample
+    // stage: they arrive during the reductions and the solves
+    if (ZPRE) {
+      const int s0 = min(tid, S - 1), s1 = tid + TPR < S ? tid + TPR : s0;
+      bpre[0] = a.best_f[s0];
+      bpre[1] = a.best_f[s1];
+#pragma unroll
+      for (int u = 0; u < 8; ++u) {
+        const int64_t k = min(u, m - 1);
+        zpre[0][u] = a.Zt[k * S + s0];
+        zpre[1][u] = a.Zt[k * S + s1];
+      }
     }
     double tot[NQ];
     group_sum<NQ, WPR>(acc, red, tot, wv);
@@ -382,57 +576,36 @@ __device__ __forceinline__ void mc_body(const McArgs& a, const int bw, double* s
         __syncthreads();
       }
     }
-    // ---- Lbl = Sigma_qb Lb^-T: forward substitution, one wave per row ----
-    auto lbl_rows = [&](const double* L) {
-      for (int i = wv; i < Q; i += WPR) {
-        double rhs[MC_MAXNB_SLOTS];
-#pragma unroll
-        for (int t2 = 0; t2 < MC_MAXNB_SLOTS; ++t2) {
-          const int j = lane + 64 * t2;
-          rhs[t2] = j < n_b ? lnew[i * m + j] : 0.0;
-        }
-        for (int kb = 0; kb < n_b; ++kb) {
-          const int slot = kb >> 6, owner = kb & 63;
-          double mine = 0.0;
-#pragma unroll
-          for (int t2 = 0; t2 < MC_MAXNB_SLOTS; ++t2)
-            if (t2 == slot) mine = rhs[t2];
-          const double y = __shfl(mine, owner, 64) / L[kb * n_b + kb];
-#pragma unroll
-          for (int t2 = 0; t2 < MC_MAXNB_SLOTS; ++t2) {
-            const int j = lane + 64 * t2;
-            if (j == kb) rhs[t2] = y;
-            else if (j > kb && j < n_b) rhs[t2] -= L[j * n_b + kb] * y;
-          }
-        }
-#pragma unroll
-        for (int t2 = 0; t2 < MC_MAXNB_SLOTS; ++t2) {
-          const int j = lane + 64 * t2;
-          if (j < n_b) lnew[i * m + j] = rhs[t2];
-        }
-      }
-    };
-    if (lb_lds) lbl_rows(lbs);
-    else lbl_rows(Lb);
+    // ---- Lbl = Sigma_qb Lb^-T: forward substitution ---------------------
+    if (lb_lds) solve16<Q, false, sizeof(TV) == 4>(lbs, n_b, lnew, m, lnew, m, wv, WPR);
+    else solve_any<Q, false, sizeof(TV) == 4>(Lb, n_b, lnew, m, lnew, m, wv, WPR);
     __syncthreads();
 
     // ---- Schur complement and its Cholesky --------------------------------
     if (tid < Q * Q) {
       const int i = tid / Q, j = tid % Q;
       double s = 0.0;
+#pragma unroll 4
       for (int kb = 0; kb < n_b; ++kb) s = fma(lnew[i * m + kb], lnew[j * m + kb], s);
       gA[i * Q + j] = sqq[i * Q + j] - s;  // gA used as scratch for the Schur block
     }
     __syncthreads();
-    if (tid == 0) {
+    if (wv == 0) {
       int st = 0;
       bool ok = false;
-      bool has_nan = false;
-      for (int i = 0; i < Q * Q; ++i) has_nan |= (gA[i] != gA[i]);
+      const int i = min(lane, Q - 1);
+      double ar[Q], l[Q];
+      bool mine = false;
+#pragma unroll
+      for (int j = 0; j < Q; ++j) {
+        ar[j] = gA[i * Q + j];
+        mine |= ar[j] != ar[j];
+      }
+      const bool has_nan = __ballot(mine) != 0;
       const int first = joint ? t : 0, last = joint ? t : a.max_tries;
       for (int attempt = first; attempt <= last && !has_nan; ++attempt) {
         const double jit = attempt == 0 ? 0.0 : a.jitter * pow(10.0, (double)(attempt - 1));
-        ok = small_chol<Q>(gA, jit, lbr);
+        ok = small_chol<Q>(ar, jit, i, l);
         if (ok) {
           if (attempt > 0) st |= BTA_STATUS_JITTER;
           break;
@@ -440,9 +613,10 @@ __device__ __forceinline__ void mc_body(const McArgs& a, const int bw, double* s
       }
       if (has_nan) st |= BTA_STATUS_NAN;
       else if (!ok) st |= BTA_STATUS_NOT_PSD;
-      if (!ok)
-        for (int i = 0; i < Q * Q; ++i) lbr[i] = NAN;
-      scal[0] = (double)st;
+      if (lane < Q)
+#pragma unroll
+        for (int j = 0; j < Q; ++j) lbr[i * Q + j] = !ok ? NAN : j <= i ? l[j] : 0.0;
+      if (lane == 0) scal[0] = (double)st;
     }
     __syncthreads();
     st_bits = (int)scal[0];
@@ -477,25 +651,46 @@ __device__ __forceinline__ void mc_body(const McArgs& a, const int bw, double* s
       log_fatplus_grad<TM>(y[i] - bf, tr, rtr, &v[i], &dv[i]);
       M = fmax(M, v[i]);
     }
-    TM P = 0, sdp = 0, dp[Q];
-    int nties = 0;
+    if constexpr (sizeof(TM) == 4) {
+      TM P = 0, sdp = 0, dp[Q];
+      int nties = 0;
 #pragma unroll
-    for (int i = 0; i < Q; ++i) {
-      const TM z = sizeof(TM) == 4 ? (TM)((M - v[i]) * rtm) : (TM)((M - v[i]) / tm);
-      const TM den = (TM)2 + (TM)2 * z + z * z;
-      P += div_tm((TM)2, den);
-      dp[i] = div_tm((TM)-2 * ((TM)2 + (TM)2 * z), den * den);
-      sdp += dp[i];
-      nties += (v[i] == M);
-    }
-    const double u = M + tm * (double)log(P);
-    uu[s] = u;
-    lmax = fmax(lmax, u);
-    const TM cm = div_tm((TM)1 + div_tm(sdp, P), (TM)nties);
+      for (int i = 0; i < Q; ++i) {
+        const TM z = (TM)((M - v[i]) * rtm);
+        const TM den = (TM)2 + (TM)2 * z + z * z;
+        P += div_tm((TM)2, den);
+        dp[i] = div_tm((TM)-2 * ((TM)2 + (TM)2 * z), den * den);
+        sdp += dp[i];
+        nties += (v[i] == M);
+      }
+      const double u = M + tm * (double)log(P);
+      uu[s] = u;
+      lmax = fmax(lmax, u);
+      const TM cm = div_tm((TM)1 + div_tm(sdp, P), (TM)nties);
 #pragma unroll
-    for (int i = 0; i < Q; ++i) {
-      const TM du = (v[i] == M ? cm : (TM)0) - div_tm(dp[i], P);
-      G[s * Q + i] = (double)du * dv[i];
+      for (int i = 0; i < Q; ++i) {
+        const TM du = (v[i] == M ? cm : (TM)0) - div_tm(dp[i], P);
+        G[i * S + s] = (double)du * dv[i];
+      }
+    } else {
+      double P = 0.0, sdp = 0.0, dp[Q], nties = 0.0;
+#pragma unroll
+      for (int i = 0; i < Q; ++i) {
+        const double z = (M - v[i]) * rtm;
+        const double rden = div_normal(1.0, fma(z, z, fma(2.0, z, 2.0)));
+        P = fma(2.0, rden, P);
+        dp[i] = -4.0 * (1.0 + z) * rden * rden;
+        sdp += dp[i];
+        nties += v[i] == M ? 1.0 : 0.0;
+      }
+      const double u = M + tm * log_pos(P);
+      uu[s] = u;
+      lmax = fmax(lmax, u);
+      const double rP = div_normal(1.0, P);
+      const double cm = div_normal(fma(sdp, rP, 1.0), nties);
+#pragma unroll
+      for (int i = 0; i < Q; ++i)
+        G[i * S + s] = ((v[i] == M ? cm : 0.0) - dp[i] * rP) * dv[i];
     }
   };
   // Each thread carries the samples s0 and s0 + TPR through the products: the
@@ -505,17 +700,37 @@ __device__ __forceinline__ void mc_body(const McArgs& a, const int bw, double* s
   for (int s0 = tid; s0 < S; s0 += 2 * TPR) {
     const bool two = s0 + TPR < S;
     const int s1 = two ? s0 + TPR : s0;
-    const double bf0 = a.best_f[s0], bf1 = a.best_f[s1];
+    const bool pre = ZPRE && s0 == tid;
+    double bf0, bf1;
+    if (pre) {
+      bf0 = bpre[0];
+      bf1 = bpre[1];
+    } else {
+      bf0 = a.best_f[s0];
+      bf1 = a.best_f[s1];
+    }
     double y0[Q], y1[Q];
 #pragma unroll
     for (int i = 0; i < Q; ++i) y0[i] = y1[i] = mu[i];
     for (int k0 = 0; k0 < m; k0 += 8) {
       double lc[Q][8], z0[8], z1[8];
+      if (pre && k0 == 0) {
+#pragma unroll
+        for (int u = 0; u < 8; ++u) {
+          z0[u] = zpre[0][u];
+          z1[u] = zpre[1][u];
+        }
+      } else {
+#pragma unroll
+        for (int u = 0; u < 8; ++u) {
+          const int64_t k = k0 + u < m ? k0 + u : m - 1;
+          z0[u] = a.Zt[k * S + s0];
+          z1[u] = a.Zt[k * S + s1];
+        }
+      }
 #pragma unroll
       for (int u = 0; u < 8; ++u) {
         const int k = k0 + u < m ? k0 + u : m - 1;
-        z0[u] = a.Zt[(int64_t)k * S + s0];
-        z1[u] = a.Zt[(int64_t)k * S + s1];
 #pragma unroll
         for (int i = 0; i < Q; ++i) lc[i][u] = lnew[i * m + k];
       }
@@ -528,8 +743,15 @@ __device__ __forceinline__ void mc_body(const McArgs& a, const int bw, double* s
             y1[i] = fma(lc[i][u], z1[u], y1[i]);
           }
     }
-    sample_tail(s0, bf0, y0);
-    if (two) sample_tail(s0 + TPR, bf1, y1);
+    // one or two candidates leave room between the dependent operations of a sample:
+    // its partner's go there (a thread without one repeats its own)
+    if (sizeof(TM) == 8 && Q <= 2 && __any(two)) {
+      sample_tail(s0, bf0, y0);
+      sample_tail(s1, bf1, y1);
+    } else {
+      sample_tail(s0, bf0, y0);
+      if (two) sample_tail(s1, bf1, y1);
+    }
   }
   if (bad) scal[1] = 1.0;  // every writer stores the same value
 
@@ -538,23 +760,32 @@ __device__ __forceinline__ void mc_body(const McArgs& a, const int bw, double* s
   const double Mu = group_max1<WPR>(lmax, red, wv);
   double lsum[1] = {0.0};
   for (int s = tid; s < S; s += TPR) {  // uu keeps exp(u - max) for the adjoint
-    const double e = exp(uu[s] - Mu);
+    const double e = sizeof(TM) == 4 ? exp(uu[s] - Mu) : exp_nonpos(uu[s] - Mu);
     uu[s] = e;
     lsum[0] += e;
   }
   double tsum[1];
   group_sum<1, WPR>(lsum, red, tsum, wv);
-  if (tid == 0 && live) {
-    a.value[b] = Mu + log(tsum[0]) - log((double)S);
-    int st = (int)scal[0];
-    if (scal[1] != 0.0) st |= BTA_STATUS_NAN;
-    a.status[b] = st;
+  auto write_value = [&]() {
+    if (tid == TPR - 1 && live) {
+      a.value[b] = Mu + log(tsum[0]) - log((double)S);
+      int st = (int)scal[0];
+      if (scal[1] != 0.0) st |= BTA_STATUS_NAN;
+      a.status[b] = st;
+    }
+  };
+  if (!a.grad) {
+    write_value();
+    return;
   }
-  if (!a.grad) return;
 
   // ---- dmu, d[Lbl | Lbr] = (w G)^T Z with the logmeanexp weights w --------
-  constexpr int MREG = 32 / Q - 1;  // per-thread accumulators while m <= MREG
-  if (m <= MREG) {
+  // per-thread accumulators while m <= MREG (FP32 samples; in FP64 the registers they
+  // take cost more than the second pass over G)
+  constexpr bool f32 = sizeof(TM) == 4;
+  constexpr int MREG = 32 / Q - 1;
+  if (f32 && m <= MREG) {
+    if constexpr (f32) {
     constexpr int NV = Q * (MREG + 1);
     double acc[NV];
 #pragma unroll
@@ -564,7 +795,7 @@ __device__ __forceinline__ void mc_body(const McArgs& a, const int bw, double* s
       double gw[Q];
 #pragma unroll
       for (int i = 0; i < Q; ++i) {
-        gw[i] = G[s * Q + i] * w;
+        gw[i] = G[i * S + s] * w;
         acc[i * (MREG + 1) + MREG] += gw[i];
       }
 #pragma unroll
@@ -607,67 +838,97 @@ __device__ __forceinline__ void mc_body(const McArgs& a, const int bw, double* s
       else dlnew[i * m + k] = k < n_b + i + 1 ? tot : 0.0;
     }
     __syncthreads();
+    }
   } else {
   for (int s = tid; s < S; s += TPR) {
     const double w = uu[s] / tsum[0];
 #pragma unroll
-    for (int i = 0; i < Q; ++i) G[s * Q + i] *= w;
+    for (int i = 0; i < Q; ++i) G[i * S + s] *= w;
   }
   __syncthreads();
 
-  // one wave per (i, k) for wide baselines
-  for (int task = wv; task < Q * (m + 1); task += WPR) {
-    const int i = task / (m + 1), k = task % (m + 1);
-    if (k < m && k >= n_b + i + 1) {  // upper part of Lbr: no dependence
-      if (lane == 0) dlnew[i * m + k] = 0.0;
-      continue;
+  // wide baselines: wave w sums the columns w, w + WPR, .. (four at a time, with all
+  // rows i: the base samples are read once and the wave sums share their exchanges);
+  // column m, the means, takes base samples of 1
+  for (int k0 = wv; k0 <= m; k0 += 4 * WPR) {
+    double acc[4 * Q];
+#pragma unroll
+    for (int e = 0; e < 4 * Q; ++e) acc[e] = 0.0;
+#pragma unroll 4
+    for (int s = lane; s < S; s += 64) {
+      double z[4];
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        const int k = k0 + u * WPR;
+        z[u] = a.Zt[(int64_t)min(k, m - 1) * S + s];
+        z[u] = k < m ? z[u] : 1.0;
+      }
+#pragma unroll
+      for (int i = 0; i < Q; ++i) {
+        const double gi = G[i * S + s];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) acc[u * Q + i] = fma(gi, z[u], acc[u * Q + i]);
+      }
     }
-    double acc = 0.0;
-    if (k == m) {
-      for (int s = lane; s < S; s += 64) acc += G[s * Q + i];
-    } else {
-      const double* zr = a.Zt + (int64_t)k * S;
-      for (int s = lane; s < S; s += 64) acc = fma(G[s * Q + i], zr[s], acc);
-    }
-    acc = wave_sum(acc);
-    if (lane == 0) {
-      if (k == m) dmu[i] = acc;
-      else dlnew[i * m + k] = acc;
+    int e;
+    const double tot = wave_sum_spread<4 * Q>(acc, &e);
+    const int i = e % Q, k = k0 + e / Q * WPR;
+    if (e >= 0 && k <= m) {
+      if (k == m) dmu[i] = tot;
+      else dlnew[i * m + k] = k < n_b + i + 1 ? tot : 0.0;  // (upper part of Lbr: none)
     }
   }
   __syncthreads();
   }
 
   // ---- Cholesky backward of Lbr (torch's formula), gA symmetric ----------
-  if (tid == 0) {
-    double T[Q * Q], Mm[Q * Q], Y[Q * Q];
-    for (int i = 0; i < Q; ++i)
-      for (int j = 0; j < Q; ++j) {
-        double t = 0.0;
-        if (j <= i)
-          for (int k = 0; k < Q; ++k) t += lbr[k * Q + i] * dlnew[k * m + n_b + j];
-        T[i * Q + j] = t;  // tril(L^T dL)
+  // by the restart's first wave: lane (i, j) forms an entry of tril(L^T dL), lane j a
+  // column of Y, lane r a row of gA; T and Y pass through red.  (Where a rounded
+  // product is added rather than fused, it is the rounding the one-lane form had.)
+  if (wv == 0) {
+    double* Ts = red;
+    double* Ys = red + 64;
+    const int e = min(lane, Q * Q - 1), ti = e / Q, tj = e % Q, c = min(lane, Q - 1);
+    double t = 0.0;
+#pragma unroll
+    for (int k = 0; k < Q; ++k) t = fma(lbr[k * Q + ti], dlnew[k * m + n_b + tj], t);
+    Ts[e] = tj <= ti ? t : 0.0;
+    const double rc = 1.0 / lbr[c * Q + c];
+    double rd[Q], y[Q];
+#pragma unroll
+    for (int i = 0; i < Q; ++i) rd[i] = lane_bcast(rc, i);
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    // Y = L^-T Mm, Mm = the symmetric half of T: back substitution per column
+#pragma unroll
+    for (int i = Q - 1; i >= 0; --i) {
+      double s = 0.5 * (i >= c ? Ts[i * Q + c] : Ts[c * Q + i]);
+#pragma unroll
+      for (int k = i + 1; k < Q; ++k) {
+        const double p = -lbr[k * Q + i];
+        s = k == i + 1 && i == c ? s + fma(p, y[k], 0.0) : fma(p, y[k], s);
       }
-    for (int i = 0; i < Q; ++i)
-      for (int j = 0; j < Q; ++j)
-        Mm[i * Q + j] = 0.5 * (i >= j ? T[i * Q + j] : T[j * Q + i]);
-    // reciprocal diagonal once: the two solves below multiply by it
-    double rd[Q];
-    for (int i = 0; i < Q; ++i) rd[i] = 1.0 / lbr[i * Q + i];
-    // Y = L^-T Mm : solve L^T Y = Mm (upper, back substitution per column)
-    for (int j = 0; j < Q; ++j)
-      for (int i = Q - 1; i >= 0; --i) {
-        double s = Mm[i * Q + j];
-        for (int k = i + 1; k < Q; ++k) s -= lbr[k * Q + i] * Y[k * Q + j];
-        Y[i * Q + j] = s * rd[i];
+      y[i] = i ? s * rd[i] : s;  // row 0 is scaled where it is used
+    }
+#pragma unroll
+    for (int i = 0; i < Q; ++i) Ys[i * Q + c] = y[i];
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    // gA = Y L^-1: x L = y for each row
+#pragma unroll
+    for (int j = Q - 1; j >= 0; --j) {
+      double s = Ys[c * Q + j];
+      if (j + 1 < Q) {
+        const double l = lbr[(j + 1) * Q + j];
+        s = c == 0 ? fma(s, rd[0], fma(-y[j + 1], l, 0.0)) : fma(-y[j + 1], l, s);
+      } else {
+        s = c == 0 ? s * rd[0] : s;
       }
-    // gA = Y L^-1 : solve gA L = Y, i.e. for each row r: x L = y
-    for (int r = 0; r < Q; ++r)
-      for (int j = Q - 1; j >= 0; --j) {
-        double s = Y[r * Q + j];
-        for (int k = j + 1; k < Q; ++k) s -= gA[r * Q + k] * lbr[k * Q + j];
-        gA[r * Q + j] = s * rd[j];
-      }
+#pragma unroll
+      for (int k = j + 2; k < Q; ++k) s = fma(-y[k], lbr[k * Q + j], s);
+      y[j] = s * rd[j];
+    }
+    if (lane < Q)
+#pragma unroll
+      for (int j = 0; j < Q; ++j) gA[c * Q + j] = y[j];
   }
   __syncthreads();
   // dLbl -= 2 gA Lbl  (Schur = Sigma_qq - Lbl Lbl^T)
@@ -679,41 +940,13 @@ __device__ __forceinline__ void mc_body(const McArgs& a, const int bw, double* s
     dlnew[i * m + kb] -= 2.0 * s;
   }
   __syncthreads();
-  // ---- dSigma_qb = dLbl Lb^-1 : back substitution, one wave per row -------
-  auto dsqb_rows = [&](const double* L) {
-    for (int i = wv; i < Q; i += WPR) {
-      double rhs[MC_MAXNB_SLOTS];
-#pragma unroll
-      for (int t = 0; t < MC_MAXNB_SLOTS; ++t) {
-        const int j = lane + 64 * t;
-        rhs[t] = j < n_b ? dlnew[i * m + j] : 0.0;
-      }
-      for (int kb = n_b - 1; kb >= 0; --kb) {
-        const int slot = kb >> 6, owner = kb & 63;
-        double mine = 0.0;
-#pragma unroll
-        for (int t = 0; t < MC_MAXNB_SLOTS; ++t)
-          if (t == slot) mine = rhs[t];
-        const double zz = __shfl(mine, owner, 64) / L[kb * n_b + kb];
-#pragma unroll
-        for (int t = 0; t < MC_MAXNB_SLOTS; ++t) {
-          const int j = lane + 64 * t;
-          if (j == kb) rhs[t] = zz;
-          else if (j < kb) rhs[t] -= L[kb * n_b + j] * zz;
-        }
-      }
-#pragma unroll
-      for (int t = 0; t < MC_MAXNB_SLOTS; ++t) {
-        const int j = lane + 64 * t;
-        if (j < n_b) dsqb[i * n_b + j] = rhs[t];
-      }
-    }
-  };
-  if (lb_lds) dsqb_rows(lbs);
-  else dsqb_rows(Lb);
+  // ---- dSigma_qb = dLbl Lb^-1: back substitution ---------------------------
+  if (lb_lds) solve16<Q, true, sizeof(TV) == 4>(lbs, n_b, dlnew, m, dsqb, n_b, wv, WPR);
+  else solve_any<Q, true, sizeof(TV) == 4>(Lb, n_b, dlnew, m, dsqb, n_b, wv, WPR);
   __syncthreads();
 
   // ---- dV = gq V with gq = -2 s^2 gA: the q x q block for the gradient stage
+  write_value();  // (here, where no barrier waits for its logarithms)
   if (!live) return;
   for (int e = tid; e < Q * Q; e += TPR) a.gq[r0 * Q + e] = -2.0 * ys2 * gA[e];
   for (int e = tid; e < Q * (n_b + 1); e += TPR) {
@@ -728,6 +961,7 @@ __device__ __forceinline__ void mc_body(const McArgs& a, const int bw, double* s
     double acc = 0.0;
     for (int i2 = 0; i2 < Q; ++i2)
       acc -= 2.0 * ys2 * gA[i * Q + i2] * hh[i * m + i2] * (xij - xq[i2 * MC_MAXD + j]);
+#pragma unroll 4
     for (int kb = 0; kb < n_b; ++kb)
       acc -= ys2 * dsqb[i * n_b + kb] * hh[i * m + Q + kb] * (xij - a.bs[kb * d + j]);
     a.dxs_extra[(r0 + i) * d + j] = acc;
