@@ -14,8 +14,9 @@
 //   post_covar_kernel      xs, K_x and the 64-column partials of K_x alpha
 //   post_cov_small_kernel  mq <= POST_SMALL_MQ: V V^T on MFMA for 16 consecutive
 //                          rows, k(xs, xs), and all the outputs
-//   post_cov_joint_kernel  above: lower 128 x 64 tiles of V V^T, the same
-//                          epilogue, the upper triangle mirrored
+//   post_cov_tiles_kernel, post_cov_joint_kernel  above: lower 32 x 32 or 128 x 64
+//                          tiles of V V^T, the same epilogue, the upper triangle
+//                          mirrored
 // Adjoint: U = V L^-1 = K_x K^-1 (with xs and V kept from the moments' call, or K_x
 // and V formed again: 120 of 520 us at 256 x 4 points and n = 2048), then
 //   post_grad_kernel       g_rc = y_std dmean_r alpha_c - sum_j S_rj U_jc with
@@ -28,6 +29,7 @@
 #include "gemm.h"
 #include "gemm_d.h"
 #include "gemm_tile.h"
+#include "gemm_w_body.h"
 #include "kernels.h"
 
 #include <algorithm>
@@ -302,6 +304,83 @@ __global__ __launch_bounds__(256, 2) void post_cov_joint_kernel(PostOutArgs a) {
     }
 }
 
+// The same from 32 x 32 lower tiles (gemm_w_body.h), for outputs of too few 128 x 64
+// tiles to fill the chip: at mq = 1500, n = 1000 those are 156 tiles of which each
+// runs 2048 matrix products a wave, 101 us; the 1176 small ones take 66 us.  Both
+// halves are written in rows of 256 bytes from the tile in LDS.
+template <int KIND>
+__global__ __launch_bounds__(256, 2) void post_cov_tiles_kernel(PostOutArgs a) {
+  constexpr int T = 32;
+  __shared__ __attribute__((aligned(1024))) unsigned char lds[w_lds<2, 2, 4, 16, 2>()];
+  static_assert(4 * T * T * 8 + 2 * T * (PC_MAXD + 1) * 8 <= w_lds<2, 2, 4, 16, 2>(),
+                "the coordinates follow the partial tiles");
+  const int mq = a.rows.mq, mp = a.rows.mq_pad, d = a.d;
+  const int64_t bi = blockIdx.y;
+  const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6, l16 = lane & 15, gq = lane >> 4;
+  int ti, tj;
+  decode_tile((int)blockIdx.x, BTA_GEMM_C_LOWER, mp / T, mp / T, ti, tj);
+  const double* V = a.V + bi * mp * a.n_pad;
+  const double* xs = a.xs + bi * mp * d;
+  // the tile's row and column points, on their way during the products
+  double xv[2 * T * PC_MAXD / 256];
+#pragma unroll
+  for (int u = 0; u < 2 * T * PC_MAXD / 256; ++u) {
+    const int e = tid + 256 * u;
+    xv[u] = 0.0;
+    if (e < 2 * T * d) {
+      const int r = e / d, p = r < T ? ti * T + r : tj * T + r - T;
+      if (p < mq) xv[u] = xs[(int64_t)p * d + e % d];
+    }
+  }
+  w_partials<2, 2, 4, 16, 2, false>(V, a.n_pad, V, a.n_pad, ti * T, tj * T, 0, (int)a.n_pad, lds);
+  const double* red = (const double*)lds;
+  double* xr = (double*)lds + 4 * T * T;  // 64 x (PC_MAXD + 1), rows then columns
+#pragma unroll
+  for (int u = 0; u < 2 * T * PC_MAXD / 256; ++u) {
+    const int e = tid + 256 * u;
+    if (e < 2 * T * d) xr[e / d * (PC_MAXD + 1) + e % d] = xv[u];
+  }
+  // wave wv finishes fragment (wv / 2, wv % 2)
+  const int rl = 16 * (wv >> 1), cl = 16 * (wv & 1) + l16;
+  double o[4], r2[4] = {0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+  for (int q = 0; q < 4; ++q) o[q] = w_sum<2, 2, 4>(red, wv, q, lane);
+  __syncthreads();
+  for (int j = 0; j < d; ++j) {
+    const double c = xr[(T + cl) * (PC_MAXD + 1) + j];
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      const double df = xr[(rl + Mfma<double>::row(gq, q)) * (PC_MAXD + 1) + j] - c;
+      r2[q] = fma(df, df, r2[q]);
+    }
+  }
+  double* ot = (double*)lds;  // 32 x 33 (the partial tiles are read)
+  const double ys2 = a.y_std * a.y_std;
+#pragma unroll
+  for (int q = 0; q < 4; ++q)
+    ot[(rl + Mfma<double>::row(gq, q)) * (T + 1) + cl] =
+        ys2 * (kern_value_k<KIND>(r2[q], a.s) - o[q]);
+  __syncthreads();
+  for (int e = tid; e < T * T; e += 256) {
+    const int r = e / T, c = e % T;
+    const int row = ti * T + r, col = tj * T + c;
+    const double lo = ot[r * (T + 1) + c], up = ot[c * (T + 1) + r];
+    if (a.covar) {
+      if (row < mq && col < mq) a.covar[(bi * mq + row) * mq + col] = ti > tj || c <= r ? lo : up;
+      if (ti > tj && ti * T + c < mq)  // (tj's rows are all in use then)
+        a.covar[(bi * mq + tj * T + r) * mq + ti * T + c] = up;
+    }
+    if (a.var && row == col && row < mq) a.var[bi * mq + row] = lo;
+  }
+  if (a.mean && tj == 0)
+    for (int r = tid >> 4; r < T; r += 16) {
+      const int row = ti * T + r;
+      if (row >= mq) break;  // uniform over the 16 lanes of a row
+      const double mu = post_mean16(a, bi * mp + row);
+      if ((tid & 15) == 0) a.mean[bi * mq + row] = mu;
+    }
+}
+
 // Row layout of a call: mq_pad and the total of padded rows.
 struct PostLayout {
   int mq_pad;
@@ -424,9 +503,16 @@ int gp_posterior(const bta_gp_model* m, const double* X, int64_t batch, int mq, 
     hipLaunchKernelGGL(post_cov_small_kernel, dim3((unsigned)((batch * mq + per - 1) / per)),
                        dim3(256), 0, s, o);
   } else {
-    const int MT = (w.lay.mq_pad + D_BM - 1) / D_BM;
-    const dim3 g((unsigned)(MT * (MT + 1)), (unsigned)batch);
-    if (m->kind == BTA_KERNEL_MATERN52)
+    const int MT = (w.lay.mq_pad + D_BM - 1) / D_BM, TT = w.lay.mq_pad / 32;
+    const bool m52 = m->kind == BTA_KERNEL_MATERN52;
+    // small tiles below 1.5 large ones per CU, as for the products of gemm_w.hip
+    const bool small = 2 * (int64_t)MT * (MT + 1) * batch < 3 * (int64_t)num_cus();
+    const dim3 g((unsigned)(small ? TT * (TT + 1) / 2 : MT * (MT + 1)), (unsigned)batch);
+    if (small && m52)
+      hipLaunchKernelGGL((post_cov_tiles_kernel<BTA_KERNEL_MATERN52>), g, dim3(256), 0, s, o);
+    else if (small)
+      hipLaunchKernelGGL((post_cov_tiles_kernel<BTA_KERNEL_RBF>), g, dim3(256), 0, s, o);
+    else if (m52)
       hipLaunchKernelGGL((post_cov_joint_kernel<BTA_KERNEL_MATERN52>), g, dim3(256), 0, s, o);
     else
       hipLaunchKernelGGL((post_cov_joint_kernel<BTA_KERNEL_RBF>), g, dim3(256), 0, s, o);

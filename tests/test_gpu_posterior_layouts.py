@@ -133,3 +133,21 @@ def test_posterior_adjoint_kept_and_recomputed_agree(monkeypatch):
         model.likelihood.noise = noise
         monkeypatch.undo()
         assert torch.equal(*grads)
+
+
+@pytest.mark.parametrize("batch,mq", [(191, 17), (192, 17), (63, 97), (64, 97), (1, 1500)])
+def test_posterior_joint_tiles_both_sides_of_their_rule(batch, mq):
+    # 2 ceil(mq / 128) (ceil(mq / 128) + 1) batch against 3 x 256 CUs: 32 x 32 tiles of
+    # V V^T below, 128 x 64 above
+    print(f"[case] batch={batch} mq={mq}", flush=True)
+    gp, orc = _pair(70, 5, O.MATERN52)
+    X = torch.rand(batch, mq, 5, generator=torch.Generator().manual_seed(mq),
+                   dtype=torch.float64)
+    with torch.no_grad():
+        post = gp.posterior(X.to(DEV))
+        m_r, c_r = orc.posterior(X)
+    cov = post.covariance_matrix
+    assert (post.mean.squeeze(-1).cpu() - m_r).abs().max() < 1e-10 * m_r.abs().max()
+    assert (cov.cpu() - c_r).abs().max() < 1e-10 * c_r.abs().max()
+    assert torch.equal(cov, cov.transpose(-1, -2))
+    assert torch.equal(post.variance.squeeze(-1), cov.diagonal(dim1=-2, dim2=-1))
