@@ -21,6 +21,9 @@ int launch_gemm(const GemmArgs& g, int batch, hipStream_t s);
 // C = A op(B) for the R_pad x np matrices A and C and the triangular np x np B
 // (flags), of whose rows only the first R are used: rows of C past R rounded up to
 // 32 may stay unwritten.
+// gemm_rows_small: its arguments for the 32 x 32 tiles, and whether it takes them.
+bool gemm_rows_small(int flags, int64_t R, int64_t np, const void* A, const void* B, void* C,
+                     GemmArgs* out);
 int gemm_rows(int flags, int64_t R, int64_t R_pad, int64_t np, const void* A, const void* B,
               void* C, hipStream_t s);
 

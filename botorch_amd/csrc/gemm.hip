@@ -223,9 +223,10 @@ static int launch_cfg(const GemmArgs& g, int batch, int W, hipStream_t s) {
 
 // One triangular FP64 product with R rows in use of R_pad (a multiple of 64): the
 // small tiles need R rounded up to 32 only.
-int gemm_rows(int flags, int64_t R, int64_t R_pad, int64_t np, const void* A, const void* B,
-              void* C, hipStream_t s) {
-  GemmArgs g{};
+bool gemm_rows_small(int flags, int64_t R, int64_t np, const void* A, const void* B, void* C,
+                     GemmArgs* out) {
+  GemmArgs& g = *out;
+  g = GemmArgs{};
   g.A = A;
   g.B = B;
   g.C = C;
@@ -234,8 +235,13 @@ int gemm_rows(int flags, int64_t R, int64_t R_pad, int64_t np, const void* A, co
   g.N = g.K = (int)np;
   g.flags = flags;
   g.alpha = 1.0;
-  if (!(flags & BTA_GEMM_F32) && gemm_w_supported(g) && gemm_w_preferred(g.M, np, 1))
-    return gemm_w(g, 1, s);
+  return !(flags & BTA_GEMM_F32) && gemm_w_supported(g) && gemm_w_preferred(g.M, np, 1);
+}
+
+int gemm_rows(int flags, int64_t R, int64_t R_pad, int64_t np, const void* A, const void* B,
+              void* C, hipStream_t s) {
+  GemmArgs g;
+  if (gemm_rows_small(flags, R, np, A, B, C, &g)) return gemm_w(g, 1, s);
   g.M = (int)R_pad;
   return launch_gemm(g, 1, s);
 }

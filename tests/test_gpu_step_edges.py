@@ -46,3 +46,25 @@ def test_step_edges_match_oracle(n, d, q, n_b, b, S, kind):
     assert (gr.cpu() - g_ref).abs().max() <= 2e-5 * g_ref.abs().max()
     with torch.no_grad():
         assert torch.equal(acq(Xq.to(DEV)), v)  # value alone
+
+
+@pytest.mark.parametrize("n,q,b,S", [(64, 1, 32, 512), (130, 3, 11, 64), (1011, 3, 200, 256),
+                                     (200, 8, 40, 128), (64, 2, 3000, 64)])
+def test_fused_fp64_adjoint_matches_sequential(n, q, b, S, monkeypatch):
+    # the FP64 MC stage and U = V L^-1 in one launch against one after the other: the
+    # same arithmetic but for the number of partial sums per entry of U (4 or 8), so
+    # a few ulp of the largest gradient entry: 1e-12
+    print(f"[case] n={n} q={q} b={b} S={S}", flush=True)
+    g = torch.Generator().manual_seed(n)
+    X = torch.rand(n, 6, generator=g, dtype=torch.float64)
+    Y = torch.sin(3 * X).sum(-1, keepdim=True)
+    gp = B.SingleTaskGP(X.to(DEV), Y.to(DEV))
+    acq = B.qLogNoisyExpectedImprovement(gp, X[:9].to(DEV),
+                                         sampler=B.SobolQMCNormalSampler(torch.Size([S]), seed=0),
+                                         prune_baseline=False)
+    Xq = torch.rand(b, q, 6, generator=g, dtype=torch.float64).to(DEV)
+    v, gr = acq.value_and_grad(Xq)
+    monkeypatch.setenv("BTA_SEQUENTIAL_ADJOINT", "1")
+    v2, gr2 = acq.value_and_grad(Xq)
+    assert torch.equal(v, v2)
+    assert (gr - gr2).abs().max() <= 1e-12 * gr2.abs().max()
