@@ -197,9 +197,11 @@ static H2Plan h2_plan(const H2Args& g, bool acc64, bool shared = false) {
   H2Plan p;
   const int small = h2_tiles(g, H2Mid::TM, H2Mid::TN), wide = h2_tiles(g, H2Wide::TM, H2Wide::TN),
             large = h2_tiles(g, H2Large::TM, H2Large::TN);
-  if (!acc64 && 2 * large >= 3 * ncu && (!shared || g.N >= 6144))
+  // (the tiles 128 columns and wider read and write past an odd multiple of 64)
+  const bool n128 = g.N % 128 == 0;
+  if (!acc64 && n128 && 2 * large >= 3 * ncu && (!shared || g.N >= 6144))
     p = {H2Large::TN, large, 0, false};
-  else if (!acc64 && !shared && 4 * wide >= 7 * ncu)
+  else if (!acc64 && n128 && !shared && 4 * wide >= 7 * ncu)
     p = {H2Wide::TN, wide, 0, false};
   else if (!acc64 && !shared && small <= ncu)
     p = {64, h2_tiles(g, H2Small::TM, H2Small::TN), 0, false};
@@ -248,9 +250,9 @@ int gemm_h2_candidates(const H2Args& g, bool shared, int* out, int max) {
   }
   if (!acc64) {
     if (!shared) add(64, h2_tiles(g, H2Small::TM, H2Small::TN), 0);
-    if (!shared && h2_tiles(g, H2Wide::TM, H2Wide::TN) >= ncu)
+    if (!shared && g.N % 128 == 0 && h2_tiles(g, H2Wide::TM, H2Wide::TN) >= ncu)
       add(H2Wide::TN, h2_tiles(g, H2Wide::TM, H2Wide::TN), 0);
-    if (h2_tiles(g, H2Large::TM, H2Large::TN) >= ncu)
+    if (g.N % 128 == 0 && h2_tiles(g, H2Large::TM, H2Large::TN) >= ncu)
       add(H2Large::TN, h2_tiles(g, H2Large::TM, H2Large::TN), 0);
   }
   return k;

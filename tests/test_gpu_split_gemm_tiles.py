@@ -55,6 +55,25 @@ def test_tiles_agree_bit_for_bit(M, N):
     assert (big[0][:m].double() - ref).abs().max() < 2e-6 * ref.abs().max()
 
 
+@pytest.mark.parametrize("M,N", [(4096, 2112), (8192, 2240), (128, 64)])
+def test_odd_multiple_of_64_columns_stays_in_bounds(M, N):
+    # N = 64 modulo 128 belongs to the 64-column tiles: nothing past N is written (C's
+    # rows are followed by a guard row) and every entry agrees with the small product
+    print(f"[case] {M} x {N}", flush=True)
+    g = torch.Generator(device=DEV).manual_seed(M + N)
+    ah, al = _planes(torch.rand(M, N, generator=g, device=DEV))
+    bh, bl = _planes(torch.tril(torch.randn(N, N, generator=g, device=DEV) * 0.1))
+    C = torch.full((M + 1, N), 7.0, dtype=torch.float32, device=DEV)
+    _lib.check(_lib.lib().bta_gemm_f16x3(
+        _lib.GEMM_B_LOWER, M, N, N, 1.0, _lib.ptr(ah), _lib.ptr(al), N, None, 1.0, _lib.ptr(bh),
+        _lib.ptr(bl), N, 1.0, _lib.ptr(C), N, None, None, 1.0, 0, _lib.stream()), "gemm_f16x3")
+    assert (C[M] == 7.0).all()
+    m = min(M, 128)
+    small = _run(ah[M - m:].contiguous(), al[M - m:].contiguous(), bh, bl, m, N, N,
+                 _lib.GEMM_B_LOWER, False)[0]
+    assert torch.equal(C[M - m:M], small)
+
+
 def test_upper_tiles_agree_bit_for_bit():
     M, N = 4096, 4096
     g = torch.Generator(device=DEV).manual_seed(1)
