@@ -19,29 +19,41 @@ __device__ __forceinline__ v4d mfma64(double a, double b, v4d c) {
   return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
 }
 
-// training points of the tile and their squared norms
+// The 64 training points of a column tile, their coordinates from registers
+// (qs_load_t) and their squared norms, one copy of these per wave: no barrier between
+// writing and reading them.
 template <int KD>
 struct QsT {
   double tc[QS_CT][4 * KD + 1];
-  double tn2[QS_CT];
+  double tn2[4][QS_CT];
 };
 
 template <int KD>
-__device__ __forceinline__ void qs_stage_t(QsT<KD>& sm, const double* T, int64_t n, int d,
-                                           int64_t c0) {
+__device__ __forceinline__ void qs_load_t(double (&tv)[KD], const double* T, int n, int d,
+                                          int c0) {
   constexpr int MD = 4 * KD;
-  for (int e = threadIdx.x; e < QS_CT * MD; e += 256) {
-    const int c = e / MD, j = e % MD;
-    sm.tc[c][j] = (j < d && c0 + c < n) ? T[(c0 + c) * d + j] : 0.0;
-  }
-  __syncthreads();
-  if (threadIdx.x < QS_CT) {
-    double s = 0.0;
 #pragma unroll
-    for (int j = 0; j < MD; ++j) s = fma(sm.tc[threadIdx.x][j], sm.tc[threadIdx.x][j], s);
-    sm.tn2[threadIdx.x] = s;
+  for (int t = 0; t < KD; ++t) {
+    const int e = threadIdx.x + 256 * t, c = e / MD, j = e % MD;
+    tv[t] = (j < d && c0 + c < n) ? T[(int64_t)(c0 + c) * d + j] : 0.0;
   }
-  __syncthreads();
+}
+template <int KD>
+__device__ __forceinline__ void qs_store_t(QsT<KD>& sm, const double (&tv)[KD]) {
+#pragma unroll
+  for (int t = 0; t < KD; ++t) {
+    const int e = threadIdx.x + 256 * t;
+    sm.tc[e / (4 * KD)][e % (4 * KD)] = tv[t];
+  }
+}
+// after the barrier that follows qs_store_t
+template <int KD>
+__device__ __forceinline__ void qs_norms(QsT<KD>& sm) {
+  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+  double s = 0.0;
+#pragma unroll
+  for (int j = 0; j < 4 * KD; ++j) s = fma(sm.tc[lane][j], sm.tc[lane][j], s);
+  sm.tn2[wv][lane] = s;
 }
 
 // sum over the four 16-lane groups (same lane % 16)
@@ -69,19 +81,21 @@ __device__ __forceinline__ void qstep_covar_body(const QsCovarArgs& a, const int
   __shared__ QsKStage<TO> ks[MODE == 2 ? 2 : 1];
   const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
   const int l16 = lane & 15, g = lane >> 4;
-  const int d = a.d;
-  const int64_t c0 = (int64_t)ct * QS_CT, r0 = (int64_t)rt * QS_RT;
-  const int64_t r0w = r0 + wv * 16;
-  const int64_t rl = r0w + l16;  // this lane's row as B operand / D column
-  // Every global load of the block is issued before the staging barrier: the
-  // raw row coordinates and the first 16 columns of E (all of them for
-  // ne <= 16), so that their latency overlaps the staging of T.
-  double xr[KD], xc[KD], xl[KD];
+  const int d = a.d, ne = a.ne, n = (int)a.n, R = (int)a.R;  // (grid extents are 64 x smaller)
+  const int c0 = ct * QS_CT, r0 = rt * QS_RT;
+  const int r0w = r0 + wv * 16;
+  const int rl = r0w + l16;  // this lane's row as B operand / D column
+  // Every global load of the block is issued before the staging barrier: T, the
+  // raw row coordinates and the first 16 columns of E (all of them for ne <= 16).
+  double tv[KD], xr[KD], xc[KD], xl[KD];
+  qs_load_t<KD>(tv, a.T, n, d, c0);
+  const double* xrow = a.X + (int64_t)min(rl, R - 1) * d;
+  const double* E = a.E + (int64_t)c0 * ne + l16;
 #pragma unroll
   for (int s = 0; s < KD; ++s) {
     const int j = 4 * s + g;
-    const bool ok = j < d && rl < a.R;
-    xr[s] = ok ? a.X[rl * d + j] : 0.0;
+    const bool ok = j < d && rl < R;
+    xr[s] = ok ? xrow[j] : 0.0;
     xc[s] = ok ? a.center[j] : 0.0;
     xl[s] = ok ? a.ls[j] : 1.0;
   }
@@ -90,10 +104,12 @@ __device__ __forceinline__ void qstep_covar_body(const QsCovarArgs& a, const int
   for (int cb = 0; cb < 4; ++cb)
 #pragma unroll
     for (int q = 0; q < 4; ++q) {
-      const int64_t c = c0 + cb * 16 + g + 4 * q;
-      ev[cb][q] = (l16 < a.ne && c < a.n) ? a.E[c * a.ne + l16] : 0.0;
+      const int c = cb * 16 + g + 4 * q;
+      ev[cb][q] = (l16 < ne && c0 + c < n) ? E[c * ne] : 0.0;
     }
-  qs_stage_t<KD>(sm, a.T, a.n, d, c0);
+  qs_store_t<KD>(sm, tv);
+  __syncthreads();
+  qs_norms<KD>(sm);
 
   // scaled row coordinates: lane (g, l16) holds x[rl][4s + g]
   double xb[KD];
@@ -104,7 +120,7 @@ __device__ __forceinline__ void qstep_covar_body(const QsCovarArgs& a, const int
     const double v = (xr[s] - xc[s]) / xl[s];
     xb[s] = v;
     xn2 = fma(v, v, xn2);
-    if (ct == 0 && j < d) a.xs_out[rl * d + j] = v;
+    if (ct == 0 && j < d) a.xs_out[(int64_t)rl * d + j] = v;
   }
   xn2 = sum_groups(xn2);
 
@@ -118,9 +134,9 @@ __device__ __forceinline__ void qstep_covar_body(const QsCovarArgs& a, const int
 #pragma unroll
     for (int q = 0; q < 4; ++q) {
       const int cl = cb * 16 + g + 4 * q;
-      const double r2 = fmax(sm.tn2[cl] + xn2 - 2.0 * cr[q], 0.0);
+      const double r2 = fmax(sm.tn2[wv][cl] + xn2 - 2.0 * cr[q], 0.0);
       double k = kern_value_k<KIND>(r2, a.s);
-      k = (c0 + cl < a.n && rl < a.R) ? k : 0.0;
+      k = (c0 + cl < n && rl < R) ? k : 0.0;
       kv[cb][q] = k;
       if (MODE == 2) {
         // kscale is a power of two: scaling after the FP32 rounding is exact
@@ -138,46 +154,41 @@ __device__ __forceinline__ void qstep_covar_body(const QsCovarArgs& a, const int
   {
     constexpr int V = 16 / (int)sizeof(TO);  // elements per 16-byte chunk
     constexpr int CPR = QS_CT / V;           // chunks per row
-    for (int e = tid; e < QS_RT * CPR; e += 256) {
-      const int r = e / CPR, cc = (e % CPR) * V;
-      const int64_t o = (r0 + r) * a.ldk + c0 + cc;
+    const int64_t o0 = (int64_t)(r0 + tid / CPR) * a.ldk + c0 + tid % CPR * V;
+#pragma unroll
+    for (int e0 = 0; e0 < QS_RT * CPR; e0 += 256) {
+      const int r = (tid + e0) / CPR, cc = tid % CPR * V;
+      const int64_t o = o0 + e0 / CPR * a.ldk;
       *(int4*)((TO*)a.K + o) = *(const int4*)&ks[0].k[r][cc];
       if (MODE == 2) *(int4*)(a.Klo + o) = *(const int4*)&ks[MODE == 2 ? 1 : 0].k[r][cc];
     }
   }
   // Ppart[r][j][ct] = sum_c K[r][c] E[c][j] in chunks of 16 columns j
   const int64_t nct = a.n_pad / QS_CT;
-  for (int j0 = 0; j0 < a.ne; j0 += 16) {
+  for (int j0 = 0; j0 < ne; j0 += 16) {
     const int jj = j0 + l16;
     v4d p = {0.0, 0.0, 0.0, 0.0};
 #pragma unroll
     for (int cb = 0; cb < 4; ++cb)
 #pragma unroll
       for (int q = 0; q < 4; ++q) {
-        const int64_t c = c0 + cb * 16 + g + 4 * q;
+        const int c = cb * 16 + g + 4 * q;
         const double e =
-            j0 == 0 ? ev[cb][q] : ((jj < a.ne && c < a.n) ? a.E[c * a.ne + jj] : 0.0);
+            j0 == 0 ? ev[cb][q] : ((jj < ne && c0 + c < n) ? E[c * ne + j0] : 0.0);
         p = mfma64(kv[cb][q], e, p);
       }
     // D layout: lane (g, l16) reg q = P[r0w + g + 4q][jj]
+    double* pp = a.Ppart + ((int64_t)(r0w + g) * ne + jj) * nct + ct;
+    const int64_t step = 4 * (int64_t)ne * nct;
 #pragma unroll
-    for (int q = 0; q < 4; ++q) {
-      const int64_t r = r0w + g + 4 * q;
-      if (jj < a.ne && r < a.R) a.Ppart[(r * a.ne + jj) * nct + ct] = p[q];
-    }
+    for (int q = 0; q < 4; ++q)
+      if (jj < ne && r0w + g + 4 * q < R) pp[q * step] = p[q];
   }
 }
 
 // U rows that 16 rows of a wave can mix, in steps of 4: 28 rows at q = 7.
 constexpr int QS_KU = 7;
 constexpr int QS_E_LDS = 16;  // columns of E staged in LDS (the rest is read per block)
-
-template <int KD>
-struct QsGradT {
-  double tc[QS_CT][4 * KD + 1];
-  double tn2[4][QS_CT];  // one copy per wave: no barrier between writing and reading it
-  double e[QS_CT][QS_E_LDS + 1];
-};
 
 // One tile of the gradient stage (column tile ct, row tile rt); 256 threads.
 // A tile is ~80 matrix products a wave, so what it waits for shows: every load of the
@@ -188,9 +199,9 @@ struct QsGradT {
 template <int KD, typename TU, int KIND>
 __device__ __forceinline__ void qstep_grad_body(const QsGradArgs& a, const int ct,
                                                 const int rt) {
-  constexpr int MD = 4 * KD;
-  constexpr int NB = (MD + 1 + 15) / 16;  // 16-column blocks of [T | 1]
-  __shared__ QsGradT<KD> sm;
+  constexpr int NB = (4 * KD + 1 + 15) / 16;  // 16-column blocks of [T | 1]
+  __shared__ QsT<KD> sm;
+  __shared__ double es[QS_CT][QS_E_LDS + 1];
   const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
   const int l16 = lane & 15, g = lane >> 4;
   const int d = a.d, q = a.q, ne = a.ne;
@@ -207,11 +218,7 @@ __device__ __forceinline__ void qstep_grad_body(const QsGradArgs& a, const int c
 
   // ---- loads ----------------------------------------------------------------
   double tv[KD], ev[4];
-#pragma unroll
-  for (int t = 0; t < KD; ++t) {
-    const int e = tid + 256 * t, c = e / MD, j = e % MD;
-    tv[t] = (j < d && c0 + c < n) ? a.T[(int64_t)(c0 + c) * d + j] : 0.0;
-  }
+  qs_load_t<KD>(tv, a.T, n, d, c0);
   const int ec = tid >> 2;
 #pragma unroll
   for (int t = 0; t < 4; ++t) {
@@ -242,20 +249,11 @@ __device__ __forceinline__ void qstep_grad_body(const QsGradArgs& a, const int c
       if (rvalid && u >= rblk && u < rblk + q) mb[s] = a.gq[rc * q + (u - rblk)];
     }
   }
+  qs_store_t<KD>(sm, tv);
 #pragma unroll
-  for (int t = 0; t < KD; ++t) {
-    const int e = tid + 256 * t;
-    sm.tc[e / MD][e % MD] = tv[t];
-  }
-#pragma unroll
-  for (int t = 0; t < 4; ++t) sm.e[ec][4 * t + (tid & 3)] = ev[t];
+  for (int t = 0; t < 4; ++t) es[ec][4 * t + (tid & 3)] = ev[t];
   __syncthreads();
-  {
-    double s = 0.0;
-#pragma unroll
-    for (int j = 0; j < MD; ++j) s = fma(sm.tc[lane][j], sm.tc[lane][j], s);
-    sm.tn2[wv][lane] = s;
-  }
+  qs_norms<KD>(sm);
   double xn2 = 0.0;
 #pragma unroll
   for (int s = 0; s < KD; ++s) xn2 = fma(xb[s], xb[s], xn2);
@@ -274,7 +272,7 @@ __device__ __forceinline__ void qstep_grad_body(const QsGradArgs& a, const int c
     v4d ga = {0.0, 0.0, 0.0, 0.0};
 #pragma unroll
     for (int s = 0; s < 4; ++s)
-      if (4 * s < ne) ga = mfma64(sm.e[cb * 16 + l16][4 * s + g], db[s], ga);
+      if (4 * s < ne) ga = mfma64(es[cb * 16 + l16][4 * s + g], db[s], ga);
     for (int j0 = QS_E_LDS; j0 < ne; j0 += 4) {
       const int j = j0 + g;
       const double ea = (j < ne && ca < n) ? a.E[(int64_t)ca * ne + j] : 0.0;
