@@ -5,8 +5,9 @@
 // table of per-model launch arguments (built once by bta_qlognei_batch_prepare
 // with qlognei_step_args, copied into the caller's workspace):
 //   covariance tiles      block -> (model, column tile, row tile)
-//   V = K_x L^-T          persistent workers over one list of (model, tile) of
-//                         all models, longest K range first
+//   V = K_x L^-T          one list of (model, tile) of all models, longest K range
+//                         first: a workgroup per 128 x 128 tile, or persistent
+//                         workers over 128 x 64 tiles for small batches
 //   U = V L^-1 + MC       workers over the adjoint tile list, then one
 //                         workgroup per (model, restart) for the MC stage
 //   gradient tiles        as the covariance tiles
@@ -81,6 +82,15 @@ __global__ __launch_bounds__(256, 2) void gemm_h2_list_kernel(const H2Args* __re
   gemm_h2_list_body(tab, tiles, total, blockIdx.x, gridDim.x, lds);
 }
 
+// The 128 x 128 tiles (sixteen waves), a workgroup each.
+__global__ __launch_bounds__(64 * H2Wide::NW, H2Wide::NW / 4) void gemm_h2_list_wide_kernel(
+    const H2Args* __restrict__ tab, const int4* __restrict__ tiles) {
+  __shared__ __attribute__((aligned(1024))) unsigned char lds[H2Wide::STAGES * H2Wide::STAGE];
+  const int4 e = tiles[blockIdx.x];
+  const H2Args g = tab[e.x];
+  gemm_h2_tile(H2Wide(), g, e.y, e.z, lds);
+}
+
 // Workgroups [0, W): adjoint GEMM workers; [W, W + mc blocks): the MC stage,
 // one workgroup per (model, restart), or per (model, two restarts) for a model
 // whose McArgs::nr is 2, as in its one-model step.
@@ -109,28 +119,51 @@ struct BatchTiles {
   std::vector<int4> fwd, adj;
 };
 
-// K chunks of 32 of tile (tm, tn) of a 64-column split GEMM with a triangular
-// B (BTA_GEMM_B_LOWER: K range [0, 64 (tn + 1)); B_UPPER: [64 tn, K)).
-static int tile_chunks(const H2Args& g, int tn) {
+// K chunks of 32 of tile (tm, tn), tw columns wide, of a split GEMM with a
+// triangular B (BTA_GEMM_B_LOWER: K range [0, tw (tn + 1)); B_UPPER: [tw tn, K)).
+static int tile_chunks(const H2Args& g, int tn, int tw) {
   int kb = 0, ke = g.K;
-  if (g.flags & BTA_GEMM_B_LOWER) ke = std::min(ke, (tn + 1) * 64);
-  if (g.flags & BTA_GEMM_B_UPPER) kb = std::max(kb, tn * 64);
+  if (g.flags & BTA_GEMM_B_LOWER) ke = std::min(ke, (tn + 1) * tw);
+  if (g.flags & BTA_GEMM_B_UPPER) kb = std::max(kb, tn * tw);
   return ke > kb ? (ke - kb + 31) / 32 : 0;
 }
 
-// Appends every 128 x 64 tile of problem p.
-static void add_tiles(const H2Args& g, int p, std::vector<int4>& out) {
-  for (int tn = 0; tn < g.N / 64; ++tn)
+// Appends every 128 x tw tile of problem p.
+static void add_tiles(const H2Args& g, int p, int tw, std::vector<int4>& out) {
+  for (int tn = 0; tn < g.N / tw; ++tn)
     for (int tm = 0; tm < g.M / H2_BM; ++tm) out.push_back(make_int4(p, tm, tn, 0));
 }
 
 // Longest K range first (ties: problem, then column, then row tile), so that
-// h2_tile_of pairs heavy with light tiles across the whole batch.
-static void order_tiles(const std::vector<H2Args>& tab, std::vector<int4>& t) {
+// h2_tile_of pairs heavy with light tiles across the whole batch; then the row
+// tiles of one (problem, column), which share their panel of B, are dealt to
+// positions of one residue modulo 8.  Worker p runs on XCD p % 8 and h2_tile_of
+// keeps or mirrors that residue (the worker counts are multiples of 8), so the
+// panel is read into one L2 instead of as many as there are row tiles.  32 models of
+// 128 to 4096 points, 512 rows: the adjoint list (128 x 64 tiles) takes 379 us in plain
+// order, 363 so.
+static void order_tiles(const std::vector<H2Args>& tab, int tw, std::vector<int4>& t) {
   std::stable_sort(t.begin(), t.end(), [&](const int4& a, const int4& b) {
-    const int ca = tile_chunks(tab[a.x], a.z), cb = tile_chunks(tab[b.x], b.z);
+    const int ca = tile_chunks(tab[a.x], a.z, tw), cb = tile_chunks(tab[b.x], b.z, tw);
     return ca > cb;
   });
+  constexpr int NX = 8;
+  std::vector<int4> cls[NX];
+  for (size_t i = 0; i < t.size();) {
+    size_t e = i + 1;
+    while (e < t.size() && t[e].x == t[i].x && t[e].z == t[i].z) ++e;
+    int c = 0;
+    for (int k = 1; k < NX; ++k)
+      if (cls[k].size() < cls[c].size()) c = k;
+    cls[c].insert(cls[c].end(), t.begin() + i, t.begin() + e);
+    i = e;
+  }
+  size_t at[NX] = {};
+  for (size_t i = 0; i < t.size(); ++i) {
+    int c = (int)(i % NX);
+    for (int k = 0; at[c] == cls[c].size() && k < NX; ++k) c = (c + 1) % NX;
+    t[i] = cls[c][at[c]++];
+  }
 }
 
 // Worker count for a tile list: the schedule of h2_tile_of with worker w on
@@ -148,7 +181,7 @@ static int list_workers(const std::vector<H2Args>& tab, const std::vector<int4>&
     for (int w = 0; w < W; ++w)
       for (int j = 0; j * W < total; ++j) {
         const int k = h2_tile_of(j, w, W);
-        if (k < total) cu[w % ncu] += 0.55 * tile_chunks(tab[t[k].x], t[k].z) + 6.0;
+        if (k < total) cu[w % ncu] += 0.55 * tile_chunks(tab[t[k].x], t[k].z, 64) + 6.0;
       }
     const double m = *std::max_element(cu.begin(), cu.end());
     if (m < bt) {
@@ -260,6 +293,7 @@ int qlognei_batch_prepare(const bta_qlognei_batch_item* items, int nm, void* ws,
   std::vector<FinishArgs> fin(nm);
   std::vector<int> cov_start(nm + 1, 0), mc_start(nm + 1, 0), fin_start(nm + 1, 0);
   BatchTiles T;
+  int64_t wide_tiles = 0;
   for (int i = 0; i < nm; ++i) {
     cov[i] = A[i].c;
     fwd[i] = A[i].fwd;
@@ -277,11 +311,22 @@ int qlognei_batch_prepare(const bta_qlognei_batch_item* items, int nm, void* ws,
     cov_start[i + 1] = cov_start[i] + (int)cb;
     mc_start[i + 1] = mc_start[i] + (int)(A[i].mc.nr == 2 ? (A[i].b + 1) / 2 : A[i].b);
     fin_start[i + 1] = fin_start[i] + (int)fb;
-    add_tiles(fwd[i], i, T.fwd);
-    if (grad) add_tiles(adj[i], i, T.adj);
+    wide_tiles += (int64_t)(fwd[i].M / H2Wide::TM) * (fwd[i].N / H2Wide::TN);
   }
-  order_tiles(fwd, T.fwd);
-  order_tiles(adj, T.adj);
+  // The forward list in 128 x 128 tiles from 1.75 of them per CU: they move two thirds
+  // of the bytes per product, which bounds the 128 x 64 ones (0.62 us a CU and chunk
+  // against 0.39 for the products alone).  512 rows per model, 128 x 64 / 128 x 128
+  // tiles, us: 32 models of 128 to 4096 points 313 / 212; with 2 tiles per CU, 4 x 4096
+  // points 161 / 125, 8 x 2048 85 / 68, 16 x 1024 48 / 42; with 1, 2 x 4096 74 / 83, 4 x
+  // 2048 44 / 47, 8 x 1024 27 / 28.
+  // (The adjoint list shares its launch with the MC stage, which has four waves.)
+  const bool wide = 4 * wide_tiles >= 7 * (int64_t)num_cus();
+  for (int i = 0; i < nm; ++i) {
+    add_tiles(fwd[i], i, wide ? H2Wide::TN : H2Mid::TN, T.fwd);
+    if (grad) add_tiles(adj[i], i, H2Mid::TN, T.adj);
+  }
+  order_tiles(fwd, wide ? H2Wide::TN : H2Mid::TN, T.fwd);
+  order_tiles(adj, H2Mid::TN, T.adj);
   // the exact layout (tile lists no longer than their bound)
   BatchLayout E;
   rc = batch_layout(items, nm, &T, E);
@@ -318,7 +363,8 @@ int qlognei_batch_prepare(const bta_qlognei_batch_item* items, int nm, void* ws,
   P.fin_blocks = fin_start[nm];
   P.fwd_tiles = (int)T.fwd.size();
   P.adj_tiles = (int)T.adj.size();
-  P.fwd_workers = list_workers(fwd, T.fwd);
+  // (more workers than tiles: the list holds 128 x 128 tiles)
+  P.fwd_workers = wide ? P.fwd_tiles + 1 : list_workers(fwd, T.fwd);
   P.adj_workers = grad ? list_workers(adj, T.adj) : 0;
   P.off_cov = E.cov;
   P.off_fwd = E.fwd;
@@ -389,9 +435,14 @@ int qlognei_batch_value_grad(const bta_qlognei_batch_plan* plan, hipStream_t s) 
     default: covar_list<8>(P, b, s); break;
   }
   BTA_LAUNCH_CHECK("qstep_covar_list_kernel");
-  hipLaunchKernelGGL(gemm_h2_list_kernel, dim3((unsigned)P.fwd_workers), dim3(256), 0, s,
-                     (const H2Args*)(b + P.off_fwd), (const int4*)(b + P.off_fwd_tiles),
-                     P.fwd_tiles);
+  const H2Args* ft = (const H2Args*)(b + P.off_fwd);
+  const int4* fl = (const int4*)(b + P.off_fwd_tiles);
+  if (P.fwd_workers > P.fwd_tiles)
+    hipLaunchKernelGGL(gemm_h2_list_wide_kernel, dim3((unsigned)P.fwd_tiles),
+                       dim3(64 * H2Wide::NW), 0, s, ft, fl);
+  else
+    hipLaunchKernelGGL(gemm_h2_list_kernel, dim3((unsigned)P.fwd_workers), dim3(256), 0, s, ft, fl,
+                       P.fwd_tiles);
   BTA_LAUNCH_CHECK("gemm_h2_list_kernel");
   switch (P.q) {
     case 1: adjoint_mc_list<1>(P, b, s); break;
