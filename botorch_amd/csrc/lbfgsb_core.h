@@ -644,6 +644,7 @@ __host__ __device__ inline int cauchy(C& c, View& w) {
     const int slot = (s.head + j) % m;
     const double* wc = (k < col ? w.wy : w.ws) + (size_t)slot * n;
     double acc = 0.0;
+#pragma unroll 4
     for (int i = 0; i < n; ++i) acc += wc[i] * w.d[i];
     w.p[k] = k < col ? acc : theta * acc;
   }
@@ -810,6 +811,7 @@ __host__ __device__ inline double list_dot(const double* a, const double* b,
                                            const int32_t* list, int cnt, bool up) {
   double acc = 0.0;
   if (up) {
+#pragma unroll 4
     for (int t = 0; t < cnt; ++t) acc += a[list[t]] * b[list[t]];
   } else {
     for (int t = cnt - 1; t >= 0; --t) acc += a[list[t]] * b[list[t]];
@@ -1234,9 +1236,11 @@ __host__ __device__ inline void matupd(C& c, View& w, double rr, double dr) {
     const int slot = (s.head + j) % m;
     double acc = 0.0;
     if (k < col - 1) {
+#pragma unroll 4
       for (int i = 0; i < n; ++i) acc += w.d[i] * w.wy[(size_t)slot * n + i];
       w.sy[(col - 1) * m + j] = acc;
     } else {
+#pragma unroll 4
       for (int i = 0; i < n; ++i) acc += w.ws[(size_t)slot * n + i] * w.d[i];
       w.ss[j * m + (col - 1)] = acc;
     }

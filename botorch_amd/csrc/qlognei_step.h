@@ -163,26 +163,6 @@ __device__ __forceinline__ void log_fatplus_grad(double x, double tau, double rt
   }
 }
 
-// x / l with r = 1 / l (correctly rounded), equal to the division: q is within two
-// ulps after the product, faithful after the first residual correction and correctly
-// rounded after the second (Markstein, "Computation of elementary functions on the IBM
-// RISC System/6000 processor", 1990).  An infinite x stays infinite.
-__device__ __forceinline__ double div_by(double x, double l, double r) {
-  const double q0 = x * r;
-  const double q1 = fma(fma(-q0, l, x), r, q0);
-  const double q2 = fma(fma(-q1, l, x), r, q1);
-  return fabs(q0) < INFINITY ? q2 : q0;
-}
-
-// v of lane l of the wave (l uniform)
-__device__ __forceinline__ double lane_bcast(double v, int l) {
-  const int2 p = __builtin_bit_cast(int2, v);
-  int2 r;
-  r.x = __builtin_amdgcn_readlane(p.x, l);
-  r.y = __builtin_amdgcn_readlane(p.y, l);
-  return __builtin_bit_cast(double, r);
-}
-
 // Triangular solves with the baseline factor L (n_b x n_b, row-major) for the Q rows of
 // x (pitch px): x <- x L^-T (forward) or out <- x L^-1 (back), the subtractions of an
 // element in column order.  Columns are eliminated one after the other, so the chain
