@@ -522,8 +522,8 @@ __device__ __forceinline__ void potrf_strip(const StepArgs& a, unsigned char* sm
 
 // Rank-64 update of one trailing lower 128 x 64 tile (tile row tm holds the
 // 2 tm + 2 tiles tn <= 2 tm + 1; rem = rows of the trailing matrix).  The
-// wave's part of C is loaded before the products: its latency overlaps the
-// first chunks of the main loop instead of following it.
+// wave's part of C is loaded behind the first three chunks of the main loop, whose
+// products then run while it is on its way.
 __device__ __forceinline__ void potrf_bulk_tile(const StepArgs& a, int t, int rem,
                                                 unsigned char* smem) {
   const int j = a.j;
@@ -535,20 +535,41 @@ __device__ __forceinline__ void potrf_bulk_tile(const StepArgs& a, int t, int re
   int tm = 0;
   while ((tm + 1) * (tm + 2) <= t) ++tm;  // tile rows before tm hold tm (tm + 1) tiles
   const int tn = t - tm * (tm + 1);
+  // (entries outside the matrix or above the diagonal are read at the nearest row and
+  // column inside and not stored)
   double cv[4][2][4];
+  auto load_c = [&]() {
+#pragma unroll
+    for (int mi = 0; mi < 4; ++mi)
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        const int row = min(tm * D_BM + wy * 64 + mi * 16 + Mfma<double>::row(gq, q), rem - 1);
+#pragma unroll
+        for (int ni = 0; ni < 2; ++ni) {
+          const int col = tn * 64 + wx * 32 + ni * 16 + l16;
+          cv[mi][ni][q] = Cm[(int64_t)row * lda + min(col, rem - 1)];
+        }
+      }
+  };
+  v4d acc[4][2];
+  d_mainloop<64, false, false, 32>(P, lda, P, lda, tm * D_BM, tn * 64, rem, rem, 0, LEAF, smem,
+                                   acc, load_c);
+  // tiles with neither the diagonal nor the matrix's end store without a test per entry
+  const bool full = tn * 64 + 63 <= tm * D_BM && (tm + 1) * D_BM <= rem;
 #pragma unroll
   for (int mi = 0; mi < 4; ++mi)
 #pragma unroll
     for (int q = 0; q < 4; ++q) {
       const int row = tm * D_BM + wy * 64 + mi * 16 + Mfma<double>::row(gq, q);
 #pragma unroll
-      for (int ni = 0; ni < 2; ++ni) {
-        const int col = tn * 64 + wx * 32 + ni * 16 + l16;
-        cv[mi][ni][q] = (row < rem && col <= row) ? Cm[(int64_t)row * lda + col] : 0.0;
+      for (int ni = 0; ni < 2; ++ni) cv[mi][ni][q] -= acc[mi][ni][q];
+      double* p = Cm + (int64_t)row * lda + tn * 64 + wx * 32 + l16;
+      if (full) {
+        p[0] = cv[mi][0][q];
+        p[16] = cv[mi][1][q];
       }
     }
-  v4d acc[4][2];
-  d_mainloop<64, false, false>(P, lda, P, lda, tm * D_BM, tn * 64, rem, rem, 0, LEAF, smem, acc);
+  if (full) return;
 #pragma unroll
   for (int mi = 0; mi < 4; ++mi)
 #pragma unroll
@@ -557,7 +578,7 @@ __device__ __forceinline__ void potrf_bulk_tile(const StepArgs& a, int t, int re
 #pragma unroll
       for (int ni = 0; ni < 2; ++ni) {
         const int col = tn * 64 + wx * 32 + ni * 16 + l16;
-        if (row < rem && col <= row) Cm[(int64_t)row * lda + col] = cv[mi][ni][q] - acc[mi][ni][q];
+        if (row < rem && col <= row) Cm[(int64_t)row * lda + col] = cv[mi][ni][q];
       }
     }
 }
@@ -585,20 +606,20 @@ __device__ __forceinline__ void inv_partial(const StepArgs& a, int4 t, unsigned 
   const int wy = wv >> 1, wx = wv & 1, l16 = lane & 15, gq = lane >> 4;
   const int row0 = q * D_BM, col0 = c * LEAF;
   double cv[4][2][4];
+  auto load_c = [&]() {
 #pragma unroll
-  for (int mi = 0; mi < 4; ++mi)
+    for (int mi = 0; mi < 4; ++mi)
 #pragma unroll
-    for (int qq = 0; qq < 4; ++qq) {
-      const int row = row0 + wy * 64 + mi * 16 + Mfma<double>::row(gq, qq);
+      for (int qq = 0; qq < 4; ++qq) {
+        const int row = min(row0 + wy * 64 + mi * 16 + Mfma<double>::row(gq, qq), np - 1);
 #pragma unroll
-      for (int ni = 0; ni < 2; ++ni) {
-        const int col = col0 + wx * 32 + ni * 16 + l16;
-        cv[mi][ni][qq] = (!first && row < np) ? X[(int64_t)row * ldx + col] : 0.0;
+        for (int ni = 0; ni < 2; ++ni)
+          cv[mi][ni][qq] = X[(int64_t)row * ldx + col0 + wx * 32 + ni * 16 + l16];
       }
-    }
+  };
   v4d acc[4][2];
-  d_mainloop<64, false, true>(a.A, a.lda, X, ldx, row0, col0, np, np, k0 * LEAF, k1 * LEAF, smem,
-                              acc);
+  d_mainloop<64, false, true, 32>(a.A, a.lda, X, ldx, row0, col0, np, np, k0 * LEAF, k1 * LEAF,
+                                  smem, acc, load_c);
 #pragma unroll
   for (int mi = 0; mi < 4; ++mi)
 #pragma unroll
@@ -607,7 +628,8 @@ __device__ __forceinline__ void inv_partial(const StepArgs& a, int4 t, unsigned 
 #pragma unroll
       for (int ni = 0; ni < 2; ++ni) {
         const int col = col0 + wx * 32 + ni * 16 + l16;
-        if (row < np) X[(int64_t)row * ldx + col] = cv[mi][ni][qq] + acc[mi][ni][qq];
+        if (row < np)
+          X[(int64_t)row * ldx + col] = (first ? 0.0 : cv[mi][ni][qq]) + acc[mi][ni][qq];
       }
     }
 }

@@ -107,12 +107,18 @@ __device__ __forceinline__ void frag_mn(uint32_t a0, double (&x)[F][2]) {
 // N x K (ldb) or, with BKN, K x N.  Rows/columns at or past M/N read the
 // in-bounds ones 64 earlier.  All 256 threads must call it; it ends with a
 // barrier, so the caller may reuse the LDS afterwards.
-template <int BN, bool AKM, bool BKN>
+// pre(): exactly PRE loads to registers, issued behind the first three chunks' loads, so
+// that they arrive while those are multiplied (K at least three chunks where PRE > 0).
+struct DNoPre {
+  __device__ void operator()() const {}
+};
+template <int BN, bool AKM, bool BKN, int PRE = 0, typename F = DNoPre>
 __device__ __forceinline__ void d_mainloop(const double* __restrict__ A, int64_t lda,
                                            const double* __restrict__ B, int64_t ldb, int row0,
                                            int col0, int M, int N, int kb, int ke,
                                            unsigned char* lds,
-                                           v4d (&acc)[DCfg<BN>::FM][DCfg<BN>::FN]) {
+                                           v4d (&acc)[DCfg<BN>::FM][DCfg<BN>::FN],
+                                           F pre = F()) {
   using C = DCfg<BN>;
   constexpr int S = C::STAGES;
   const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
@@ -218,8 +224,11 @@ __device__ __forceinline__ void d_mainloop(const double* __restrict__ A, int64_t
   // across, in particular no LDS read above the wait and the barrier (another
   // wave's direct loads fill part of the stage, and only the barrier orders
   // them).
-  auto arrive = [&](int later) {
-    if (later >= 2)
+  // (early: the PRE loads are younger than chunk ci's)
+  auto arrive = [&](int later, bool early) {
+    if (PRE > 0 && early)
+      d_wait_vmcnt<2 * C::LOADS_W + PRE>();
+    else if (later >= 2)
       d_wait_vmcnt<2 * C::LOADS_W>();
     else if (later == 1)
       d_wait_vmcnt<C::LOADS_W>();
@@ -247,13 +256,22 @@ __device__ __forceinline__ void d_mainloop(const double* __restrict__ A, int64_t
 #pragma unroll
   for (int ci = 0; ci < S - 1; ++ci)
     if (ci < nk) issue(ci);
+  if (PRE > 0) {
+    // the counts of arrive() rely on this order: the chunks' loads, then pre's, then
+    // the first wait
+    __asm__ __volatile__("" ::: "memory");
+    __builtin_amdgcn_sched_barrier(0);
+    pre();
+    __builtin_amdgcn_sched_barrier(0);
+    __asm__ __volatile__("" ::: "memory");
+  }
   // Chunk it's fragments are read one iteration ahead, so its MFMAs overlap
   // the reads of chunk it + 1.  Chunks in flight: it + 2 .. it + S (the
   // issue at iteration it reuses chunk it's stage, whose reads finished at
   // it - 1).
   double af[C::FM][2], bf[C::FN][2], an[C::FM][2], bn[C::FN][2];
   if (nk > 0) {
-    arrive(min(S - 2, nk - 1));
+    arrive(min(S - 2, nk - 1), nk > 4);
     if (S - 1 < nk) issue(S - 1);
     read(0, af, bf);
     wait_ties(af, bf);
@@ -261,7 +279,7 @@ __device__ __forceinline__ void d_mainloop(const double* __restrict__ A, int64_t
   for (int it = 0; it < nk; ++it) {
     const bool more = it + 1 < nk;
     if (more) {
-      arrive(min(S - 2, nk - 2 - it));
+      arrive(min(S - 2, nk - 2 - it), it < 2 && nk > 4);
       if (it + S < nk) issue(it + S);
       read(it + 1, an, bn);
     }
