@@ -304,9 +304,11 @@ __device__ __forceinline__ void inv16_block(const double* S, int blk, double* V)
       const int k = 4 * t + r;
       lv[i][t] = k < i ? S[(b0 + i) * LP + b0 + k] : 0.0;
     }
+  // one division per lane, passed by readlane
+  const double rdl = 1.0 / S[(b0 + (lane & 15)) * LP + b0 + (lane & 15)];
   double rd[16];
 #pragma unroll
-  for (int i = 0; i < 16; ++i) rd[i] = 1.0 / S[(b0 + i) * LP + b0 + i];
+  for (int i = 0; i < 16; ++i) rd[i] = readlane_d(rdl, i);
   double x[4] = {0.0, 0.0, 0.0, 0.0};
 #pragma unroll
   for (int i = 0; i < 16; ++i) {
@@ -381,8 +383,8 @@ __device__ __forceinline__ void trinv64_blocked(const double* S, const double* r
 // by blocked forward substitution: wave w takes rows [16w, 16w + 16) and the
 // four 16-column blocks in turn, X_k = (T_k - sum_{m<k} X_m L_km^T) V_k^T
 // with V_k = L_kk^-1 (inv16_block), so no wave waits for another.  T is
-// formed before the factorisation; waves 1-3 invert V_0..V_2 while wave 0
-// factors the panels.  The
+// formed by waves 1-3, which also invert V_0..V_2, while wave 0 factors the
+// panels.  The
 // remaining workgroups apply column j-1's update to the trailing lower tiles
 // right of column j (the strip covers column j): A_bc -= L_b,j-1 L_c,j-1^T on
 // 128 x 64 FP64 MFMA tiles.
@@ -432,16 +434,26 @@ __device__ __forceinline__ void potrf_strip(const StepArgs& a, unsigned char* sm
       for (int q = 0; q < 4; ++q)
         dacc[u][q] = Ajj[(int64_t)(16 * dib[u] + g + 4 * q) * lda + 16 * djb[u] + l16];
   }
-  // T = A_bj - L_b,j-1 L_j,j-1^T: wave wv holds column block wv, row blocks
-  // u = 0..3, formed before the factorisation (L_b,j-1 staged in S, which
-  // takes D afterwards)
-  v4d tacc[4];
-  if (own)
+  // T = A_bj - L_b,j-1 L_j,j-1^T.  Waves 1..3 form block rows 0..2 (wave w row w - 1,
+  // tacc[k] its column block k) while wave 0 factors the panels, with their rows of
+  // L_b,j-1 in registers: S, where they are staged, takes D.  Block row 3 is formed
+  // ahead of the factorisation, wave w its column block w.  (With all of T formed
+  // ahead, a strip workgroup at n = 1000 took 15.1 K of its 43 K cycles up to the
+  // factorisation; now 11.8 K.)
+  const int wk = wave_uniform(wv);
+  const int tr = 16 * max(wk - 1, 0);
+  v4d tacc[4], tlast;
+  if (own) {
 #pragma unroll
-    for (int u = 0; u < 4; ++u)
+    for (int q = 0; q < 4; ++q) {
+      if (wk > 0)
 #pragma unroll
-      for (int q = 0; q < 4; ++q)
-        tacc[u][q] = Abj[(int64_t)(16 * u + g + 4 * q) * lda + 16 * wv + l16];
+        for (int k = 0; k < 4; ++k)
+          tacc[k][q] = Abj[(int64_t)(tr + g + 4 * q) * lda + 16 * k + l16];
+      tlast[q] = Abj[(int64_t)(48 + g + 4 * q) * lda + 16 * wk + l16];
+    }
+  }
+  double tl[16];  // -L_b,j-1, block row wk - 1
   if (j > 0) {
     stage64x2(Ajj - LEAF, Bf, Q, S, lda, own);  // L_j,j-1 -> Bf, L_b,j-1 -> S
     __syncthreads();
@@ -453,14 +465,15 @@ __device__ __forceinline__ void potrf_strip(const StepArgs& a, unsigned char* sm
           dacc[u] = __builtin_amdgcn_mfma_f64_16x16x4f64(
               -Bf[(16 * dib[u] + l16) * LP + 4 * s + g], Bf[(16 * djb[u] + l16) * LP + 4 * s + g],
               dacc[u], 0, 0, 0);
-    if (own)
+    if (own) {
 #pragma unroll
-      for (int u = 0; u < 4; ++u)
-#pragma unroll
-        for (int s = 0; s < 16; ++s)
-          tacc[u] = __builtin_amdgcn_mfma_f64_16x16x4f64(
-              -S[(16 * u + l16) * LP + 4 * s + g], Bf[(16 * wv + l16) * LP + 4 * s + g], tacc[u],
-              0, 0, 0);
+      for (int s = 0; s < 16; ++s) {
+        tl[s] = -S[(tr + l16) * LP + 4 * s + g];
+        tlast = __builtin_amdgcn_mfma_f64_16x16x4f64(-S[(48 + l16) * LP + 4 * s + g],
+                                                     Bf[(16 * wk + l16) * LP + 4 * s + g], tlast,
+                                                     0, 0, 0);
+      }
+    }
     __syncthreads();  // S (L_b,j-1) read by every wave
   }
 #pragma unroll
@@ -469,8 +482,24 @@ __device__ __forceinline__ void potrf_strip(const StepArgs& a, unsigned char* sm
   __syncthreads();
   // while wave 0 factors panel p, wave p (p >= 1) inverts the diagonal block
   // p - 1 finished before
+  // and in panel 0 every wave, later the ones not inverting, form two blocks of T
+  auto t_block = [&](int k) {
+    const double* b = Bf + (16 * k + l16) * LP + g;
+#pragma unroll
+    for (int s = 0; s < 16; ++s)
+      tacc[k] = __builtin_amdgcn_mfma_f64_16x16x4f64(tl[s], b[4 * s], tacc[k], 0, 0, 0);
+  };
   auto bg = [&](int p) {
-    if (own && p >= 1 && wv == p) inv16_block<VP, false>(S, p - 1, Vs);
+    if (!own) return;
+    if (p >= 1 && wk == p) inv16_block<VP, false>(S, p - 1, Vs);
+    if (j > 0 && p == 0) {
+      t_block(0);
+      t_block(1);
+    }
+    if (j > 0 && (p == 1 ? wk != 1 : p == 2 && wk == 1)) {
+      t_block(2);
+      t_block(3);
+    }
   };
   chol64_blocked(S, rdiag, colv, flags, flags + 1, bg);
   if (flags[0] >= 0) {
@@ -499,9 +528,11 @@ __device__ __forceinline__ void potrf_strip(const StepArgs& a, unsigned char* sm
     }
     return;
   }
+  st16(Bf, 48, 16 * wk, tlast);
+  if (wk == 0) inv16_block<VP, false>(S, 3, Vs);
+  else
 #pragma unroll
-  for (int u = 0; u < 4; ++u) st16(Bf, 16 * u, 16 * wv, tacc[u]);
-  if (wv == 0) inv16_block<VP, false>(S, 3, Vs);
+    for (int k = 0; k < 4; ++k) st16(Bf, tr, 16 * k, tacc[k]);
   __syncthreads();
   const int r0 = 16 * wv;
 #pragma unroll
