@@ -419,28 +419,33 @@ __device__ __forceinline__ void potrf_strip(const StepArgs& a, unsigned char* sm
   double* Ajj = a.A + (int64_t)j * LEAF * lda + (int64_t)j * LEAF;
   double* Abj = a.A + (int64_t)b * LEAF * lda + (int64_t)j * LEAF;
   const double* Q = Abj - LEAF;  // L_b,j-1 (j > 0)
-  // D blocks (ib, jb), jb <= ib (10 of them), dealt round-robin over the waves
+  // D blocks (ib, jb), jb <= ib: wave w updates (w, 0) ahead of the factorisation, whose
+  // first panel reads no other, and waves 1..3 two more each while wave 0 is on it.
+  const int wk = wave_uniform(wv);
+  auto d_row = [&](int u) { return u == 0 ? wk : wk == 1 ? 1 + (u - 1) : wk == 2 ? 1 + u : 3; };
+  auto d_col = [&](int u) { return u == 0 ? 0 : wk == 1 ? 1 : wk == 2 ? 3 - u : 1 + u; };
   v4d dacc[3];
-  int dib[3], djb[3];
 #pragma unroll
-  for (int u = 0; u < 3; ++u) {
-    const int bi = wv + 4 * u;
-    int ib = 0;
-    while ((ib + 1) * (ib + 2) / 2 <= bi) ++ib;
-    dib[u] = ib;
-    djb[u] = bi - ib * (ib + 1) / 2;
-    if (bi < 10)
+  for (int u = 0; u < 3; ++u)
+    if (u == 0 || wk > 0)
 #pragma unroll
       for (int q = 0; q < 4; ++q)
-        dacc[u][q] = Ajj[(int64_t)(16 * dib[u] + g + 4 * q) * lda + 16 * djb[u] + l16];
-  }
+        dacc[u][q] = Ajj[(int64_t)(16 * d_row(u) + g + 4 * q) * lda + 16 * d_col(u) + l16];
+  auto d_block = [&](int u) {
+    const double* x = Bf + (16 * d_row(u) + l16) * LP + g;
+    const double* y = Bf + (16 * d_col(u) + l16) * LP + g;
+    if (j > 0)
+#pragma unroll
+      for (int s = 0; s < 16; ++s)
+        dacc[u] = __builtin_amdgcn_mfma_f64_16x16x4f64(-x[4 * s], y[4 * s], dacc[u], 0, 0, 0);
+  };
   // T = A_bj - L_b,j-1 L_j,j-1^T.  Waves 1..3 form block rows 0..2 (wave w row w - 1,
   // tacc[k] its column block k) while wave 0 factors the panels, with their rows of
   // L_b,j-1 in registers: S, where they are staged, takes D.  Block row 3 is formed
-  // ahead of the factorisation, wave w its column block w.  (With all of T formed
+  // ahead of the factorisation, wave w its column block w.  (With all of D and T formed
   // ahead, a strip workgroup at n = 1000 took 15.1 K of its 43 K cycles up to the
-  // factorisation; now 11.8 K.)
-  const int wk = wave_uniform(wv);
+  // factorisation and the log likelihood's call 410 us; 387 with T beside the panels,
+  // 365 with D's blocks there too.)
   const int tr = 16 * max(wk - 1, 0);
   v4d tacc[4], tlast;
   if (own) {
@@ -457,14 +462,7 @@ __device__ __forceinline__ void potrf_strip(const StepArgs& a, unsigned char* sm
   if (j > 0) {
     stage64x2(Ajj - LEAF, Bf, Q, S, lda, own);  // L_j,j-1 -> Bf, L_b,j-1 -> S
     __syncthreads();
-#pragma unroll
-    for (int u = 0; u < 3; ++u)
-      if (wv + 4 * u < 10)
-#pragma unroll
-        for (int s = 0; s < 16; ++s)
-          dacc[u] = __builtin_amdgcn_mfma_f64_16x16x4f64(
-              -Bf[(16 * dib[u] + l16) * LP + 4 * s + g], Bf[(16 * djb[u] + l16) * LP + 4 * s + g],
-              dacc[u], 0, 0, 0);
+    d_block(0);
     if (own) {
 #pragma unroll
       for (int s = 0; s < 16; ++s) {
@@ -476,13 +474,11 @@ __device__ __forceinline__ void potrf_strip(const StepArgs& a, unsigned char* sm
     }
     __syncthreads();  // S (L_b,j-1) read by every wave
   }
-#pragma unroll
-  for (int u = 0; u < 3; ++u)
-    if (wv + 4 * u < 10) st16(S, 16 * dib[u], 16 * djb[u], dacc[u]);
+  st16(S, 16 * wk, 0, dacc[0]);
   __syncthreads();
-  // while wave 0 factors panel p, wave p (p >= 1) inverts the diagonal block
-  // p - 1 finished before
-  // and in panel 0 every wave, later the ones not inverting, form two blocks of T
+  // while wave 0 factors panel 0, waves 1..3 finish D; while it factors panel p >= 1,
+  // wave p inverts the diagonal block p - 1 finished before and the other two form two
+  // blocks of T each
   auto t_block = [&](int k) {
     const double* b = Bf + (16 * k + l16) * LP + g;
 #pragma unroll
@@ -490,13 +486,20 @@ __device__ __forceinline__ void potrf_strip(const StepArgs& a, unsigned char* sm
       tacc[k] = __builtin_amdgcn_mfma_f64_16x16x4f64(tl[s], b[4 * s], tacc[k], 0, 0, 0);
   };
   auto bg = [&](int p) {
+    if (p == 0) {
+#pragma unroll
+      for (int u = 1; u < 3; ++u) {
+        d_block(u);
+        st16(S, 16 * d_row(u), 16 * d_col(u), dacc[u]);
+      }
+    }
     if (!own) return;
     if (p >= 1 && wk == p) inv16_block<VP, false>(S, p - 1, Vs);
-    if (j > 0 && p == 0) {
+    if (j == 0) return;
+    if (p == 1 ? wk != 1 : p == 2 && wk == 1) {
       t_block(0);
       t_block(1);
-    }
-    if (j > 0 && (p == 1 ? wk != 1 : p == 2 && wk == 1)) {
+    } else if (p == 2 ? wk == 3 : p == 3 && wk != 3) {
       t_block(2);
       t_block(3);
     }
