@@ -426,8 +426,10 @@ class SingleTaskGP(torch.nn.Module):
         L = _lib.lib()
         n, d = X.shape
         n_pad = _lib.round_up(n, 128)
-        ls = self.covar_module.lengthscale.detach().to(device=dev,
-                                                       dtype=torch.float64).contiguous()
+        # a copy: without a constraint transform the lengthscale is the parameter itself,
+        # and the cache has to keep the values it was built with
+        ls = self.covar_module.lengthscale.detach().to(
+            device=dev, dtype=torch.float64, copy=True).contiguous()
         center = torch.empty(d, dtype=torch.float64, device=dev)
         xs = torch.empty(n_pad, d, dtype=torch.float64, device=dev)
         st = _lib.stream()
