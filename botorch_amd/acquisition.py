@@ -401,17 +401,18 @@ class BatchedQLogNEI:
         self.q = q
         self.need_grad = need_grad
         dev = self.acqfs[0].X_baseline.device
-        # every model's buffers are slices of one tensor per kind, so that a step
-        # fills, reads back and hands out each kind in one operation
+        # every model's results are slices of one tensor per kind, so that a step
+        # reads back and hands out each kind in one operation
         sizes = [(b, q, acq.X_baseline.shape[-1]) for acq, b in zip(self.acqfs, restarts)]
         n_x, n_b = sum(b * q * d for b, q, d in sizes), sum(restarts)
-        self._flat_X = torch.zeros(n_x, dtype=torch.float64, device=dev)
         self._flat_value = torch.empty(n_b, dtype=torch.float64, device=dev)
         self._flat_grad = (torch.empty(n_x, dtype=torch.float64, device=dev) if need_grad
                            else None)
         self._flat_status = torch.empty(n_b, dtype=torch.int32, device=dev)
         self._sizes = sizes
-        self.X, self.value = self._split_x(self._flat_X), self._split_b(self._flat_value)
+        self.X = [torch.zeros(size, dtype=torch.float64, device=dev) for size in sizes]
+        self._x_storages = {buf.untyped_storage().data_ptr() for buf in self.X}
+        self.value = self._split_b(self._flat_value)
         self.grad = self._split_x(self._flat_grad) if need_grad else [None] * len(acqfs)
         self.status = self._split_b(self._flat_status)
         self._states = []
@@ -457,19 +458,24 @@ class BatchedQLogNEI:
                                                            _lib.stream()),
                    "qlognei_batch_value_grad")
 
+    def _fill(self, Xs) -> None:
+        """X[i] <- Xs[i], one after the other; in one launch where no source lies in
+        the buffers (their own tensors may be passed: nothing is to copy then)."""
+        pairs = [(buf, X) for buf, X in zip(self.X, Xs) if X is not buf]
+        with torch.no_grad():
+            if pairs and all(X.shape == buf.shape and X.device == buf.device
+                             and X.untyped_storage().data_ptr() not in self._x_storages
+                             for buf, X in pairs):
+                torch._foreach_copy_([buf for buf, _ in pairs], [X for _, X in pairs])
+            else:
+                for buf, X in pairs:
+                    buf.copy_(X)
+
     def value_and_grad(self, Xs):
         """Copies Xs[i] (restarts[i] x q x d) into the buffers, runs the step and
         returns ([value_i], [grad_i]), raising like the one-model step on failed
         samples."""
-        Xs = list(Xs)
-        buf = self._flat_X
-        if len(Xs) == len(self._sizes) and all(
-                X.shape == size and X.device == buf.device and X.dtype == buf.dtype
-                for X, size in zip(Xs, self._sizes)):
-            torch.cat([X.detach().reshape(-1) for X in Xs], out=buf)
-        else:
-            for dst, X in zip(self.X, Xs):
-                dst.copy_(X)
+        self._fill(list(Xs))
         self.launch()
         bits = self._flat_status.cpu().numpy()
         row = 0
