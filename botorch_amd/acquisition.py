@@ -401,20 +401,14 @@ class BatchedQLogNEI:
         self.q = q
         self.need_grad = need_grad
         dev = self.acqfs[0].X_baseline.device
-        # every model's results are slices of one tensor per kind, so that a step
-        # reads back and hands out each kind in one operation
         sizes = [(b, q, acq.X_baseline.shape[-1]) for acq, b in zip(self.acqfs, restarts)]
-        n_x, n_b = sum(b * q * d for b, q, d in sizes), sum(restarts)
-        self._flat_value = torch.empty(n_b, dtype=torch.float64, device=dev)
-        self._flat_grad = (torch.empty(n_x, dtype=torch.float64, device=dev) if need_grad
-                           else None)
-        self._flat_status = torch.empty(n_b, dtype=torch.int32, device=dev)
-        self._sizes = sizes
         self.X = [torch.zeros(size, dtype=torch.float64, device=dev) for size in sizes]
         self._x_storages = {buf.untyped_storage().data_ptr() for buf in self.X}
-        self.value = self._split_b(self._flat_value)
-        self.grad = self._split_x(self._flat_grad) if need_grad else [None] * len(acqfs)
-        self.status = self._split_b(self._flat_status)
+        self.value = [torch.empty(b, dtype=torch.float64, device=dev) for b in restarts]
+        self.grad = [torch.empty_like(x) for x in self.X] if need_grad else [None] * len(acqfs)
+        # the status words are slices of one tensor: a step reads them in one copy
+        self._flat_status = torch.empty(sum(restarts), dtype=torch.int32, device=dev)
+        self.status = list(self._flat_status.split(list(restarts)))
         self._states = []
         items = (_lib.QLogNEIBatchItem * len(acqfs))()
         for i, (acq, b) in enumerate(zip(self.acqfs, restarts)):
@@ -443,14 +437,6 @@ class BatchedQLogNEI:
                                                self.ws.numel(), ctypes.byref(self.plan),
                                                _lib.stream()), "qlognei_batch_prepare")
 
-    def _split_x(self, flat: Tensor):
-        """The models' b x q x d parts of a flat tensor."""
-        parts = flat.split([b * q * d for b, q, d in self._sizes])
-        return [p.view(size) for p, size in zip(parts, self._sizes)]
-
-    def _split_b(self, flat: Tensor):
-        return list(flat.split([b for b, _, _ in self._sizes]))
-
     def launch(self) -> None:
         """Enqueue one step over every model (reads ``X``, writes ``value``,
         ``grad``, ``status``); no host synchronisation."""
@@ -477,20 +463,26 @@ class BatchedQLogNEI:
         samples."""
         self._fill(list(Xs))
         self.launch()
+        # the caller's copies, tensors of their own, made while the step runs
+        results = self.value + self.grad if self.need_grad else self.value
+        out = [torch.empty_like(t) for t in results]
+        torch._foreach_copy_(out, results)
+        values, grads = out[:len(self.value)], out[len(self.value):]
         bits = self._flat_status.cpu().numpy()
         row = 0
         for i, acq in enumerate(self.acqfs):
-            mine = bits[row:row + self._sizes[i][0]]
-            row += self._sizes[i][0]
+            mine = bits[row:row + self.value[i].numel()]
+            row += self.value[i].numel()
             if (mine & _CACHED_ROOT_FAILED).any():
                 # this model's cached-root update failed: its acquisition function
                 # samples it again from the joint posterior (and warns)
                 v, g = acq._run(self.X[i], self.need_grad)
                 self.value[i].copy_(v)
+                values[i].copy_(v)
                 if self.need_grad:
                     self.grad[i].copy_(g)
+                    grads[i].copy_(g)
                 self.status[i].zero_()
                 mine[:] = 0
         _raise_on_status(int(np.bitwise_or.reduce(bits, initial=0)))
-        return (self._split_b(self._flat_value.clone()),
-                self._split_x(self._flat_grad.clone()) if self.need_grad else None)
+        return values, grads if self.need_grad else None

@@ -76,3 +76,38 @@ def test_buffers_take_points_that_require_grad():
     step.launch()
     assert _same([step.value, step.grad], want)
     assert _same(step.value_and_grad(_points(step, 2)), want)
+
+
+def test_results_are_independent_of_each_other_and_of_the_buffers():
+    """Editing or keeping one model's result touches no other's: own storage, own
+    version counter (a graph that saved another result stays valid)."""
+    step = _step()
+    Xs = _points(step, 3)
+    values, grads = step.value_and_grad(Xs)
+    parts = values + grads
+    assert len({t.untyped_storage().data_ptr() for t in parts + step.value + step.grad}) == 12
+    assert all(t.untyped_storage().nbytes() == t.numel() * 8 for t in parts)
+    w = torch.ones_like(grads[0], requires_grad=True)
+    loss = (w * grads[0]).sum()  # saves grads[0]
+    kept = [t.clone() for t in parts]
+    for t in values + grads[1:]:
+        t.mul_(2.0)
+    loss.backward()
+    assert torch.equal(w.grad, grads[0])
+    again = step.value_and_grad(Xs)
+    assert _same(again, [kept[:3], kept[3:]])
+
+
+def test_a_failed_models_results_come_from_the_joint_posterior():
+    step = _step()
+    Xs = _points(step, 4)
+    want = step.value_and_grad(Xs)
+    step.acqfs[1]._keep["Lb"].zero_()
+    with pytest.warns(B.BotorchWarning, match="Falling back"):
+        v1, g1 = step.acqfs[1].value_and_grad(Xs[1])
+    with pytest.warns(B.BotorchWarning, match="Falling back"):
+        values, grads = step.value_and_grad(Xs)
+    assert torch.equal(values[1], v1) and torch.equal(grads[1], g1)
+    assert torch.equal(step.value[1], v1) and torch.equal(step.grad[1], g1)
+    for i in (0, 2):
+        assert torch.equal(values[i], want[0][i]) and torch.equal(grads[i], want[1][i])
