@@ -186,13 +186,18 @@ def load(path: str = LIB_PATH) -> ctypes.CDLL:
                 raise RuntimeError(
                     f"{path} is missing: build it with `python -m botorch_amd.build`.")
             lib = ctypes.CDLL(path)
-            for name, (res, args) in SIGNATURES.items():
-                fn = getattr(lib, name)
-                fn.restype = res
-                fn.argtypes = args
-            if lib.bta_abi_version() != ABI_VERSION:
-                raise RuntimeError(f"{path} has C ABI {lib.bta_abi_version()}, this binding "
-                                   f"expects {ABI_VERSION}: rebuild the library.")
+            try:
+                version = lib.bta_abi_version()
+                if version != ABI_VERSION:
+                    raise RuntimeError(f"{path} has C ABI {version}, this binding expects "
+                                       f"{ABI_VERSION}: rebuild the library.")
+                for name, (res, args) in SIGNATURES.items():
+                    fn = getattr(lib, name)
+                    fn.restype = res
+                    fn.argtypes = args
+            except AttributeError as e:  # a version gains entry points without a new number
+                raise RuntimeError(f"{path} lacks an entry point of this binding: rebuild the "
+                                   f"library ({e}).") from e
             _lib = lib
     return _lib
 
