@@ -366,18 +366,23 @@ class SingleTaskGP(torch.nn.Module):
     def kernel_kind(self) -> int:
         return self.covar_module.kind
 
-    def _host_values(self, extra=()):
-        """The hyperparameters, the outcome statistics and the tensors ``extra`` as
-        host numbers, read in one copy (each read of its own waits for the GPU):
-        (lengthscale list, outputscale, noise, constant, (y_mean, y_std), the values
-        of each extra tensor as a flat list)."""
+    def _host_values(self, extra=(), stats=False):
+        """The hyperparameters and the tensors ``extra`` as host numbers, with ``stats``
+        the outcome statistics too, read in one copy (each read of its own waits for the
+        GPU): (lengthscale list, outputscale, noise, constant, (y_mean, y_std), the
+        values of each extra tensor as a flat list)."""
         with torch.no_grad():
             k = self.covar_module
-            t = getattr(self, "outcome_transform", None)
             parts = [k.lengthscale, k.outputscale, self.likelihood.noise,
                      self.mean_module.constant]
+            t = getattr(self, "outcome_transform", None) if stats else None
             if t is not None:
                 parts += [t.means, t.stdvs]
+            for p in parts[1:]:
+                if p.numel() != 1:
+                    raise RuntimeError(f"a Tensor with {p.numel()} elements cannot be converted "
+                                       "to Scalar")
+            first_extra = len(parts)
             parts += extra
             flat = [p.detach().reshape(-1) for p in parts]
             dev, dt = flat[0].device, torch.float64
@@ -388,9 +393,8 @@ class SingleTaskGP(torch.nn.Module):
         for p in flat:
             out.append(vals[i:i + p.numel()])
             i += p.numel()
-        stats = (out[4][0], out[5][0]) if t is not None else (0.0, 1.0)
-        return (out[0], out[1][0], out[2][0], out[3][0], stats,
-                out[len(out) - len(extra):] if extra else [])
+        y_stats = (out[4][0], out[5][0]) if t is not None else (0.0, 1.0)
+        return out[0], out[1][0], out[2][0], out[3][0], y_stats, out[first_extra:]
 
     def hyperparameters(self) -> dict:
         _, outputscale, noise, constant, _, _ = self._host_values()
@@ -416,7 +420,7 @@ class SingleTaskGP(torch.nn.Module):
     def prediction_cache(self) -> dict:
         """L, L^-1, alpha and the C struct describing the model; rebuilt when a
         hyperparameter changed (like gpytorch's prediction strategy reset)."""
-        lengthscale, outputscale, noise, constant, y_stats, _ = self._host_values()
+        lengthscale, outputscale, noise, constant, y_stats, _ = self._host_values(stats=True)
         key = (tuple(lengthscale), outputscale, noise, constant, y_stats,
                float(self.cholesky_jitter), int(self.refine_solves))
         if self._cache is not None and self._cache_key == key:
