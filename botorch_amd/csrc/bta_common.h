@@ -172,15 +172,17 @@ __device__ __forceinline__ double kern_grad_factor_k(double r2, double s) {
   return s * exp_nonpos(-0.5 * r2);
 }
 
-// x / l with r = 1 / l (correctly rounded), equal to the division: q is within two
-// ulps after the product, faithful after the first residual correction and correctly
-// rounded after the second (Markstein, "Computation of elementary functions on the IBM
-// RISC System/6000 processor", 1990).  An infinite x stays infinite.
-__device__ __forceinline__ double div_by(double x, double l, double r) {
+// x / l with r = 1 / l (correctly rounded), equal to the division while x's residuals
+// stay normal (|x| > 1e-290): q is within two ulps after the product, faithful after the
+// first residual correction and correctly rounded after the second (Markstein,
+// "Computation of elementary functions on the IBM RISC System/6000 processor", 1990).
+// A product of 0 (also by an infinite l), infinity or NaN is the quotient already; its
+// residual would be NaN or lose the sign.
+__host__ __device__ __forceinline__ double div_by(double x, double l, double r) {
   const double q0 = x * r;
   const double q1 = fma(fma(-q0, l, x), r, q0);
   const double q2 = fma(fma(-q1, l, x), r, q1);
-  return fabs(q0) < INFINITY ? q2 : q0;
+  return q0 != 0.0 && fabs(q0) < INFINITY ? q2 : q0;
 }
 
 // v of lane l of the wave (l uniform)
