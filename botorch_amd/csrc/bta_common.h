@@ -100,10 +100,11 @@ __host__ __device__ __forceinline__ double div_normal(double n, double d) {
   return fma(fma(-d, q, n), r, q);
 }
 
-// log x for 0 < x < infinity (NaN gives NaN, infinity infinity): x = 2^k (1 + f) with
-// 1 + f in [sqrt 1/2, sqrt 2), s = f / (2 + f), log(1 + f) = 2 atanh s summed as
-// f - (f^2 / 2 - s (f^2 / 2 + R)) as in fdlibm, R = sum_{i >= 1} 2 s^2i / (2 i + 1) by
-// its Taylor series to s^22 (remainder < 1e-18 relative), and k ln 2 in two parts.
+// log x for finite x > 0 (NaN gives NaN, infinity infinity; the callers hold x above 0):
+// x = 2^k (1 + f) with 1 + f in [sqrt 1/2, sqrt 2), s = f / (2 + f), log(1 + f) =
+// 2 atanh s summed as f - (f^2 / 2 - s (f^2 / 2 + R)) as in fdlibm, R = sum_{i >= 1}
+// 2 s^2i / (2 i + 1) by its Taylor series to s^22 (remainder < 1e-18 relative), and
+// k ln 2 in two parts.
 __host__ __device__ __forceinline__ double log_pos(double x) {
   int k;
 #ifdef __HIP_DEVICE_COMPILE__
@@ -133,7 +134,7 @@ __host__ __device__ __forceinline__ double log_pos(double x) {
   const double h = 0.5 * f * f;
   const double lo = fma(s, h + r, kf * 1.90821492927058770002e-10);
   const double v = fma(kf, 6.93147180369123816490e-01, f - (h - lo));
-  return x < 1.7976931348623157e308 ? v : x + x;
+  return x <= 1.7976931348623157e308 ? v : x + x;
 }
 
 // sqrt(r2) for r2 >= 1e-30: v_rsq_f64 seed, one Goldschmidt step for the

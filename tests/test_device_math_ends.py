@@ -11,7 +11,7 @@ HIPCC = shutil.which("hipcc") or "/opt/rocm/bin/hipcc"
 
 
 @pytest.mark.skipif(not os.path.exists(HIPCC), reason="hipcc not installed")
-@pytest.mark.parametrize("what", ["div"])
+@pytest.mark.parametrize("what", ["div", "log"])
 def test_quotients_and_logs_at_the_ends_of_their_ranges(tmp_path, what):
     exe = tmp_path / "div_log_ends_check"
     src = os.path.join(HERE, "native", "div_log_ends_check.hip")
