@@ -8,7 +8,8 @@
 // 400 baseline points with 2048 samples took.  Here the host only draws the random
 // bits (packed, one word per matrix row); the kernel scrambles the direction
 // numbers of its 64 dimensions in LDS (a parity per bit) and each thread walks 16
-// points of one dimension.  The points are the engine's bit for bit; the normal
+// points of one dimension.  The points are the engine's bit for bit (the first one that
+// of the default dtype float32; a caller under another one replaces it); the normal
 // quantile differs from the CPU's by rounding.
 #include "bta_common.h"
 
@@ -47,7 +48,7 @@ __global__ __launch_bounds__(256) void sobol_normal_kernel(const uint32_t* __res
   for (uint32_t g = (uint32_t)i ^ ((uint32_t)i >> 1); g; g &= g - 1) x ^= st[dl][__ffs(g) - 1];
   const int64_t end = i + SB_PTS < n ? i + SB_PTS : n;
   for (;;) {
-    // (the engine keeps its first point in single precision)
+    // (the engine keeps its first point in the default dtype, float32)
     const double u = (i == 0 ? (double)(float)x : (double)x) * 0x1p-30;
     const double v = 0.5 + (1.0 - eps) * (u - 0.5);
     out[i * d + dim] = erfinv(2.0 * v - 1.0) * 1.4142135623730951;

@@ -41,7 +41,18 @@ def _device_normal_samples(d: int, n: int, device, seed: int) -> Tensor:
         base = bits.data_ptr()
         _lib.check(L.bta_sobol_normal(base, base + 4 * d * 30, base + 8 * d * 30, d, n,
                                       _lib.ptr(out), _lib.stream()), "sobol_normal")
+        if torch.get_default_dtype() != torch.float32:
+            # the engine keeps its first point (the shift) in the default dtype; the
+            # kernel's is the single-precision one
+            out[0] = _normal_quantile((shift.to(torch.int64) / 2**30).to(torch.float64)).to(
+                out.device)
     return out
+
+
+def _normal_quantile(u: Tensor) -> Tensor:
+    """The inverse-normal transform with the eps clamp of sampling/qmc.py:80-83."""
+    v = 0.5 + (1 - torch.finfo(u.dtype).eps) * (u - 0.5)
+    return torch.erfinv(2 * v - 1) * math.sqrt(2)
 
 
 def draw_sobol_normal_samples(d: int, n: int, device=None, dtype=torch.float64,
@@ -52,9 +63,7 @@ def draw_sobol_normal_samples(d: int, n: int, device=None, dtype=torch.float64,
             and n <= DEVICE_POINTS):
         return _device_normal_samples(d, n, device, seed)
     eng = SobolEngine(dimension=d, scramble=True, seed=seed)
-    u = eng.draw(n, dtype=dtype)
-    v = 0.5 + (1 - torch.finfo(u.dtype).eps) * (u - 0.5)
-    return (torch.erfinv(2 * v - 1) * math.sqrt(2)).to(device=device)
+    return _normal_quantile(eng.draw(n, dtype=dtype)).to(device=device)
 
 
 def draw_sobol_samples(bounds: Tensor, n: int, q: int, batch_shape=None,

@@ -224,7 +224,8 @@ int bta_sobol_scramble(uint32_t seed, int32_t d, uint32_t* rows, uint32_t* shift
 
 /* out[i][j] (n x d) = sqrt2 erfinv(2 v - 1), v = 1/2 + (1 - eps)(u - 1/2), for the
  * points u_i of the engine with the unscrambled direction numbers cols (d x 30),
- * rows and shift of bta_sobol_scramble.  n <= 4194240. */
+ * rows and shift of bta_sobol_scramble; u_0 is rounded to single precision, as the
+ * engine does under torch's default dtype float32.  n <= 4194240. */
 int bta_sobol_normal(const uint32_t* cols, const uint32_t* rows, const uint32_t* shift,
                      int32_t d, int64_t n, double* out, bta_stream_t stream);
 
