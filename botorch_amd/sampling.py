@@ -28,23 +28,30 @@ DEVICE_DRAW = 1 << 16
 DEVICE_POINTS = 65535 * 64  # of one bta_sobol_normal call
 
 
-def _device_normal_samples(d: int, n: int, device, seed: int) -> Tensor:
-    L = _lib.lib()
-    bits = torch.empty(2 * d * 30 + d, dtype=torch.int32)
+def _scramble_bits(d: int, seed: int) -> Tensor:
+    """Host words, also under a default device: the direction numbers (d x 30), the
+    scrambling rows (d x 30) and the shifts (d) of bta_sobol_normal."""
+    bits = torch.empty(2 * d * 30 + d, dtype=torch.int32, device="cpu")
     cols, rows, shift = bits.split([d * 30, d * 30, d])
     cols.copy_(SobolEngine(dimension=d, scramble=False).sobolstate.reshape(-1))
-    _lib.check(L.bta_sobol_scramble(seed, d, rows.data_ptr(), shift.data_ptr()),
+    _lib.check(_lib.load().bta_sobol_scramble(seed, d, rows.data_ptr(), shift.data_ptr()),
                "sobol_scramble")
+    return bits
+
+
+def _device_normal_samples(d: int, n: int, device, seed: int) -> Tensor:
+    L = _lib.lib()
+    host = _scramble_bits(d, seed)
     out = torch.empty(n, d, dtype=torch.float64, device=device)
     with torch.cuda.device(out.device):
-        bits = bits.to(out.device)
+        bits = host.to(out.device)
         base = bits.data_ptr()
         _lib.check(L.bta_sobol_normal(base, base + 4 * d * 30, base + 8 * d * 30, d, n,
                                       _lib.ptr(out), _lib.stream()), "sobol_normal")
         if torch.get_default_dtype() != torch.float32:
             # the engine keeps its first point (the shift) in the default dtype; the
             # kernel's is the single-precision one
-            out[0] = _normal_quantile((shift.to(torch.int64) / 2**30).to(torch.float64)).to(
+            out[0] = _normal_quantile((host[-d:].to(torch.int64) / 2**30).to(torch.float64)).to(
                 out.device)
     return out
 

@@ -37,3 +37,19 @@ def test_device_draw_follows_the_default_dtype(default_dtype, dtype, d, n):
     assert d * n >= sampling.DEVICE_DRAW and z.dtype == torch.float64
     assert torch.isfinite(ref).all()
     assert (z.cpu() - ref).abs().max() < 4e-15
+
+
+def test_scrambling_bits_are_host_words_under_any_default_device():
+    with torch.device("meta"):  # a GPU default would hand a device pointer to host code
+        bits = sampling._scramble_bits(3, 11)
+    assert bits.device.type == "cpu" and bits.dtype == torch.int32
+    shift = SobolEngine(dimension=3, scramble=True, seed=11).shift
+    assert torch.equal(bits[-3:].to(torch.int64), shift)
+
+
+@pytest.mark.gpu
+def test_device_draw_under_a_default_device():
+    z = sampling.draw_sobol_normal_samples(512, 128, device="cuda", seed=3)
+    with torch.device("cuda"):
+        again = sampling.draw_sobol_normal_samples(512, 128, device="cuda", seed=3)
+    assert torch.equal(z, again)
