@@ -66,8 +66,8 @@ def draw_sobol_normal_samples(d: int, n: int, device=None, dtype=torch.float64,
                               seed: int | None = None) -> Tensor:
     """n x d quasi-normal samples (utils/sampling.py:114-143, qmc.py:80-83)."""
     if (device is not None and torch.device(device).type == "cuda" and dtype == torch.float64
-            and seed is not None and 0 <= seed < 2**32 and d * n >= DEVICE_DRAW
-            and n <= DEVICE_POINTS):
+            and type(seed) is int and 0 <= seed < 2**32  # (the engine refuses other types)
+            and d * n >= DEVICE_DRAW and n <= DEVICE_POINTS):
         return _device_normal_samples(d, n, device, seed)
     eng = SobolEngine(dimension=d, scramble=True, seed=seed)
     return _normal_quantile(eng.draw(n, dtype=dtype)).to(device=device)

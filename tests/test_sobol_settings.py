@@ -6,6 +6,7 @@ Tolerance of the draw: the points are equal and the two inverse error functions 
 within a few ulp of |z| <= 6.3: 4e-15 absolute."""
 import math
 
+import numpy as np
 import pytest
 import torch
 from torch.quasirandom import SobolEngine
@@ -53,3 +54,10 @@ def test_device_draw_under_a_default_device():
     with torch.device("cuda"):
         again = sampling.draw_sobol_normal_samples(512, 128, device="cuda", seed=3)
     assert torch.equal(z, again)
+
+
+@pytest.mark.parametrize("seed", [np.int64(3), 3.0, True, np.array(3), torch.tensor(3)])
+def test_seeds_the_engine_refuses_are_refused(seed):
+    for device in ("cpu", "cuda"):
+        with pytest.raises((TypeError, RuntimeError), match="integer|manual_seed"):
+            sampling.draw_sobol_normal_samples(512, 128, device=device, seed=seed)
