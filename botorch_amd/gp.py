@@ -694,10 +694,15 @@ class GPyTorchPosterior:
             if zv.stride(-1) != 1 and m > 1:
                 zv = zv.contiguous()
             mean, L = self._mean.reshape(nb, m), Lt.reshape(nb, m, m)
-            if torch.is_grad_enabled() and (Lt.requires_grad or mean.requires_grad):
-                out = _MvnSampleFn.apply(mean, L, zv)
-            else:
-                out = _mvn_sample(mean, L, zv)
+            need_L = torch.is_grad_enabled() and Lt.requires_grad
+            # the mean is added by torch where only torch can differentiate it: alone,
+            # by a tangent or by a function transform
+            apart = _transformed(mean) or (torch.is_grad_enabled() and mean.requires_grad
+                                           and not need_L)
+            base = torch.zeros(nb, m, dtype=L.dtype, device=L.device) if apart else mean
+            out = _MvnSampleFn.apply(base, L, zv) if need_L else _mvn_sample(base, L, zv)
+            if apart:
+                out = out + mean
             return out.reshape(*sample_shape, *self._mean.shape, 1)
         zf = z.reshape(S, nb, m).permute(1, 0, 2).contiguous()  # nb x S x m
         if torch.is_grad_enabled() and Lt.requires_grad:
@@ -718,6 +723,12 @@ class GPyTorchPosterior:
 MVN_SAMPLE_MAX = 16
 
 
+def _transformed(t: Tensor) -> bool:
+    """Whether t carries a forward-mode tangent or a function transform is active."""
+    return (torch._C._are_functorch_transforms_active()
+            or torch.autograd.forward_ad.unpack_dual(t).tangent is not None)
+
+
 def _mvn_sample(mean: Tensor, Lt: Tensor, z: Tensor) -> Tensor:
     """mean + L z: S x nb x m for mean nb x m, L nb x m x m and z S x nb x m (any
     strides but the last)."""
@@ -732,7 +743,8 @@ def _mvn_sample(mean: Tensor, Lt: Tensor, z: Tensor) -> Tensor:
 
 class _MvnSampleFn(torch.autograd.Function):
     """Samples mean + L z with dmean = sum g and dL = tril(sum g z^T); the base
-    samples are constants."""
+    samples are constants.  The samples are linear in the mean: its gradient can be
+    differentiated again (dL's cannot)."""
 
     @staticmethod
     def forward(ctx, mean: Tensor, Lt: Tensor, z: Tensor):
@@ -749,6 +761,8 @@ class _MvnSampleFn(torch.autograd.Function):
         _lib.check(_lib.lib().bta_mvn_sample_backward(
             _lib.ptr(g), z.data_ptr(), z.stride(0), z.stride(1), S, nb, m, _lib.ptr(dmean),
             _lib.ptr(dL), _lib.stream()), "mvn_sample_backward")
+        if torch.is_grad_enabled():  # create_graph
+            dmean = g.sum(0)
         return dmean, dL, None
 
 

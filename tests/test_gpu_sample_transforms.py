@@ -1,6 +1,5 @@
-"""Posterior samples under the other ways of differentiating: a second derivative through
-the mean, forward mode and function transforms over the mean, and saved tensors that come
-back from hooks on another device and in another type.
+"""Posterior samples under the other ways of differentiating and mapping them: a second
+derivative through the mean, forward mode, vmap and batched gradients over the mean.
 
 The samples are mean + L z, linear in the mean: every expected value is formed from the
 samples themselves, up to one rounding per operation (1e-13 of values of order 10)."""
@@ -21,8 +20,7 @@ def _parts():
     A = torch.randn(NB, M, M, generator=g, dtype=torch.float64)
     cov = (A @ A.transpose(-1, -2) + M * torch.eye(M, dtype=torch.float64)).to(DEV)
     mean = torch.randn(NB, M, generator=g, dtype=torch.float64).to(DEV)
-    # exact in single precision: a hook may keep them so
-    z = torch.randn(S, NB, M, generator=g, dtype=torch.float32).double().to(DEV)
+    z = torch.randn(S, NB, M, generator=g, dtype=torch.float64).to(DEV)
     w = torch.randn(S, NB, M, generator=g, dtype=torch.float64).to(DEV)
     return mean, cov, z, w
 
@@ -55,11 +53,17 @@ def test_forward_mode_in_the_mean():
         assert (primal - _samples(mean, cov, z)).abs().max() < 1e-13 * primal.abs().max()
 
 
-def test_function_transforms_over_the_mean():
+def test_vmap_over_the_mean():
+    mean, cov, z, _ = _parts()
+    means = torch.stack([mean, 2 * mean, -mean])
+    y = torch.func.vmap(lambda mu: _samples(mu, cov, z))(means)
+    for mu, ys in zip(means, y):
+        assert (ys - _samples(mu, cov, z)).abs().max() < 1e-13 * ys.abs().max()
+
+
+def test_batched_gradients_of_the_mean():
     mean, cov, z, w = _parts()
-    f = lambda mu: (_samples(mu, cov, z) * w).sum()  # noqa: E731
-    g = torch.func.grad(f)(mean)
-    assert (g - w.sum(0)).abs().max() < 1e-13 * w.abs().sum(0).max()
-    t = torch.randn_like(mean)
-    _, tangent = torch.func.jvp(f, (mean,), (t,))
-    assert (tangent - (w.sum(0) * t).sum()).abs() < 1e-12 * (w.abs().sum(0) * t.abs()).sum()
+    mean.requires_grad_(True)
+    ws = torch.stack([w, 2 * w])
+    (g,) = torch.autograd.grad(_samples(mean, cov, z), mean, ws, is_grads_batched=True)
+    assert (g - ws.sum(1)).abs().max() < 1e-13 * ws.abs().sum(1).max()
