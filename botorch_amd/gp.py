@@ -583,6 +583,11 @@ class _PosteriorFn(torch.autograd.Function):
     @staticmethod
     def backward(ctx, dmean: Tensor | None, dcov: Tensor | None):
         Xc, keep = ctx.saved_tensors
+        # (hooks may return them on another device, in another type or layout)
+        dev = ctx.cache["xs"].device
+        Xc = Xc.to(device=dev, dtype=torch.float64).contiguous()
+        if keep is not None:
+            keep = keep.to(device=dev, dtype=torch.uint8).contiguous()
         return SingleTaskGP._posterior_backward(ctx.cache, Xc, dmean, dcov, keep), None
 
 
@@ -756,6 +761,9 @@ class _MvnSampleFn(torch.autograd.Function):
         (z,) = ctx.saved_tensors
         S, nb, m = z.shape
         g = g.to(torch.float64).contiguous()
+        z = z.to(device=g.device, dtype=torch.float64)  # (as a hook may return it)
+        if z.stride(-1) != 1 and m > 1:
+            z = z.contiguous()
         dmean = torch.empty(nb, m, dtype=torch.float64, device=g.device)
         dL = torch.empty(nb, m, m, dtype=torch.float64, device=g.device)
         _lib.check(_lib.lib().bta_mvn_sample_backward(
