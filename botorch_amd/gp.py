@@ -13,8 +13,11 @@ solve and posterior contraction runs in libbotorch_amd (HIP) through
 """
 from __future__ import annotations
 
+import collections
 import ctypes
 import math
+import threading
+import weakref
 
 import torch
 from torch import Tensor
@@ -513,7 +516,7 @@ class SingleTaskGP(torch.nn.Module):
 
     def _posterior_call(self, Xf: Tensor, for_grad: bool):
         """The moments, the prediction cache they came from and, for_grad, the buffer
-        the adjoint takes over (None above KEEP_BYTES: it then recomputes)."""
+        the adjoint takes over (None past KEEP_BYTES: it then recomputes)."""
         c = self.prediction_cache()
         L = _lib.lib()
         m = ctypes.byref(c["model"])
@@ -523,7 +526,7 @@ class SingleTaskGP(torch.nn.Module):
         cov = torch.empty(nb, mq, mq, dtype=torch.float64, device=dev)
         ws = _lib.workspace(L.bta_gp_posterior_workspace_size(m, nb, mq), dev)
         size = L.bta_gp_posterior_keep_size(m, nb, mq) if for_grad else 0
-        keep = _lib.workspace(size, dev) if 0 < size <= KEEP_BYTES else None
+        keep = _kept.take(size, dev)
         if keep is not None:
             _lib.check(L.bta_gp_posterior_keep(m, _lib.ptr(Xf), nb, mq, _lib.ptr(mean),
                                                _lib.ptr(cov), None, _lib.ptr(keep), _lib.ptr(ws),
@@ -563,9 +566,42 @@ class SingleTaskGP(torch.nn.Module):
         raise UnsupportedError("use posterior(); the prior MVN is not materialised")
 
 
-# Largest buffer (scaled points and V = K_x L^-T) a posterior that requires grad holds
-# for its adjoint
+# What all posteriors that wait for their backward may hold on a device in buffers for
+# their adjoints (scaled points and V = K_x L^-T)
 KEEP_BYTES = 256 << 20
+
+
+class _KeptBuffers:
+    """Hands out the adjoints' buffers while those alive on the device stay within
+    KEEP_BYTES.  A buffer counts until the graph (or a saved-tensor hook) lets go of it.
+    Its finalizer may run in any thread and anywhere the collector does, also under the
+    lock: it only appends to a deque, which the next call takes off the count."""
+
+    def __init__(self):
+        self._lock = threading.Lock()
+        self._used = collections.Counter()
+        self._freed = collections.deque()
+
+    def take(self, size: int, device) -> Tensor | None:
+        if not 0 < size <= KEEP_BYTES:
+            return None
+        with self._lock:
+            while self._freed:
+                dev, n = self._freed.popleft()
+                self._used[dev] -= n
+            if self._used[device] + size > KEEP_BYTES:
+                return None
+            self._used[device] += size
+        try:
+            keep = _lib.workspace(size, device)
+        except BaseException:
+            self._freed.append((device, size))
+            raise
+        weakref.finalize(keep, self._freed.append, (device, size)).atexit = False
+        return keep
+
+
+_kept = _KeptBuffers()
 
 
 class _PosteriorFn(torch.autograd.Function):

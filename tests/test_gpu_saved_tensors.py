@@ -1,5 +1,6 @@
 """Saved tensors of posteriors and samples that come back from hooks on another device,
-in another type or layout.  The compared gradients come from the same kernels on the same
+in another type or layout, and the bound on what posteriors hold until their backward.
+The compared gradients come from the same kernels on the same
 inputs: equal bit for bit."""
 import pytest
 import torch
@@ -76,3 +77,30 @@ def test_saved_posterior_tensors_may_come_back_in_another_type(monkeypatch, kept
     with torch.autograd.graph.saved_tensors_hooks(pack, lambda t: t):
         loss = grad()
     assert torch.equal(torch.autograd.grad(loss, X)[0], want)
+
+
+def test_many_live_posteriors_hold_a_bounded_amount(monkeypatch):
+    gp = _model()
+    g = torch.Generator().manual_seed(1)
+    Xs = [torch.rand(64, 4, 3, generator=g, dtype=torch.float64).to(DEV) for _ in range(20)]
+    gp.prediction_cache()
+    alone = []
+    for X in Xs:
+        X.requires_grad_(True)
+        post = gp.posterior(X)
+        (dx,) = torch.autograd.grad(post.covariance_matrix.square().sum(), X)
+        alone.append(dx)
+    per = 256 * 128 * 8  # rows x n_pad doubles of V
+    limit = 4 * per
+    monkeypatch.setattr(G, "KEEP_BYTES", limit)
+    for _ in range(2):  # what the first round held is free again in the second
+        torch.cuda.synchronize()
+        before = torch.cuda.memory_allocated()
+        posts = [gp.posterior(X) for X in Xs]
+        held = torch.cuda.memory_allocated() - before
+        outputs = len(Xs) * (64 * 4 * 4 + 64 * 4) * 8
+        assert per < held < limit + outputs + len(Xs) * 64 * 1024, held
+        loss = sum(p.covariance_matrix.square().sum() for p in posts)
+        together = torch.autograd.grad(loss, Xs)
+        assert all(torch.equal(a, b) for a, b in zip(alone, together))
+        del posts, loss, together
