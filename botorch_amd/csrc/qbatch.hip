@@ -138,8 +138,9 @@ static void add_tiles(const H2Args& g, int p, int tw, std::vector<int4>& out) {
 // h2_tile_of pairs heavy with light tiles across the whole batch; then the row
 // tiles of one (problem, column), which share their panel of B, are dealt to
 // positions of one residue modulo 8.  Worker p runs on XCD p % 8 and h2_tile_of
-// keeps or mirrors that residue (the worker counts are multiples of 8), so the
-// panel is read into one L2 instead of as many as there are row tiles.  32 models of
+// keeps or mirrors that residue (the worker counts are multiples of 8, or one worker
+// per tile in a single round), so the panel is read into one L2 instead of as many as
+// there are row tiles.  32 models of
 // 128 to 4096 points, 512 rows: the adjoint list (128 x 64 tiles) takes 379 us in plain
 // order, 363 so.
 static void order_tiles(const std::vector<H2Args>& tab, int tw, std::vector<int4>& t) {
@@ -274,7 +275,7 @@ int qlognei_batch_prepare(const bta_qlognei_batch_item* items, int nm, void* ws,
                 i);
       return BTA_ERR_UNSUPPORTED;
     }
-    int bn = 0, wk = 0;  // the split GEMMs' shape and alignment checks
+    // the split GEMMs' shape and alignment checks
     rc = gemm_h2_check(A[i].fwd);
     if (!rc && grad) rc = gemm_h2_check(A[i].adj);
     if (rc) return rc;

@@ -393,7 +393,9 @@ typedef struct bta_qlognei_batch_item {
   int32_t* status;                /* b, BTA_STATUS_* bits */
 } bta_qlognei_batch_item;
 
-/* Written by bta_qlognei_batch_prepare; offsets are bytes into ws. */
+/* Written by bta_qlognei_batch_prepare; offsets are bytes into ws.  More fwd_workers than
+ * fwd_tiles: the forward list holds 128 x 128 tiles, a workgroup each, else 128 x 64 ones
+ * dealt to that many workers. */
 typedef struct bta_qlognei_batch_plan {
   void* ws;
   int32_t n_items, q, kind, kd, grad;
