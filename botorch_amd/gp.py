@@ -571,33 +571,39 @@ class SingleTaskGP(torch.nn.Module):
 KEEP_BYTES = 256 << 20
 
 
+class _KeptRef(weakref.ref):
+    __slots__ = ("device", "size")
+
+
 class _KeptBuffers:
     """Hands out the adjoints' buffers while those alive on the device stay within
     KEEP_BYTES.  A buffer counts until the graph (or a saved-tensor hook) lets go of it.
-    Its finalizer may run in any thread and anywhere the collector does, also under the
-    lock: it only appends to a deque, which the next call takes off the count."""
+    Its weak reference's callback may run in any thread and anywhere the collector does,
+    also under the lock: it only appends to a deque, which the next call takes off the
+    count."""
 
     def __init__(self):
         self._lock = threading.Lock()
-        self._used = collections.Counter()
-        self._freed = collections.deque()
+        self._used = {}  # device -> bytes
+        self._alive = {}  # the references, by identity
+        self._dead = collections.deque()
 
     def take(self, size: int, device) -> Tensor | None:
         if not 0 < size <= KEEP_BYTES:
             return None
         with self._lock:
-            while self._freed:
-                dev, n = self._freed.popleft()
-                self._used[dev] -= n
-            if self._used[device] + size > KEEP_BYTES:
+            while self._dead:
+                ref = self._dead.popleft()
+                del self._alive[id(ref)]
+                self._used[ref.device] -= ref.size
+            used = self._used.get(device, 0) + size
+            if used > KEEP_BYTES:
                 return None
-            self._used[device] += size
-        try:
             keep = _lib.workspace(size, device)
-        except BaseException:
-            self._freed.append((device, size))
-            raise
-        weakref.finalize(keep, self._freed.append, (device, size)).atexit = False
+            ref = _KeptRef(keep, self._dead.append)
+            ref.device, ref.size = device, size
+            self._alive[id(ref)] = ref
+            self._used[device] = used
         return keep
 
 
@@ -621,8 +627,10 @@ class _PosteriorFn(torch.autograd.Function):
         Xc, keep = ctx.saved_tensors
         # (hooks may return them on another device, in another type or layout)
         dev = ctx.cache["xs"].device
-        Xc = Xc.to(device=dev, dtype=torch.float64).contiguous()
-        if keep is not None:
+        if Xc.dtype != torch.float64 or Xc.device != dev or not Xc.is_contiguous():
+            Xc = Xc.to(device=dev, dtype=torch.float64).contiguous()
+        if keep is not None and (keep.dtype != torch.uint8 or keep.device != dev
+                                 or not keep.is_contiguous()):
             keep = keep.to(device=dev, dtype=torch.uint8).contiguous()
         return SingleTaskGP._posterior_backward(ctx.cache, Xc, dmean, dcov, keep), None
 
@@ -797,9 +805,8 @@ class _MvnSampleFn(torch.autograd.Function):
         (z,) = ctx.saved_tensors
         S, nb, m = z.shape
         g = g.to(torch.float64).contiguous()
-        z = z.to(device=g.device, dtype=torch.float64)  # (as a hook may return it)
-        if z.stride(-1) != 1 and m > 1:
-            z = z.contiguous()
+        if z.dtype != torch.float64 or z.device != g.device or (z.stride(-1) != 1 and m > 1):
+            z = z.to(g).contiguous()  # (as a hook may return it)
         dmean = torch.empty(nb, m, dtype=torch.float64, device=g.device)
         dL = torch.empty(nb, m, m, dtype=torch.float64, device=g.device)
         _lib.check(_lib.lib().bta_mvn_sample_backward(
