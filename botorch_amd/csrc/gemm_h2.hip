@@ -38,7 +38,8 @@
 // 64 x 64 (three workgroups per CU) has the shortest chunk, 0.3 us against 0.5,
 // which is what counts while each CU has one tile or less; 128 x 256 with eight
 // waves of 64 x 64 moves half the bytes per product and runs large products at the
-// rate of a plain FP16 matrix product (1030 TFLOP/s), 128 x 128 with sixteen waves
+// rate of a plain FP16 matrix product (1047 TFLOP/s in the last line, 970 inside a whole
+// step of that size; plain 1030-1090), 128 x 128 with sixteen waves
 // of 32 x 32 fills the gap where 128 x 256 gives a CU one tile only.  128 x 64 lies
 // between, and is the tile of the launches that share CUs with other work.
 // Triangular K ranges follow gemm_kernel; for 128 x 64 a cost model picks the

@@ -27,8 +27,9 @@
 // Pareto term is exactly 1; the second fat minima's logs over the objectives are
 // one log of the product of their sums (each in [1, 2]); exp is left out where it
 // is below half an ulp of the Cauchy term beside it; logs by log_pos (about 35
-// instructions against the math library's 90), divisions by div_normal.  4096 x 6 pairs, 40 cells, 2 objectives: forward 49 -> 34 us,
-// backward 95 (768 waves, one lane per (b, s, k)) -> 50 us.
+// instructions against the math library's 90), divisions by div_normal.  4096 x 6
+// pairs, 40 cells, 2 objectives: forward 49 -> 34 us, backward 95 (768 waves, one lane
+// per (b, s, k)) -> 50 us; the call through autograd, which the host bounds, stays 126.
 #include "bta_common.h"
 
 namespace bta {

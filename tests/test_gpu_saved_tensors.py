@@ -93,7 +93,7 @@ def test_many_live_posteriors_hold_a_bounded_amount(monkeypatch):
     per = 256 * 128 * 8  # rows x n_pad doubles of V
     limit = 4 * per
     monkeypatch.setattr(G, "KEEP_BYTES", limit)
-    for _ in range(2):  # what the first round held is free again in the second
+    for _ in range(2):  # what the first pass held is free again in the second
         torch.cuda.synchronize()
         before = torch.cuda.memory_allocated()
         posts = [gp.posterior(X) for X in Xs]
