@@ -21,6 +21,7 @@ import weakref
 
 import torch
 from torch import Tensor
+from torch.autograd.forward_ad import unpack_dual
 
 from . import _lib
 from .exceptions import InputDataError, NanError, NotPSDError, UnsupportedError
@@ -381,10 +382,6 @@ class SingleTaskGP(torch.nn.Module):
             t = getattr(self, "outcome_transform", None) if stats else None
             if t is not None:
                 parts += [t.means, t.stdvs]
-            for p in parts[1:]:
-                if p.numel() != 1:
-                    raise RuntimeError(f"a Tensor with {p.numel()} elements cannot be converted "
-                                       "to Scalar")
             first_extra = len(parts)
             parts += extra
             flat = [p.detach().reshape(-1) for p in parts]
@@ -396,8 +393,14 @@ class SingleTaskGP(torch.nn.Module):
         for p in flat:
             out.append(vals[i:i + p.numel()])
             i += p.numel()
-        y_stats = (out[4][0], out[5][0]) if t is not None else (0.0, 1.0)
-        return out[0], out[1][0], out[2][0], out[3][0], y_stats, out[first_extra:]
+        try:
+            (outputscale,), (noise,), (constant,) = out[1:4]
+            (y_mean,), (y_std,) = out[4:6] if t is not None else ((0.0,), (1.0,))
+        except ValueError:
+            n = next(len(v) for v in out[1:first_extra] if len(v) != 1)
+            raise RuntimeError(
+                f"a Tensor with {n} elements cannot be converted to Scalar") from None
+        return out[0], outputscale, noise, constant, (y_mean, y_std), out[first_extra:]
 
     def hyperparameters(self) -> dict:
         _, outputscale, noise, constant, _, _ = self._host_values()
@@ -775,7 +778,7 @@ MVN_SAMPLE_MAX = 16
 def _transformed(t: Tensor) -> bool:
     """Whether t carries a forward-mode tangent or a function transform is active."""
     return (torch._C._are_functorch_transforms_active()
-            or torch.autograd.forward_ad.unpack_dual(t).tangent is not None)
+            or unpack_dual(t).tangent is not None)
 
 
 def _mvn_sample(mean: Tensor, Lt: Tensor, z: Tensor) -> Tensor:
