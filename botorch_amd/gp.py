@@ -474,7 +474,8 @@ class SingleTaskGP(torch.nn.Module):
         m.linv = _lib.ptr(Linv)
         m.alpha = _lib.ptr(alpha)
         self._cache = {"model": m, "xs": xs, "center": center, "lengthscale": ls, "L": Lmat,
-                       "Linv": Linv, "alpha": alpha, "n_pad": n_pad, "jitter": jit.value}
+                       "Linv": Linv, "alpha": alpha, "n_pad": n_pad, "jitter": jit.value,
+                       "stream": st.value or 0}
         self._cache_key = key
         return self._cache
 
@@ -533,11 +534,11 @@ class SingleTaskGP(torch.nn.Module):
         if keep is not None:
             _lib.check(L.bta_gp_posterior_keep(m, _lib.ptr(Xf), nb, mq, _lib.ptr(mean),
                                                _lib.ptr(cov), None, _lib.ptr(keep), _lib.ptr(ws),
-                                               ws.numel(), _lib.stream()), "gp_posterior")
+                                               ws.numel(), _stream_for(c)), "gp_posterior")
         else:
             _lib.check(L.bta_gp_posterior(m, _lib.ptr(Xf), nb, mq, _lib.ptr(mean),
                                           _lib.ptr(cov), None, _lib.ptr(ws), ws.numel(),
-                                          _lib.stream()), "gp_posterior")
+                                          _stream_for(c)), "gp_posterior")
         return mean, cov, c, keep
 
     @staticmethod
@@ -558,11 +559,11 @@ class SingleTaskGP(torch.nn.Module):
         if keep is not None:
             _lib.check(L.bta_gp_posterior_backward_kept(
                 m, nb, mq, _lib.ptr(dm), _lib.ptr(dc), _lib.ptr(dX), _lib.ptr(keep),
-                _lib.ptr(ws), ws.numel(), _lib.stream()), "gp_posterior_backward")
+                _lib.ptr(ws), ws.numel(), _stream_for(c)), "gp_posterior_backward")
         else:
             _lib.check(L.bta_gp_posterior_backward(
                 m, _lib.ptr(Xf), nb, mq, _lib.ptr(dm), _lib.ptr(dc), _lib.ptr(dX), _lib.ptr(ws),
-                ws.numel(), _lib.stream()), "gp_posterior_backward")
+                ws.numel(), _stream_for(c)), "gp_posterior_backward")
         return dX
 
     def forward(self, X: Tensor):
@@ -572,6 +573,18 @@ class SingleTaskGP(torch.nn.Module):
 # What all posteriors that wait for their backward may hold on a device in buffers for
 # their adjoints (scaled points and V = K_x L^-T)
 KEEP_BYTES = 256 << 20
+
+
+def _stream_for(c: dict) -> ctypes.c_void_p:
+    """The current stream, for a call that reads the prediction cache c.  Where it is not
+    the one the cache was built on, the cache's memory is held until it is done: the last
+    reference may go right behind the call (the graph's, once its backward is enqueued)."""
+    s = torch.cuda.current_stream()
+    if s.cuda_stream != c["stream"]:
+        for t in c.values():
+            if torch.is_tensor(t):
+                t.record_stream(s)
+    return ctypes.c_void_p(s.cuda_stream)
 
 
 class _KeptRef(weakref.ref):
